@@ -653,14 +653,28 @@ int onepass_reg_tiles(const SplitArgs& a) {
   }
 }
 
+// Longest rows first (SplitArgs::longest_first) with more waves than the CUs
+// hold at once (8 each at 16 and 32 tiles per wave), where the order decides
+// what the launch ends on; below, every workgroup starts at once, and the
+// lengths' extra round trip costs (µs, B=128 S=256 32/8, 2048 waves, all rows
+// equal: 25.9 without, 27.3 with).
+constexpr int kOrderWavesPerCU = 8;
+
 template <int D, int LAYOUT>
-hipError_t launch_onepass_reg(const SplitArgs& a, int tpw, hipStream_t stream) {
+hipError_t launch_onepass_reg(const SplitArgs& args, int tpw, hipStream_t stream) {
+  SplitArgs a = args;
   const int g = a.num_heads_q / a.num_heads_kv;
   const int nw = (a.nblk + tpw - 1) / tpw;
   const size_t need = fmha_decode::onepass_reg_lds_bytes<D>(nw, tpw, LAYOUT);
   plan_note("onepass_matrix_core_regs(D=%d G=%d layout=%s waves_per_row=%d tiles_per_wave=%d blocks=%d)", D, g,
             layout_name(LAYOUT), nw, tpw, a.nblk);
-  const dim3 grid((uint32_t)((int64_t)a.batch * a.num_heads_kv));
+  const int64_t units = (int64_t)a.batch * a.num_heads_kv;
+  const int64_t cus = device_cus() > 0 ? device_cus() : 256;
+  a.longest_first = a.len_mode != fmha_decode::kLenUniform && a.batch > 1 && a.batch <= fmha_decode::kOrderBatches &&
+                    units * nw > kOrderWavesPerCU * cus;
+  const uint32_t round_tiles = (uint32_t)(nw * fmha_decode::onepass_reg_round_tiles(D, tpw, LAYOUT));
+  a.round_inv = (65536u + round_tiles - 1) / round_tiles;
+  const dim3 grid((uint32_t)units);
   const dim3 block((uint32_t)(kBlockThreads * nw));
   if (tpw == 8) {
     hipLaunchKernelGGL((fmha_decode::onepass_mfma_reg_kernel<D, 8, kOnepassRegMaxWaves, LAYOUT>), grid, block, need,

@@ -93,6 +93,13 @@ struct SplitArgs {
   // 1: the statistics pass ran and ml holds each head's global max and sum;
   // 0: every P.V wave reduces its heads' block statistics (m, l) itself.
   int32_t stat_pass;
+  // Register single pass: 1: workgroups take the batches longest row first
+  // (longest_first; at most kOrderBatches batches), 0: as they come.
+  int32_t longest_first;
+  // Register single pass: ceil(2^16 / n) for the n tiles that the
+  // workgroup's waves stage in one round, so that x / n is x * round_inv >>
+  // 16 (exact for x * n < 2^16; x is below 512 and n at most 64).
+  uint32_t round_inv;
 };
 
 // KV heads of the cache in memory, and the one launch head hk reads.
@@ -126,6 +133,57 @@ __device__ __forceinline__ int split_len_l(const SplitArgs& a, uint64_t b) {
 }
 
 constexpr int kSplitBlockRows = kMaxSeq;  // rows per scores wave
+
+// The batch that workgroup group i (< batch) of a single-pass launch serves
+// with SplitArgs::longest_first: the one with the i-th longest row, in 16-row
+// blocks, ties in batch order, so that the longest rows start first and the
+// launch does not end on one of them alone.  Every lane of the wave calls it;
+// every wave of every workgroup finds the same order.
+constexpr int kOrderBatches = 256;
+
+template <int LAYOUT>
+__device__ __forceinline__ uint32_t longest_first(const SplitArgs& a, uint32_t i, int lane) {
+  constexpr int NP = kOrderBatches / kWaveSize;
+  if (__builtin_expect(!a.longest_first, 1)) return i;  // the search stays out of the other launches' straight-line code
+  int blocks[NP];  // -1: no batch
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const int b = p * kWaveSize + lane;
+    blocks[p] = -1;
+    if (b < a.batch) {
+      const int S = split_len_l<LAYOUT>(a, (uint64_t)b);
+      blocks[p] = S < 0 || S > a.max_rows ? 0 : (S + kSplitBlockRows - 1) / kSplitBlockRows;
+    }
+  }
+  // Rows of at least v blocks, as a count over the wave.
+  auto at_least = [&](int v) {
+    int n = 0;
+#pragma unroll
+    for (int p = 0; p < NP; ++p) n += __popcll(__builtin_amdgcn_ballot_w64(blocks[p] >= v));
+    return n;
+  };
+  // One length for all: as they come.
+  const int first = __builtin_amdgcn_readfirstlane(blocks[0]);
+  if (at_least(first) == a.batch && at_least(first + 1) == 0) return i;
+  // v: the i-th largest block count, bit by bit.
+  int v = 0;
+  for (int bit = 31 - __clz(a.nblk); bit >= 0; --bit)
+    if (at_least(v | (1 << bit)) > (int)i) v |= 1 << bit;
+  int r = (int)i - at_least(v + 1);  // its place among the rows of v blocks
+  uint32_t found = i;
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const uint64_t m = __builtin_amdgcn_ballot_w64(blocks[p] == v);
+    const int n = __popcll(m);
+    if (r >= 0 && r < n) {
+      const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+      found = (uint32_t)(p * kWaveSize) +
+              (uint32_t)__builtin_ctzll(__builtin_amdgcn_ballot_w64(blocks[p] == v && before == r));
+    }
+    r -= n;
+  }
+  return found;
+}
 
 __device__ __forceinline__ u32x4 buffer_load16_nt(__amdgpu_buffer_rsrc_t r, uint32_t voffset) {
   return buffer_load16<kPolicyStream>(r, voffset);

@@ -663,9 +663,16 @@ __global__ __launch_bounds__(kBlockThreads * NW) void onepass_mfma_kernel(SplitA
 //   * waves 1..NW-1 hand their fp32 sums to wave 0 through LDS (the K
 //     staging's space), which adds them in wave order and writes fp16 O.
 // Rows past the wave's range are never read (out-of-range offsets read 0).
-// The tile loops are unrolled over TPW with no branch inside: the scores'
-// registers need static indices, and a branch per tile made the compiler
-// wait for every load in flight at each tile.  Packed and strided layouts,
+// A row's tiles are shared evenly among the waves whatever its length, and
+// with many workgroups the longest rows go first (longest_first): on ragged
+// batches a launch otherwise ends on one wave of a late long row (µs, 16-row
+// pages, B=64 32/8, lengths log-uniform over 128-4096, 305 MB: 117.6 with
+// shares of the longest row in batch order, 69.7; packed B=256 64/8 32-1024:
+// 92.4 / 68.6; equal lengths are unchanged, B=256 S=1024 64/8 174.7 / 174.6).
+// The tile loops are unrolled over TPW, left at the round after the wave's
+// last tile and with no other branch inside: the scores' registers need
+// static indices, and a branch per tile made the compiler wait for every
+// load in flight at each tile.  Packed and strided layouts,
 // and paged ones: pages of at least 16 rows (kLayoutPagedBlock), where a
 // tile lies in one page, K through per-lane page addresses (PagedLaneRows),
 // V through a descriptor per tile from the tile's block-table entry, which
@@ -715,7 +722,6 @@ __global__ __launch_bounds__(kBlockThreads * NWMAX) void onepass_mfma_reg_kernel
   constexpr int VW = DPC / 2;  // dwords of a lane's V run per row
   constexpr int PF = onepass_reg_pf<D, TPW>();
   constexpr int NR = kSplitBlockRows;
-  constexpr int R = TPW * NR;
   using Sh = GroupShape<D>;
   constexpr int LPH = Sh::LPH;
   constexpr int HPW = Sh::HPW;
@@ -728,9 +734,10 @@ __global__ __launch_bounds__(kBlockThreads * NWMAX) void onepass_mfma_reg_kernel
   const int nw = (int)(blockDim.x / kWaveSize);
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWaveSize));
   const uint32_t hkv = (uint32_t)a.num_heads_kv;
-  const uint32_t b = blockIdx.x / hkv;
-  const uint32_t hk = blockIdx.x - b * hkv;
-  if (b >= (uint32_t)a.batch) return;
+  const uint32_t bi = blockIdx.x / hkv;
+  const uint32_t hk = blockIdx.x - bi * hkv;
+  if (bi >= (uint32_t)a.batch) return;
+  const uint32_t b = longest_first<LAYOUT>(a, bi, lane);
   const int hq = a.num_heads_q;
   const int G = hq / (int)hkv;  // <= 16
   const int S = split_len_l<LAYOUT>(a, b);
@@ -747,8 +754,12 @@ __global__ __launch_bounds__(kBlockThreads * NWMAX) void onepass_mfma_reg_kernel
       buffer_store16(o_rsrc, (uint32_t)((k / (D / 8)) * D + (k % (D / 8)) * 8) * 2u, fill);
     return;
   }
-  const int lo = wv * R;
-  const int span = S - lo < 0 ? 0 : (S - lo < R ? S - lo : R);
+  // The row's tiles in even shares of whole staging rounds, at most TPW each
+  // (a row shorter than the call's longest still keeps every wave busy).
+  const uint32_t round_tiles = (uint32_t)(nw * RT);
+  const int share = (int)((((uint32_t)(S + NR - 1) / NR + round_tiles - 1) * a.round_inv) >> 16) * RT;
+  const int lo = wv * share * NR;
+  const int span = S - lo < 0 ? 0 : (S - lo < share * NR ? S - lo : share * NR);
   const int nt = (span + NR - 1) / NR;
   // Pages of at least 16 rows: a tile lies in one page.  Lane t < nt holds
   // the block-table entry of the wave's tile t (entry 0, which a batch with
@@ -806,6 +817,7 @@ __global__ __launch_bounds__(kBlockThreads * NWMAX) void onepass_mfma_reg_kernel
     }
 #pragma unroll
     for (int k = 0; k < TPW / RT; ++k) {
+      if (k * RT >= nt) break;
       wave_lds_sync();  // the previous round's reads of the staging are done
 #pragma unroll
       for (int j = 0; j < KR; ++j) *reinterpret_cast<u32x4*>(stage + (ph + j) * KSR + ps * D * 2 + r * 16) = kb[j];
@@ -845,6 +857,7 @@ __global__ __launch_bounds__(kBlockThreads * NWMAX) void onepass_mfma_reg_kernel
   float l = 0.0f;
 #pragma unroll
   for (int t = 0; t < TPW; ++t) {
+    if (t % RT == 0 && t >= nt) break;
 #pragma unroll
     for (int e = 0; e < 4; ++e) l += t * NR + 4 * q + e < span ? expf(x[t][e] - cm) : 0.0f;
   }
@@ -968,6 +981,7 @@ __global__ __launch_bounds__(kBlockThreads * NWMAX) void onepass_mfma_reg_kernel
   if (nt > 0) {
 #pragma unroll
     for (int t = 0; t < TPW; ++t) {
+      if (t % RT == 0 && t >= nt) break;
       bf16x4_v pa;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {

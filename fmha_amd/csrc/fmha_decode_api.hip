@@ -525,106 +525,76 @@ constexpr size_t kWorkspaceAlign = 256;
 size_t align_up(size_t x) { return (x + kWorkspaceAlign - 1) / kWorkspaceAlign * kWorkspaceAlign; }
 
 struct SplitPlan {
-  int chunk_rows = 16;
-  int nchunks = 1;
-  int nblk = 1;
+  int nblk = 1;      // 16-row blocks of a row
+  int pv_shift = 8;  // log2 of the rows of a P.V workgroup
+  int pv_fine = 8;   // the least the device may make it
+  int pv_few = 1, pv_many = 1, pv_big = 12;  // SplitArgs
+  int npv = 1;       // P.V workgroups of a row, at most
   int64_t units = 0;
-  size_t off_t = 0, off_m = 0, off_l = 0, off_ml = 0, off_opart = 0, total = 0;
+  size_t off_t = 0, off_st = 0, off_done = 0, off_opart = 0, total = 0;
 };
 
-// P.V waves the VALU split pass aims for.  A wave keeps two sub-blocks of V
-// in flight: 2 * 16 rows of 1 KiB (the wave's heads' share of a row) for
-// G <= 4, half that for G = 8 (8-row sub-blocks), and less again when the
-// batch has fewer KV heads than a wave holds (idle lanes).  The target is
-// 512 waves of the full kind, scaled up by those two factors, so that the V
-// requests in flight per CU stay about the same and the pass runs in one
-// round of long waves: fewer, longer chunks also mean fewer partial outputs
-// to combine.  Measured against a fixed 2048 (µs): B=1 S=131072 Hq=32 Hkv=8
-// D=128 118.4 -> 105.5; B=64 S=4096 200.5 -> 188.7; B=16 Hq=16 Hkv=8 S=8192
-// D=256 186.7 -> 175.5; B=32 Hq=64 Hkv=8 S=8192 234.0 -> 216.5; B=4 Hq=32
-// Hkv=4 S=32768 D=64 (half the lanes idle) 72.0 -> 72.1.
-int64_t split_target_waves(int hq, int hkv, int d) {
-  const int heads_per_wave = kWaveSize / (d / 8);
-  const int g = hq / hkv;
-  const int active = hkv < heads_per_wave ? hkv : heads_per_wave;
-  return (int64_t)512 * (g >= 8 ? 2 : 1) * heads_per_wave / active;
-}
+// The split passes' workspace and the rows of a P.V workgroup: the largest
+// of 256 to 4096 that leaves kPvMinGroups workgroups, about two for each CU
+// (all of them at once: µs of the call at 2048 / 4096 rows, 32/8 B=8 S=32768
+// 194.4 / 192.3, 64/8 218.6 / 207.0; more, shorter ones pay a workgroup's 8
+// us of start and end again: B=1 S=131072, P.V alone, 71 / 59 / 54 at 512 /
+// 1024 / 2048), and divides rows of more than 1024.  Where the lengths turn
+// out to leave fewer than kPvFewGroups (from 4096 rows, 1024 at D = 256, on
+// kPvMinGroups) the device makes it up to four times smaller (row_piece; µs
+// of ragged calls by rows, their workgroups in brackets: B=48 8/1 over
+// 250-8000 rows 26.9 (420) / 25.1 (210) / 26.6 (105) at 256 / 512 / 1024;
+// B=6 64/8 over 1024-32768 64.9 (430) / 63.3 (215) / 73.4 (107) at 1024 /
+// 2048 / 4096; D=64 B=22 8/8 over 666-21321 65.3 (512) / 71.5 (256) at 2048 /
+// 4096; D=256 B=10 8/8 over 360-11516 65.8 (504) / 69.6 (252) at 512 / 1024).
+constexpr int64_t kPvMinGroups = 448, kPvFewGroups = 192;
+constexpr int kPvMinShift = 8, kPvMaxShift = 12;
 
-// Scores: one wave per 16-row block.  P.V: chunks of C rows (C in
-// {64, ..., 1024}, or the rows' own multiple of 16 when shorter), the
-// largest that still gives the pass's target wave count where the work
-// allows.  VALU passes: split_target_waves waves of HPW KV heads (1024 rows
-// against 512 measured 0-3% faster where it keeps that count: B=256 S=1024
-// Hq=32 Hkv=8 192.9 -> 187.9 µs).  Matrix-core passes (kv_groups launch KV
-// heads per cache head): one wave per (batch, cache KV head, chunk, pair of
-// 16-column tiles; one tile at D = 256), 2048 of them for groups of up to 8
-// query heads and 1024 above (whose waves fill their tiles), half that at
-// D = 256 (µs by C = 256 / 512 / 1024: B=8 S=32768 64/8 239/226/223, 40/8
-// 244/233/227; B=64 S=4096 32/4 129/123/122, 64/4 (G = 16) 150/143/136;
-// B=8 S=32768 8/1 48/55/74 (C = 128: 46); D=64 B=32 S=4096 64/8
-// 90/87/91; D=256 B=16 S=4096 64/8 110/108/136; MQA B=8 S=32768 32/1
-// 72/82/111).
-SplitPlan plan_split(int64_t batch, int hq, int hkv, int max_rows, int d, int kv_groups, int layout) {
+SplitPlan plan_split(int64_t batch, int hq, int hkv, int max_rows, int d) {
   SplitPlan p;
   const int heads_per_wave = kWaveSize / (d / 8);
-  const int64_t upb = (hkv + heads_per_wave - 1) / heads_per_wave;
-  p.units = upb * batch;
-  int64_t per_chunk = p.units;  // P.V waves per chunk of every batch
-  int64_t target = split_target_waves(hq, hkv, d);
-  if (split_on_matrix_cores(hq / hkv, kv_groups, layout, hkv, d, max_rows)) {
-    const int hkv_mem = hkv / kv_groups;
-    const int g_mem = hq / hkv_mem;
-    const int tw = d == 256 ? 1 : 2;
-    per_chunk = batch * hkv_mem * (((g_mem + 15) / 16 + tw - 1) / tw);
-    target = (g_mem <= 8 ? 2048 : 1024) / (d == 256 ? 2 : 1);
-  }
-  int c = 1024;
-  while (c > 64 && per_chunk * ((max_rows + c - 1) / c) < target) c /= 2;
-  // Pages of fewer than 16 rows put every row at its own place in memory:
-  // the P.V waves, which walk their chunk a sub-block at a time, then wait
-  // on scattered requests, and shorter chunks (more waves) hide that (µs by
-  // C = 128 / 256 / 512 / 1024 on one-row pages, B=64 S=4096 Hq=32 Hkv=8:
-  // 243/220/227/309; B=8 S=32768: 239/230/256/312; Hq=64 Hkv=8
-  // 268/251/314/387; B=16 S=8192 16/16: 206/193/195/255; matrix cores,
-  // B=64 S=4096 64/4: 245/219/-/274).
-  if (layout == fmha_decode::kLayoutPaged && c > 256) c = 256;
-  // Fewer KV heads than a wave holds, on the VALU passes: a P.V wave's
-  // 2^shift lane groups take chunks of one row, so rows get at least 2^shift
-  // chunks where chunks of 64 rows or more allow it: on paged caches for any
-  // shift (µs, 16-row pages, chunks as before / now: B=2048 S=512 Hq/Hkv
-  // 4/1 192 / 121, B=1024 S=1024 140 / 115, B=2048 S=512 8/2 254 / 216, D=64
-  // 2/1 80 / 65; one-row pages B=2048 S=512 4/1 141 / 118, D=64 2/1 88 /
-  // 64), on packed and strided ones from four lane groups up (packed B=2048
-  // S=512 4/1 123 / 115, D=64 2/1 66 / 62; with two, 8/2, 195 / 210).
-  if (!split_on_matrix_cores(hq / hkv, kv_groups, layout, hkv, d, max_rows)) {
-    int shift = 0;
-    while ((hkv << (shift + 1)) <= heads_per_wave && heads_per_wave % (hkv << (shift + 1)) == 0) ++shift;
-    if (shift >= (fmha_decode::is_paged_layout(layout) ? 1 : 2))
-      while (c > 64 && ((int64_t)c << shift) > max_rows) c /= 2;
-  }
-  // FMHA_DECODE_SPLIT_CHUNK=<64|...|2048> overrides C (for sweeps; the
-  // workspace size follows, and a launch checks its workspace against it).
+  p.units = (hkv + heads_per_wave - 1) / heads_per_wave * batch;
+  const auto groups = [&](int shift) { return max_rows <= 0 ? 1 : ((int64_t)max_rows + (1 << shift) - 1) >> shift; };
+  p.pv_shift = kPvMaxShift;
+  while (p.pv_shift > kPvMinShift &&
+         (batch * hkv * groups(p.pv_shift) < kPvMinGroups || (max_rows > 1024 && groups(p.pv_shift) < 2)))
+    --p.pv_shift;
+  // FMHA_DECODE_SPLIT_CHUNK=<128|...|4096>: rows of a P.V workgroup instead
+  // (for sweeps; the workspace size follows, and a launch checks its
+  // workspace against it).
+  bool forced = false;
   if (const char* e = std::getenv("FMHA_DECODE_SPLIT_CHUNK")) {
     const int v = std::atoi(e);
-    if (v >= 64 && v <= 2048 && (v & (v - 1)) == 0) c = v;
+    forced = v >= 128 && v <= 4096 && (v & (v - 1)) == 0;
+    if (forced) p.pv_shift = fmha_decode::ilog2(v);
   }
-  const int fit = max_rows <= 16 ? 16 : (max_rows + 15) / 16 * 16;  // no longer than the rows need
-  if (c > fit) c = fit;
-  p.chunk_rows = c;
-  p.nchunks = max_rows <= 0 ? 1 : (max_rows + c - 1) / c;
+  const bool adapts = !forced && batch <= fmha_decode::kOrderBatches;
+  p.pv_fine = !adapts || p.pv_shift <= kPvMinShift ? p.pv_shift
+              : p.pv_shift - 2 > kPvMinShift       ? p.pv_shift - 2
+                                                   : kPvMinShift;
+  p.pv_few = (int)((kPvFewGroups + hkv - 1) / hkv);
+  p.pv_many = (int)((kPvMinGroups + hkv - 1) / hkv);
+  p.pv_big = d == 256 ? 10 : 12;
+  p.npv = (int)groups(p.pv_fine);
   p.nblk = max_rows <= 0 ? 1 : (max_rows + fmha_decode::kSplitBlockRows - 1) / fmha_decode::kSplitBlockRows;
   const size_t heads = (size_t)batch * hq;
+  const size_t fans = (size_t)(p.npv + fmha_decode::kPvFan - 1) / fmha_decode::kPvFan;
   size_t off = 0;
   p.off_t = off;
   off += align_up(heads * (size_t)p.nblk * fmha_decode::kSplitBlockRows * 4);
-  p.off_m = off;
-  off += align_up(heads * (size_t)p.nblk * 4);
-  p.off_l = off;
-  off += align_up(heads * (size_t)p.nblk * 4);
-  p.off_ml = off;
-  off += align_up(heads * 2 * 4);
-  p.off_opart = off;
-  if (p.nchunks > 1) off += align_up(heads * (size_t)p.nchunks * d * 4);
+  p.off_st = off;
+  off += align_up(heads * (size_t)p.nblk * 8);
+  if (p.npv > 1) {
+    p.off_done = off;
+    off += align_up((size_t)batch * hkv * (1 + fans) * 4);
+    // Partial outputs of every piece: those of pv_shift rows, or the shorter
+    // ones the device takes, less than twice pv_many and one per batch.
+    const int64_t coarse = batch * groups(p.pv_shift), fine = batch * groups(p.pv_fine);
+    const int64_t few = 2 * (int64_t)p.pv_many + batch;
+    const int64_t pieces = coarse > few ? coarse : (fine < few ? fine : few);
+    p.off_opart = off;
+    off += align_up((size_t)pieces * hq * d * 4);
+  }
   p.total = off;
   return p;
 }
@@ -908,21 +878,14 @@ extern "C" size_t fmha_decode_splitkv_workspace_size(int32_t batch, int32_t num_
       (head_dim != 64 && head_dim != 128 && head_dim != 256))
     return 0;
   const int g = num_heads_q % num_heads_kv == 0 ? num_heads_q / num_heads_kv : 0;
-  // The plan of whichever passes the layout takes: the larger of the packed
-  // layout's and the short-page layout's, which can differ.
-  auto plan_total = [&](int hq, int hkv, int kvg) {
-    const size_t a = plan_split(batch, hq, hkv, max_seqlen_kv, head_dim, kvg, fmha_decode::kLayoutPacked).total;
-    const size_t b = plan_split(batch, hq, hkv, max_seqlen_kv, head_dim, kvg, fmha_decode::kLayoutPaged).total;
-    return a > b ? a : b;
-  };
-  if (g == 0 || valu_group(g)) return plan_total(num_heads_q, num_heads_kv, 1);
+  if (g == 0 || valu_group(g)) return plan_split(batch, num_heads_q, num_heads_kv, max_seqlen_kv, head_dim).total;
   // G > 8: ns groups of 8 per KV head on Hkv * ns launch KV heads; Q and O
   // copies unless G is a multiple of 8.  G = 3, 5-7: the copies padded to
   // 4 or 8, and the plan for Hkv * GP heads.
   const int gp = long_row_group(g);
   const int ns = g > 8 ? gp / 8 : 1;
   const size_t pad = gp == g ? 0 : 2 * group_pad_bytes(batch, num_heads_kv, gp, head_dim);
-  return pad + plan_total(num_heads_kv * gp, num_heads_kv * ns, ns);
+  return pad + plan_split(batch, num_heads_kv * gp, num_heads_kv * ns, max_seqlen_kv, head_dim).total;
 }
 
 namespace {
@@ -931,12 +894,12 @@ namespace {
 // layout-independent fields of the launch.  kv_span_bytes: the largest byte
 // range one wave's K/V descriptor covers in the caller's layout (must stay
 // below 2^30, as must one batch's scores and partial outputs).
-int split_prepare(int layout, const void* Q, const void* K, const void* V, void* O, int32_t max_seqlen_kv,
+int split_prepare(const void* Q, const void* K, const void* V, void* O, int32_t max_seqlen_kv,
                   int32_t batch, int32_t num_heads_q, int32_t num_heads_kv, int32_t kv_groups, int32_t head_dim,
                   float softmax_scale, void* workspace, size_t workspace_bytes, int64_t kv_span_bytes, SplitArgs& a) {
-  const SplitPlan plan = plan_split(batch, num_heads_q, num_heads_kv, max_seqlen_kv, head_dim, kv_groups, layout);
+  const SplitPlan plan = plan_split(batch, num_heads_q, num_heads_kv, max_seqlen_kv, head_dim);
   const int64_t padded_rows = (int64_t)plan.nblk * fmha_decode::kSplitBlockRows;
-  const int64_t part_bytes = (int64_t)num_heads_q * plan.nchunks * head_dim * 4;  // one batch's partials
+  const int64_t part_bytes = (int64_t)num_heads_q * plan.npv * head_dim * 4;  // one batch's partials
   if (kv_span_bytes >= (int64_t(1) << 30) || padded_rows * num_heads_q * 4 >= (int64_t(1) << 30) ||
       part_bytes >= (int64_t(1) << 30))
     return reject(FMHA_DECODE_ERROR_INVALID_VALUE, "max_seqlen_kv too large for this head count (%d)", max_seqlen_kv);
@@ -955,17 +918,20 @@ int split_prepare(int layout, const void* Q, const void* K, const void* V, void*
   a.v = static_cast<const uint16_t*>(V);
   a.o = static_cast<uint16_t*>(O);
   a.t = reinterpret_cast<float*>(ws + plan.off_t);
-  a.m = reinterpret_cast<float*>(ws + plan.off_m);
-  a.l = reinterpret_cast<float*>(ws + plan.off_l);
-  a.ml = reinterpret_cast<float*>(ws + plan.off_ml);
+  a.st = reinterpret_cast<fmha_decode::f32x2_v*>(ws + plan.off_st);
+  a.done = reinterpret_cast<uint32_t*>(ws + plan.off_done);
   a.opart = reinterpret_cast<float*>(ws + plan.off_opart);
   a.num_heads_q = num_heads_q;
   a.num_heads_kv = num_heads_kv;
   a.kv_groups = kv_groups;
   a.units_per_batch = (int32_t)(plan.units / batch);
   a.nblk = plan.nblk;
-  a.nchunks = plan.nchunks;
-  a.chunk_rows = plan.chunk_rows;
+  a.npv = plan.npv;
+  a.pv_shift = plan.pv_shift;
+  a.pv_fine = plan.pv_fine;
+  a.pv_few = plan.pv_few;
+  a.pv_many = plan.pv_many;
+  a.pv_big = plan.pv_big;
   a.max_rows = max_seqlen_kv;
   a.batch = batch;
   a.scale = softmax_scale;
@@ -1125,7 +1091,7 @@ int splitkv_packed(void* stream, const void* Q, const void* K, const void* V, vo
     if (numerics != Numerics::kExact && use_mfma_kernel(num_heads_q / num_heads_kv))
       return launch_mfma(stream, fmha_decode::kLayoutPacked, d, batch, head_dim_q, rows_hint);
     SplitArgs unused;
-    rc = split_prepare(fmha_decode::kLayoutPacked, Q, K, V, O, max_seqlen_kv, batch, num_heads_q, num_heads_kv, 1,
+    rc = split_prepare(Q, K, V, O, max_seqlen_kv, batch, num_heads_q, num_heads_kv, 1,
                        head_dim_q, softmax_scale, workspace, workspace_bytes, span, unused);
     if (rc != FMHA_DECODE_SUCCESS) return rc;
     d.rows_feedback = feedback_word(stream, may_allocate);
@@ -1136,7 +1102,7 @@ int splitkv_packed(void* stream, const void* Q, const void* K, const void* V, vo
       stream, Q, O, batch, num_heads_q, num_heads_kv, head_dim_q, workspace, workspace_bytes,
       [&](const void* q, void* o, int32_t hq, int32_t hkv, int32_t kvg, void* ws, size_t ws_bytes) {
         SplitArgs a;
-        int rc2 = split_prepare(fmha_decode::kLayoutPacked, q, K, V, o, max_seqlen_kv, batch, hq, hkv, kvg,
+        int rc2 = split_prepare(q, K, V, o, max_seqlen_kv, batch, hq, hkv, kvg,
                                 head_dim_q, softmax_scale, ws, ws_bytes, span, a);
         if (rc2 != FMHA_DECODE_SUCCESS) return rc2;
         a.cu = cu_seqlens_kv;
@@ -1251,7 +1217,7 @@ extern "C" int fmha_decode_fwd_splitkv_strided(void* stream, const void* Q, cons
       stream, Q, O, batch, num_heads_q, num_heads_kv, head_dim_q, workspace, workspace_bytes,
       [&](const void* q, void* o, int32_t hq, int32_t hkv, int32_t kvg, void* ws, size_t ws_bytes) {
         SplitArgs a;
-        int rc2 = split_prepare(fmha_decode::kLayoutStrided, q, K, V, o, max_seqlen_kv, batch, hq, hkv, kvg,
+        int rc2 = split_prepare(q, K, V, o, max_seqlen_kv, batch, hq, hkv, kvg,
                                 head_dim_q, softmax_scale, ws, ws_bytes, extent, a);
         if (rc2 != FMHA_DECODE_SUCCESS) return rc2;
         a.cu = seqlens_kv;
@@ -1294,7 +1260,7 @@ extern "C" int fmha_decode_fwd_splitkv_paged(void* stream, const void* Q, const 
       stream, Q, O, batch, num_heads_q, num_heads_kv, head_dim_q, workspace, workspace_bytes,
       [&](const void* q, void* o, int32_t hq, int32_t hkv, int32_t kvg, void* ws, size_t ws_bytes) {
         SplitArgs a;
-        int rc2 = split_prepare(page_layout, q, K_cache, V_cache, o, max_seqlen_kv, batch, hq, hkv, kvg, head_dim_q,
+        int rc2 = split_prepare(q, K_cache, V_cache, o, max_seqlen_kv, batch, hq, hkv, kvg, head_dim_q,
                                 softmax_scale, ws, ws_bytes, 16 * row_bytes, a);
         if (rc2 != FMHA_DECODE_SUCCESS) return rc2;
         a.cu = seqlens_kv;

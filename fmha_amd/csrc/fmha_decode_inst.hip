@@ -2,15 +2,17 @@
 // in fmha_decode_launch.hpp, one slice per compilation: fmha_amd/_build.py
 // compiles this file once for each FMHA_DECODE_PART in [0, FMHA_DECODE_PARTS)
 // and links the objects with fmha_decode_api.hip.  Part 0 holds the kernels
-// every long-row path shares (the split-KV statistics and combine passes, query-group
-// padding); every other part instantiates launchers, and with them kernels,
+// every long-row path shares (query-group padding); every other part instantiates launchers, and with them kernels,
 // that no other part does.
 //
-// FMHA_DECODE_PARTS 63
+// FMHA_DECODE_PARTS 75
 #ifndef FMHA_DECODE_PART
 #error "compile with -DFMHA_DECODE_PART=<part>"
 #endif
 #define FMHA_DECODE_INSTANTIATING
+#if FMHA_DECODE_PART >= 63  // the parts that instantiate launch_split_pv
+#define FMHA_DECODE_INSTANTIATING_PV
+#endif
 #if FMHA_DECODE_PART == 0
 #define FMHA_DECODE_SHARED_KERNELS
 #endif
@@ -20,49 +22,6 @@ namespace fmha_decode {
 namespace host {
 
 #if FMHA_DECODE_PART == 0
-
-// The statistics pass of split-KV: the global max and sum per (batch, query
-// head).  One lane per head for rows of at most 16 blocks, else one
-// workgroup per head sized to the row's block count (8 blocks per thread
-// and round).
-void launch_split_stats(const SplitArgs& a, hipStream_t stream) {
-  const uint32_t heads = (uint32_t)a.batch * (uint32_t)a.num_heads_q;
-  if (a.nblk <= 16)
-    hipLaunchKernelGGL(fmha_decode::splitkv_stats_lane_kernel, dim3((heads + 255) / 256), dim3(256), 0, stream, a);
-  else if (a.nblk <= 8 * 64)
-    hipLaunchKernelGGL(fmha_decode::splitkv_stats_kernel<64>, dim3(heads), dim3(64), 0, stream, a);
-  else if (a.nblk <= 8 * 256)
-    hipLaunchKernelGGL(fmha_decode::splitkv_stats_kernel<256>, dim3(heads), dim3(256), 0, stream, a);
-  else
-    hipLaunchKernelGGL(fmha_decode::splitkv_stats_kernel<1024>, dim3(heads), dim3(1024), 0, stream, a);
-}
-
-// The combine pass of split-KV (more than one chunk per row): partial
-// outputs summed in chunk order, one lane per 8 dims for few chunks, else a
-// workgroup per (head, 32 dims).
-template <int D>
-void launch_split_combine_d(const SplitArgs& a, hipStream_t stream) {
-  const uint32_t heads = (uint32_t)a.batch * (uint32_t)a.num_heads_q;
-  if (a.nchunks <= 16) {
-    const uint64_t lanes = (uint64_t)heads * (D / 8);
-    hipLaunchKernelGGL(fmha_decode::splitkv_combine_kernel<D>, dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0,
-                       stream, a);
-  } else if (a.nchunks <= 256) {
-    hipLaunchKernelGGL((fmha_decode::splitkv_combine_block_kernel<D, 256>), dim3(heads * (D / 32)), dim3(256), 0,
-                       stream, a);
-  } else {
-    hipLaunchKernelGGL((fmha_decode::splitkv_combine_block_kernel<D, 1024>), dim3(heads * (D / 32)), dim3(1024), 0,
-                       stream, a);
-  }
-}
-
-void launch_split_combine(const SplitArgs& a, int d, hipStream_t stream) {
-  switch (d) {
-    case 64: return launch_split_combine_d<64>(a, stream);
-    case 128: return launch_split_combine_d<128>(a, stream);
-    default: return launch_split_combine_d<256>(a, stream);
-  }
-}
 
 hipError_t launch_pad_query_group(const uint16_t* q, uint16_t* qp, uint64_t streams, int G, int GP, int D,
                                   hipStream_t stream) {
@@ -207,6 +166,30 @@ template hipError_t launch_exact<256, 2>(const DecodeArgs&, bool, int, int, hipS
 template hipError_t launch_exact<256, 4>(const DecodeArgs&, bool, int, int, hipStream_t);
 #elif FMHA_DECODE_PART == 62
 template hipError_t launch_exact<256, 8>(const DecodeArgs&, bool, int, int, hipStream_t);
+#elif FMHA_DECODE_PART == 63
+template hipError_t launch_split_pv<64, kLayoutPacked>(const SplitArgs&, hipStream_t);
+#elif FMHA_DECODE_PART == 64
+template hipError_t launch_split_pv<64, kLayoutStrided>(const SplitArgs&, hipStream_t);
+#elif FMHA_DECODE_PART == 65
+template hipError_t launch_split_pv<64, kLayoutPaged>(const SplitArgs&, hipStream_t);
+#elif FMHA_DECODE_PART == 66
+template hipError_t launch_split_pv<64, kLayoutPagedBlock>(const SplitArgs&, hipStream_t);
+#elif FMHA_DECODE_PART == 67
+template hipError_t launch_split_pv<128, kLayoutPacked>(const SplitArgs&, hipStream_t);
+#elif FMHA_DECODE_PART == 68
+template hipError_t launch_split_pv<128, kLayoutStrided>(const SplitArgs&, hipStream_t);
+#elif FMHA_DECODE_PART == 69
+template hipError_t launch_split_pv<128, kLayoutPaged>(const SplitArgs&, hipStream_t);
+#elif FMHA_DECODE_PART == 70
+template hipError_t launch_split_pv<128, kLayoutPagedBlock>(const SplitArgs&, hipStream_t);
+#elif FMHA_DECODE_PART == 71
+template hipError_t launch_split_pv<256, kLayoutPacked>(const SplitArgs&, hipStream_t);
+#elif FMHA_DECODE_PART == 72
+template hipError_t launch_split_pv<256, kLayoutStrided>(const SplitArgs&, hipStream_t);
+#elif FMHA_DECODE_PART == 73
+template hipError_t launch_split_pv<256, kLayoutPaged>(const SplitArgs&, hipStream_t);
+#elif FMHA_DECODE_PART == 74
+template hipError_t launch_split_pv<256, kLayoutPagedBlock>(const SplitArgs&, hipStream_t);
 #else
 #error "FMHA_DECODE_PART out of range"
 #endif

@@ -21,6 +21,7 @@
 #include "fmha_decode_onepass.hpp"
 #include "fmha_decode_splitkv.hpp"
 #include "fmha_decode_splitkv_group.hpp"
+#include "fmha_decode_splitkv_pv.hpp"
 
 namespace fmha_decode {
 namespace host {
@@ -247,16 +248,13 @@ hipError_t launch_mfma_layout(const fmha_decode::GroupArgs& g, int dq, int ns, i
   }
 }
 
-// Per-CU wave caps of the two streaming passes (dynamic LDS reservation).
-// Scores waves request 16 KiB of K plus G KiB of Q at once; P.V waves keep
-// two 16-row (8-row for G = 8) sub-blocks of V in flight.  Swept apart
-// (µs at scores caps 4 / 6 / 8 / 12 / 16, P.V at 8; Hq/Hkv 32/8 D=128):
-// B=64 S=4096 210.8/192.7/190.9/188.7/187.9, B=8 S=32768
-// 213.9/194.0/191.7/189.9/190.3, B=1 S=131072 116.8/107.7/106.7/104.4/105.2;
-// Hq=Hkv=16 B=16 S=8192 and the matrix-core passes (64/8 B=256 S=1024)
-// flat from 6 up.  P.V caps of 4-12 are within 1% everywhere.
+// Per-CU wave cap of the scores launch (dynamic LDS reservation): its waves
+// request 16 KiB of K plus G KiB of Q at once (µs at caps 4 / 6 / 8 / 12 /
+// 16, Hq/Hkv 32/8 D=128: B=64 S=4096 210.8/192.7/190.9/188.7/187.9, B=8
+// S=32768 213.9/194.0/191.7/189.9/190.3, B=1 S=131072
+// 116.8/107.7/106.7/104.4/105.2; Hq=Hkv=16 B=16 S=8192 and the matrix-core
+// pass flat from 6 up).
 constexpr int kSplitScoresWavesPerCU = 12;
-constexpr int kSplitPvWavesPerCU = 8;
 
 // Rows longer than 16 go through one pass (onepass_decode_kernel: one wave
 // per batch and head group, no workspace traffic, one launch) when there are
@@ -449,17 +447,63 @@ hipError_t launch_onepass_group(const SplitArgs& a, hipStream_t stream) {
 
 // Launchers of the kernels every long-row path shares, defined once in the
 // part that owns them (fmha_decode_inst.hip, FMHA_DECODE_PART 0).
-// The statistics pass of split-KV (rows of more than kPvStatBlocks blocks):
-// the global max and sum per (batch, query head).
-void launch_split_stats(const SplitArgs& a, hipStream_t stream);
-// The combine pass of split-KV (more than one chunk per row): the partial
-// outputs summed in chunk order.
-void launch_split_combine(const SplitArgs& a, int d, hipStream_t stream);
-
-// Rows of up to this many 16-row blocks: every split-KV P.V wave reduces its
-// heads' block statistics itself (no statistics pass; µs with the pass /
-// without: B=256 S=1024 Hq/Hkv 64/8 222 / 218, B=128 S=256 32/8 41 / 37).
+// Rows of more than this many 16-row blocks count their statistics as a pass
+// of the plan text: joining them takes a P.V workgroup more than one load.
 constexpr int kPvStatBlocks = 64;
+
+// P.V workgroups of the longest row as the plan has it.
+inline int split_groups(const SplitArgs& a) { return (a.max_rows + (1 << a.pv_shift) - 1) >> a.pv_shift; }
+// Phases of a split-KV plan, for its text: scores, the statistics of rows of
+// more than kPvStatBlocks blocks, P.V, and the sum over the workgroups of a
+// row with more than one.
+inline int split_passes(const SplitArgs& a) { return 2 + (a.nblk > kPvStatBlocks) + (split_groups(a) > 1); }
+// The rows of one P.V wave's share (chunk) of the longest row, for its text:
+// the row itself, rounded up to blocks, with one workgroup per row.
+inline int split_chunk_rows(const SplitArgs& a) {
+  return split_groups(a) > 1 ? (1 << a.pv_shift) / fmha_decode::kPvWaves : a.nblk * fmha_decode::kSplitBlockRows;
+}
+inline int split_chunks(const SplitArgs& a) {
+  return split_groups(a) > 1 ? (a.max_rows + split_chunk_rows(a) - 1) / split_chunk_rows(a) : 1;
+}
+
+// The P.V launch of split-KV (splitkv_pv_kernel) after the scores launch of
+// either kind; instantiated in its own parts, which the others link to.
+template <int D, int LAYOUT>
+hipError_t launch_split_pv(const SplitArgs& a, hipStream_t stream) {
+  const int g = a.num_heads_q / a.num_heads_kv;
+  const int64_t tiles = (g + 15) / 16;
+  const int64_t units = (int64_t)a.batch * a.npv * a.num_heads_kv;
+  const int64_t groups = (units + 7) / 8 * 8 * tiles;
+  if (groups > INT32_MAX) return hipErrorInvalidValue;
+  const dim3 grid((uint32_t)groups);
+  const dim3 block(a.max_rows <= fmha_decode::kPvOneWaveRows ? kBlockThreads : fmha_decode::kPvThreads);
+  if (g <= 1)
+    hipLaunchKernelGGL((fmha_decode::splitkv_pv_kernel<D, 1, LAYOUT>), grid, block, 0, stream, a);
+  else if (g <= 2)
+    hipLaunchKernelGGL((fmha_decode::splitkv_pv_kernel<D, 2, LAYOUT>), grid, block, 0, stream, a);
+  else if (g <= 4)
+    hipLaunchKernelGGL((fmha_decode::splitkv_pv_kernel<D, 4, LAYOUT>), grid, block, 0, stream, a);
+  else if (g <= 8)
+    hipLaunchKernelGGL((fmha_decode::splitkv_pv_kernel<D, 8, LAYOUT>), grid, block, 0, stream, a);
+  else
+    hipLaunchKernelGGL((fmha_decode::splitkv_pv_kernel<D, 16, LAYOUT>), grid, block, 0, stream, a);
+  return hipGetLastError();
+}
+
+#ifndef FMHA_DECODE_INSTANTIATING_PV
+extern template hipError_t launch_split_pv<64, kLayoutPacked>(const SplitArgs&, hipStream_t);
+extern template hipError_t launch_split_pv<64, kLayoutStrided>(const SplitArgs&, hipStream_t);
+extern template hipError_t launch_split_pv<64, kLayoutPaged>(const SplitArgs&, hipStream_t);
+extern template hipError_t launch_split_pv<64, kLayoutPagedBlock>(const SplitArgs&, hipStream_t);
+extern template hipError_t launch_split_pv<128, kLayoutPacked>(const SplitArgs&, hipStream_t);
+extern template hipError_t launch_split_pv<128, kLayoutStrided>(const SplitArgs&, hipStream_t);
+extern template hipError_t launch_split_pv<128, kLayoutPaged>(const SplitArgs&, hipStream_t);
+extern template hipError_t launch_split_pv<128, kLayoutPagedBlock>(const SplitArgs&, hipStream_t);
+extern template hipError_t launch_split_pv<256, kLayoutPacked>(const SplitArgs&, hipStream_t);
+extern template hipError_t launch_split_pv<256, kLayoutStrided>(const SplitArgs&, hipStream_t);
+extern template hipError_t launch_split_pv<256, kLayoutPaged>(const SplitArgs&, hipStream_t);
+extern template hipError_t launch_split_pv<256, kLayoutPagedBlock>(const SplitArgs&, hipStream_t);
+#endif
 
 // Q rows copied to, and O rows back from, a query group padded to GP rows
 // per (batch, KV head) stream (fmha_decode_group.hpp).
@@ -653,11 +697,12 @@ int onepass_reg_tiles(const SplitArgs& a) {
   }
 }
 
-// Longest rows first (SplitArgs::longest_first) with more waves than the CUs
-// hold at once (8 each at 16 and 32 tiles per wave), where the order decides
-// what the launch ends on; below, every workgroup starts at once, and the
-// lengths' extra round trip costs (µs, B=128 S=256 32/8, 2048 waves, all rows
-// equal: 25.9 without, 27.3 with).
+// Longest rows first (SplitArgs::longest_first) at 16 and 32 tiles per wave
+// with more waves than the CUs hold at once (8 each), where the order decides
+// what the launch ends on; below, every workgroup starts at once, or (8
+// tiles) ends soon, and the lengths' extra round trip costs (µs, all rows
+// equal, without / with: B=128 S=256 32/8 25.9 / 27.3, BHSD B=100 S=512
+// 16/16 69.8 / 72.9; ragged B=256 64/8 over 16-500 rows 46.4 either way).
 constexpr int kOrderWavesPerCU = 8;
 
 template <int D, int LAYOUT>
@@ -671,7 +716,7 @@ hipError_t launch_onepass_reg(const SplitArgs& args, int tpw, hipStream_t stream
   const int64_t units = (int64_t)a.batch * a.num_heads_kv;
   const int64_t cus = device_cus() > 0 ? device_cus() : 256;
   a.longest_first = a.len_mode != fmha_decode::kLenUniform && a.batch > 1 && a.batch <= fmha_decode::kOrderBatches &&
-                    units * nw > kOrderWavesPerCU * cus;
+                    tpw > 8 && units * nw > kOrderWavesPerCU * cus;
   const uint32_t round_tiles = (uint32_t)(nw * fmha_decode::onepass_reg_round_tiles(D, tpw, LAYOUT));
   a.round_inv = (65536u + round_tiles - 1) / round_tiles;
   const dim3 grid((uint32_t)units);
@@ -862,47 +907,21 @@ hipError_t launch_split_dg(const SplitArgs& a, hipStream_t stream, bool onepass_
     // Too few units for one wave each: two waves per unit.
     if (group_fits) return launch_onepass_group<D, G, LAYOUT>(ag, stream);
   }
-  // P.V sub-block rows (register budget: pages under 16 rows address every
-  // row on its own, a descriptor or a 64-bit address per row; 16 rows there
-  // leave one wave per SIMD).
-  constexpr int NR = G >= 8 || LAYOUT == fmha_decode::kLayoutPaged || LAYOUT == fmha_decode::kLayoutPagedLanes ? 8 : 16;
   SplitArgs as = a;
   as.sub_shift = shift;
   as.units_per_batch = (a.num_heads_kv + (HPW >> shift) - 1) / (HPW >> shift);
-  const int64_t upb = as.units_per_batch;
-  as.stat_pass = a.nblk > kPvStatBlocks;
-  const int64_t score_waves = (int64_t)a.batch * ((a.nblk + (1 << shift) - 1) >> shift) * upb;
-  const int64_t nwc = (a.nchunks + (1 << shift) - 1) >> shift;  // P.V waves per unit
-  const int64_t pv_waves = (int64_t)a.batch * nwc * upb;
-  if (score_waves > INT32_MAX || pv_waves > INT32_MAX) return hipErrorInvalidValue;
-  // The combine grid has one workgroup per (batch, query head, 32 dims).
-  if ((uint64_t)a.batch * (uint64_t)a.num_heads_q * (D / 32) > UINT32_MAX) return hipErrorInvalidValue;
-  const int passes = 2 + as.stat_pass + (a.nchunks > 1);
-  plan_note("split(D=%d G=%d layout=%s sub_units=%d blocks=%d chunk_rows=%d chunks=%d passes=%d)", D, G,
-            layout_name(LAYOUT), 1 << shift, a.nblk, a.chunk_rows, a.nchunks, passes);
-  {
-    constexpr auto kernel = fmha_decode::splitkv_scores_kernel<D, G, LAYOUT>;
-    hipLaunchKernelGGL(kernel, dim3((uint32_t)score_waves), dim3(kBlockThreads),
-                       lds_reserve_kernel<kernel>(kSplitScoresWavesPerCU), stream, as);
-  }
-  if (as.stat_pass) launch_split_stats(as, stream);
-  if (a.nchunks == 1) {
-    // One chunk per batch: the P.V wave writes O itself, one chunk per wave.
-    constexpr auto kernel = fmha_decode::splitkv_pv_kernel<D, G, NR, true, LAYOUT>;
-    SplitArgs ad = a;
-    ad.stat_pass = as.stat_pass;
-    const uint32_t waves = (uint32_t)a.batch * (uint32_t)a.units_per_batch;
-    hipLaunchKernelGGL(kernel, dim3(waves), dim3(kBlockThreads), lds_reserve_kernel<kernel>(kSplitPvWavesPerCU),
-                       stream, ad);
-    return hipGetLastError();
-  }
-  {
-    constexpr auto kernel = fmha_decode::splitkv_pv_kernel<D, G, NR, false, LAYOUT>;
-    hipLaunchKernelGGL(kernel, dim3((uint32_t)pv_waves), dim3(kBlockThreads),
-                       lds_reserve_kernel<kernel>(kSplitPvWavesPerCU), stream, as);
-  }
-  launch_split_combine(a, D, stream);
-  return hipGetLastError();
+  const int wpg = (a.nblk >> shift) > fmha_decode::kScoresLongBlocks ? fmha_decode::kScoresMaxWaves : 1;
+  as.sup_shift = 4 + shift + fmha_decode::ilog2(wpg);
+  as.nsup = (a.max_rows + (1 << as.sup_shift) - 1) >> as.sup_shift;
+  const int64_t groups = (int64_t)a.batch * as.nsup * as.units_per_batch;
+  if (groups > INT32_MAX) return hipErrorInvalidValue;
+  plan_note("split(D=%d G=%d layout=%s sub_units=%d blocks=%d chunk_rows=%d chunks=%d passes=%d launches=2)", D, G,
+            layout_name(LAYOUT), 1 << shift, a.nblk, split_chunk_rows(a), split_chunks(a), split_passes(a));
+  constexpr auto kernel = fmha_decode::splitkv_scores_kernel<D, G, LAYOUT>;
+  hipLaunchKernelGGL(kernel, dim3((uint32_t)groups), dim3(kBlockThreads * wpg),
+                     lds_reserve_kernel<kernel>(kSplitScoresWavesPerCU / wpg), stream, as);
+  const hipError_t err = hipGetLastError();
+  return err != hipSuccess ? err : launch_split_pv<D, RegLayout<LAYOUT>>(as, stream);
 }
 
 template <int D, int LAYOUT>
@@ -924,12 +943,9 @@ hipError_t launch_split_layout(const SplitArgs& a, int d, int g, hipStream_t str
   }
 }
 
-// Split-KV on the matrix cores (fmha_decode_splitkv_group.hpp): a's KV heads
-// are the cache's (kv_groups = 1) and G = num_heads_q / num_heads_kv any
-// size.  Scores, the statistics pass for rows of more than kPvStatBlocks
-// blocks, P.V (O directly with one chunk per row), combine.
-// P.V waves take TW tiles of 16 query heads, their accumulators TW * D/16 *
-// 4 VGPRs: 2 tiles (G <= 32 in one wave) at D = 64 and 128, one at D = 256.
+// Split-KV with the scores on the matrix cores
+// (fmha_decode_splitkv_group.hpp): a's KV heads are the cache's (kv_groups =
+// 1) and G = num_heads_q / num_heads_kv any size.
 template <int D, int LAYOUT>
 hipError_t launch_split_group_d(const SplitArgs& a, hipStream_t stream) {
   if constexpr (LAYOUT == fmha_decode::kLayoutPacked || LAYOUT == fmha_decode::kLayoutStrided ||
@@ -939,39 +955,19 @@ hipError_t launch_split_group_d(const SplitArgs& a, hipStream_t stream) {
                 LAYOUT == fmha_decode::kLayoutPagedBlock)
     if (const int nw = onepass_mfma_waves<D, LAYOUT>(a)) return launch_onepass_mfma<D, LAYOUT>(a, nw, stream);
   constexpr int HPW = kWaveSize / (D / 8);
-  constexpr int TW = D == 256 ? 1 : 2;
-  const int64_t g = a.num_heads_q / a.num_heads_kv;
-  const int64_t tiles = (g + 15) / 16;
-  const int64_t tc = (tiles + TW - 1) / TW;
-  const int64_t score_waves = (int64_t)a.batch * ((a.nblk + HPW - 1) / HPW) * a.num_heads_kv;
-  const int64_t units = (int64_t)a.batch * a.nchunks * a.num_heads_kv;
-  const int64_t pv_waves = (units + 7) / 8 * 8 * tc;
-  if (score_waves > INT32_MAX || pv_waves > INT32_MAX ||
-      (uint64_t)a.batch * (uint64_t)a.num_heads_q * (D / 32) > UINT32_MAX)
-    return hipErrorInvalidValue;
   SplitArgs am = a;
-  am.stat_pass = a.nblk > kPvStatBlocks;
-  plan_note("split_matrix_core(D=%d G=%d layout=%s blocks=%d chunk_rows=%d chunks=%d passes=%d)", D, (int)g,
-            layout_name(LAYOUT), a.nblk, a.chunk_rows, a.nchunks, 2 + am.stat_pass + (a.nchunks > 1));
-  {
-    constexpr auto kernel = fmha_decode::splitkv_scores_group_kernel<D, LAYOUT>;
-    hipLaunchKernelGGL(kernel, dim3((uint32_t)score_waves), dim3(kBlockThreads),
-                       lds_reserve_kernel<kernel>(kSplitScoresWavesPerCU), stream, am);
-  }
-  if (am.stat_pass) launch_split_stats(am, stream);
-  if (a.nchunks == 1) {
-    constexpr auto kernel = fmha_decode::splitkv_pv_group_kernel<D, TW, true, LAYOUT>;
-    hipLaunchKernelGGL(kernel, dim3((uint32_t)pv_waves), dim3(kBlockThreads),
-                       lds_reserve_kernel<kernel>(kSplitPvWavesPerCU), stream, am);
-    return hipGetLastError();
-  }
-  {
-    constexpr auto kernel = fmha_decode::splitkv_pv_group_kernel<D, TW, false, LAYOUT>;
-    hipLaunchKernelGGL(kernel, dim3((uint32_t)pv_waves), dim3(kBlockThreads),
-                       lds_reserve_kernel<kernel>(kSplitPvWavesPerCU), stream, am);
-  }
-  launch_split_combine(a, D, stream);
-  return hipGetLastError();
+  am.sup_shift = 4 + fmha_decode::ilog2(HPW);
+  am.nsup = (a.max_rows + (1 << am.sup_shift) - 1) >> am.sup_shift;
+  const int64_t groups = (int64_t)a.batch * am.nsup * a.num_heads_kv;
+  if (groups > INT32_MAX) return hipErrorInvalidValue;
+  plan_note("split_matrix_core(D=%d G=%d layout=%s blocks=%d chunk_rows=%d chunks=%d passes=%d launches=2)", D,
+            a.num_heads_q / a.num_heads_kv, layout_name(LAYOUT), a.nblk, split_chunk_rows(a), split_chunks(a),
+            split_passes(a));
+  constexpr auto kernel = fmha_decode::splitkv_scores_group_kernel<D, LAYOUT>;
+  hipLaunchKernelGGL(kernel, dim3((uint32_t)groups), dim3(kBlockThreads),
+                     lds_reserve_kernel<kernel>(kSplitScoresWavesPerCU), stream, am);
+  const hipError_t err = hipGetLastError();
+  return err != hipSuccess ? err : launch_split_pv<D, LAYOUT>(am, stream);
 }
 
 template <int LAYOUT>

@@ -5,40 +5,36 @@
 // scores, max-subtracted softmax, weights rounded to bf16 *after*
 // normalisation (as the reference's CPU loop does, fmha_host.cpp:209-226),
 // fp32 P.V, one fp16 rounding.  Because the bf16 rounding needs the global
-// max and sum before any weight is formed, the work runs in two to four
-// launches over a caller-provided workspace:
+// max and sum before any weight is formed, the work runs in two launches
+// over a caller-provided workspace:
 //
-//   1. scores:  one wave per (batch, block of 16 rows, KV-head group): the
-//               block's Q and K rows are requested at once (as in the short
-//               kernel), dot products, transposing butterfly (shared with
-//               the short kernel); scaled scores t_j -> T, and per query head
-//               the block's max m_b and sum l_b of exp(t_j - m_b).
-//   2. stats:   rows of more than kPvStatBlocks blocks only: one workgroup
-//               per (batch, query head): m = max_b m_b, L = sum_b l_b *
-//               exp(m_b - m), loads batched, reduction order fixed
-//               (deterministic).  Shorter rows skip it: each P.V wave
-//               reduces its heads' block statistics itself (row_stats).
-//   3. pv:      one wave per (batch, chunk of C rows, KV-head group), walking
-//               the chunk in sub-blocks of NR rows with two register sets:
-//               the next sub-block's V rows and scores are in flight while
-//               the current one is processed.  The 64 lanes form
-//               P_j = bf16(exp(t_j - m) / L) for the wave's heads into LDS,
-//               then packed dot2 accumulation; the chunk's fp32 partial
-//               output -> Opart, or fp16 O directly when every batch fits one
-//               chunk.
-//   4. combine: more than one chunk per row only: O = fp16(sum_c Opart),
-//               chunks added in order.
+//   1. scores (this file; groups of 8 and more on the matrix cores in
+//      fmha_decode_splitkv_group.hpp): workgroups of a few waves, one wave
+//      per block of 16 rows and KV-head group: the block's Q and K rows are
+//      requested at once (as in the short kernel), dot products, transposing
+//      butterfly (shared with the short kernel); scaled scores t_j -> T, and
+//      per query head the max m and the sum of exp(t_j - m) of the
+//      workgroup's rows, joined through LDS.
+//   2. P.V (fmha_decode_splitkv_pv.hpp): workgroups of eight waves, each
+//      joining its row's statistics, weighting a chunk of V rows and, with
+//      more than one workgroup per row, leaving a partial output; the last
+//      one of a row to finish adds them.
 //
-// The combine stays a launch of its own: folding it into pass 3 (the last
-// P.V wave of a row, found with an atomic counter, summing the partials)
-// needs an agent-scope release fence in every P.V wave, an L2 writeback
-// that measured about 350 ns of serialised L2 time per wave (B=256 S=1024
-// Hq/Hkv 64/8 with 4 chunks per row: 584 against 250 µs; B=1 S=131072
-// 32/8, 256 chunks: 137 against 106 µs).
+// The statistics and the partial outputs once had launches of their own;
+// four launches cost a short row more than its bytes (µs of kernels, B=1
+// S=3001 32/8 on 16-row pages 20.9 -> 14.1, B=8 of 47-1500 rows 16/16 D=64
+// BHSD 17.0 -> 11.8, ragged B=48 8/1 over 250-8000 rows 34.6 -> 24; long rows
+// keep their time, B=1 S=131072 104.6 -> 104.3, or gain with groups of 8,
+// B=8 S=32768 64/8 221 -> 207).  P.V workgroups find their batch in the
+// lengths (row_piece), so that those past the rows of a ragged batch come
+// last and end at once, where a grid over the longest row interleaves them
+// with the others (µs, B=6 64/8 over 1024-32768 rows on 16-row pages 80.1 /
+// 62.9; 84 with four launches); the scores launch's waves are too short for
+// the extra round trip (B=8 S=32768 32/8 92 / 97).
 //
 // K and V are each read once; T adds 4 bytes per row and query head (written
-// by 1, read by 3), the block statistics 8 bytes per 16 rows and query head,
-// Opart 4*D bytes per chunk and query head.
+// by 1, read by 2), the statistics 8 bytes per workgroup of 1 and query head
+// and the partial outputs 4*D bytes per workgroup of 2 and query head.
 #pragma once
 
 #include <type_traits>
@@ -52,6 +48,11 @@ constexpr int kLenCu = 0;       // cu[b + 1] - cu[b] (packed layout)
 constexpr int kLenArray = 1;    // cu[b] holds the length itself
 constexpr int kLenUniform = 2;  // every batch has max_rows rows
 
+typedef float f32x2_v __attribute__((ext_vector_type(2)));
+
+// P.V workgroups of a row whose partial outputs one of them adds.
+constexpr int kPvFan = 16;
+
 struct SplitArgs {
   const uint16_t* q;      // [batch, Hq, D] bf16
   const uint16_t* k;      // bf16 K rows in the launch's layout (LongRows)
@@ -59,16 +60,21 @@ struct SplitArgs {
   uint16_t* o;            // [batch, Hq, D] fp16
   const int32_t* cu;      // packed: [batch+1] row offsets; else [batch] lengths (or null, uniform)
   float* t;               // [batch, nblk, Hq, 16] scaled scores
-  float* m;               // [batch, Hq, nblk] block max
-  float* l;               // [batch, Hq, nblk] block sum of exp(t - m_b)
-  float* ml;              // [batch, Hq, 2] global max, global sum
-  float* opart;           // [batch, Hq, nchunks, D] partial outputs
+  f32x2_v* st;            // [batch, Hq, nsup] max and sum of exp(t - max) of nsup-th parts of a row
+  float* opart;           // [P.V pieces, Hkv, G, D] partial outputs
+  uint32_t* done;         // [batch, Hkv, tiles, 1 + ceil(npv / kPvFan)] finished P.V workgroups
   int32_t num_heads_q;
   int32_t num_heads_kv;
   int32_t units_per_batch;  // KV-head groups per batch: ceil(Hkv / HPW)
   int32_t nblk;           // 16-row blocks per batch row: ceil(max_rows / 16)
-  int32_t nchunks;        // P.V chunks per batch row: ceil(max_rows / chunk_rows)
-  int32_t chunk_rows;     // C, a multiple of 16
+  int32_t npv;            // P.V workgroups of the longest row, at most: ceil(max_rows / 2^pv_fine)
+  int32_t pv_shift;       // log2 of the rows of a P.V workgroup
+  int32_t pv_fine;        // the least it may be made on the device (row_piece)
+  int32_t pv_few;         // per KV head, the workgroups below which it is,
+  int32_t pv_many;        // and those below which it is from pv_big on
+  int32_t pv_big;
+  int32_t sup_shift;      // log2 of the rows of a scores workgroup
+  int32_t nsup;           // scores workgroups per batch row: ceil(max_rows / 2^sup_shift)
   int32_t max_rows;       // lengths above this are invalid (NaN output)
   int32_t batch;
   float scale;
@@ -82,17 +88,14 @@ struct SplitArgs {
   const int32_t* block_table;
   int32_t bt_stride;
   int32_t page_shift;
-  // log2 of the sub-units per wave (scores, P.V): with fewer KV heads than a
-  // wave holds, its lane groups take 2^sub_shift blocks (scores) or chunks
-  // (P.V) of the same heads instead of idling (packed and strided layouts).
+  // log2 of the sub-units per wave (scores, single pass): with fewer KV
+  // heads than a wave holds, its lane groups take 2^sub_shift blocks
+  // (scores) of the same heads, or batches (single pass), instead of idling.
   int32_t sub_shift;
   // Launch KV heads per KV head in memory (>= 1): a query group larger than
   // the kernels' G runs as kv_groups groups of G on one launch, launch head
   // hk reading memory head hk / kv_groups of num_heads_kv / kv_groups.
   int32_t kv_groups;
-  // 1: the statistics pass ran and ml holds each head's global max and sum;
-  // 0: every P.V wave reduces its heads' block statistics (m, l) itself.
-  int32_t stat_pass;
   // Register single pass: 1: workgroups take the batches longest row first
   // (longest_first; at most kOrderBatches batches), 0: as they come.
   int32_t longest_first;
@@ -134,32 +137,44 @@ __device__ __forceinline__ int split_len_l(const SplitArgs& a, uint64_t b) {
 
 constexpr int kSplitBlockRows = kMaxSeq;  // rows per scores wave
 
+// The lengths of all of a call's batches (at most kOrderBatches), batch p *
+// kWaveSize + lane in len[p]; 0 past the last.  Every load is requested at
+// once, with no branch between them.
+constexpr int kOrderBatches = 256;
+constexpr int kOrderRegs = kOrderBatches / kWaveSize;
+
+template <int LAYOUT>
+__device__ __forceinline__ void batch_lengths(const SplitArgs& a, int lane, int (&len)[kOrderRegs]) {
+#pragma unroll
+  for (int p = 0; p < kOrderRegs; ++p)
+    len[p] = split_len_l<LAYOUT>(a, (uint64_t)min(p * kWaveSize + lane, a.batch - 1));
+#pragma unroll
+  for (int p = 0; p < kOrderRegs; ++p)
+    if (p * kWaveSize + lane >= a.batch) len[p] = 0;
+}
+
 // The batch that workgroup group i (< batch) of a single-pass launch serves
 // with SplitArgs::longest_first: the one with the i-th longest row, in 16-row
 // blocks, ties in batch order, so that the longest rows start first and the
 // launch does not end on one of them alone.  Every lane of the wave calls it;
 // every wave of every workgroup finds the same order.
-constexpr int kOrderBatches = 256;
-
 template <int LAYOUT>
 __device__ __forceinline__ uint32_t longest_first(const SplitArgs& a, uint32_t i, int lane) {
-  constexpr int NP = kOrderBatches / kWaveSize;
   if (__builtin_expect(!a.longest_first, 1)) return i;  // the search stays out of the other launches' straight-line code
-  int blocks[NP];  // -1: no batch
+  int blocks[kOrderRegs];  // -1: no batch
+  batch_lengths<LAYOUT>(a, lane, blocks);
 #pragma unroll
-  for (int p = 0; p < NP; ++p) {
-    const int b = p * kWaveSize + lane;
-    blocks[p] = -1;
-    if (b < a.batch) {
-      const int S = split_len_l<LAYOUT>(a, (uint64_t)b);
-      blocks[p] = S < 0 || S > a.max_rows ? 0 : (S + kSplitBlockRows - 1) / kSplitBlockRows;
-    }
+  for (int p = 0; p < kOrderRegs; ++p) {
+    const int S = blocks[p];
+    blocks[p] = p * kWaveSize + lane >= a.batch ? -1
+                : S < 0 || S > a.max_rows       ? 0
+                                                : (S + kSplitBlockRows - 1) / kSplitBlockRows;
   }
   // Rows of at least v blocks, as a count over the wave.
   auto at_least = [&](int v) {
     int n = 0;
 #pragma unroll
-    for (int p = 0; p < NP; ++p) n += __popcll(__builtin_amdgcn_ballot_w64(blocks[p] >= v));
+    for (int p = 0; p < kOrderRegs; ++p) n += __popcll(__builtin_amdgcn_ballot_w64(blocks[p] >= v));
     return n;
   };
   // One length for all: as they come.
@@ -172,7 +187,7 @@ __device__ __forceinline__ uint32_t longest_first(const SplitArgs& a, uint32_t i
   int r = (int)i - at_least(v + 1);  // its place among the rows of v blocks
   uint32_t found = i;
 #pragma unroll
-  for (int p = 0; p < NP; ++p) {
+  for (int p = 0; p < kOrderRegs; ++p) {
     const uint64_t m = __builtin_amdgcn_ballot_w64(blocks[p] == v);
     const int n = __popcll(m);
     if (r >= 0 && r < n) {
@@ -183,6 +198,108 @@ __device__ __forceinline__ uint32_t longest_first(const SplitArgs& a, uint32_t i
     r -= n;
   }
   return found;
+}
+
+// Wave barrier between LDS writes and reads of one wave.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// What a workgroup of the split passes serves.
+struct RowPiece {
+  uint32_t b;      // batch
+  uint32_t piece;  // rows [piece << shift, (piece + 1) << shift) of it
+  int S;           // its length (maybe invalid)
+  int shift;
+};
+
+// Piece u of a call with `pieces` (those of the longest row) for each batch;
+// false for a batch's unused ones, but its first.
+template <int LAYOUT>
+__device__ __forceinline__ bool batch_piece(const SplitArgs& a, uint32_t u, int shift, uint32_t pieces, RowPiece& out) {
+  out.b = u / pieces;
+  if (out.b >= (uint32_t)a.batch) return false;
+  out.piece = u - out.b * pieces;
+  out.S = split_len_l<LAYOUT>(a, out.b);
+  out.shift = shift;
+  return out.piece == 0 || (out.S <= a.max_rows && (int)(out.piece << shift) < out.S);
+}
+
+// Sums of x over lanes 0 .. this one.
+__device__ __forceinline__ int wave_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);   // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);   // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);   // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return x;
+}
+
+// The P.V workgroups' pieces: piece u of a call whose batches have max(1,
+// ceil(S / 2^shift)) each (one for an empty or invalid batch), in batch order;
+// false past the last.  Up to kOrderBatches batches the wave adds up the
+// pieces of the lengths, so that the workgroups past the rows that exist are
+// the last of the grid, and takes shorter pieces than the host, which saw
+// only the longest row allowed, where they would leave CUs without one (µs,
+// B=30 8/8 over 140-4500 rows 45.3 with the host's 2048 rows, 37.1 with the
+// 1024 taken; plan_split has the limits); above, and with one length for all, as batch_piece.
+// Every lane of every wave of a workgroup calls it.
+template <int LAYOUT>
+__device__ __forceinline__ bool row_piece(const SplitArgs& a, uint32_t u, int lane, RowPiece& out) {
+  const auto finer = [&](int rows) {
+    int s = a.pv_shift;
+    while (s > a.pv_fine && (rows >> s) < (s >= a.pv_big ? a.pv_many : a.pv_few)) --s;
+    return s;
+  };
+  if (a.len_mode == kLenUniform || a.batch > kOrderBatches)
+    return batch_piece<LAYOUT>(a, u, a.pv_shift, ((uint32_t)a.max_rows + (1u << a.pv_shift) - 1) >> a.pv_shift, out);
+  if (a.batch == 1) {
+    out.b = 0;
+    out.piece = u;
+    out.S = split_len_l<LAYOUT>(a, 0);
+    const bool valid = out.S > 0 && out.S <= a.max_rows;
+    out.shift = finer(valid ? out.S : 0);
+    return u == 0 || (valid && (int)(u << out.shift) < out.S);
+  }
+  int len[kOrderRegs];
+  batch_lengths<LAYOUT>(a, lane, len);
+  // All valid rows (a row's part capped: the sum stays below 2^31).
+  int rows = 0;
+#pragma unroll
+  for (int p = 0; p < kOrderRegs; ++p) rows += len[p] <= 0 || len[p] > a.max_rows ? 0 : min(len[p], 1 << 22);
+  out.shift = finer(__builtin_amdgcn_readlane(wave_scan(rows), kWaveSize - 1));
+  const int round = (1 << out.shift) - 1;
+  uint32_t before = 0;  // pieces of the batches of earlier p
+#pragma unroll
+  for (int p = 0; p < kOrderRegs; ++p) {
+    if (p * kWaveSize >= a.batch) break;
+    const int x = wave_scan(p * kWaveSize + lane >= a.batch      ? 0
+                            : len[p] <= 0 || len[p] > a.max_rows ? 1
+                                                                 : (len[p] + round) >> out.shift);
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane(x, kWaveSize - 1);
+    if (u < before + total) {
+      const int l = __popcll(__builtin_amdgcn_ballot_w64(before + (uint32_t)x <= u));
+      out.b = (uint32_t)(p * kWaveSize + l);
+      out.piece = u - before - (l > 0 ? (uint32_t)__builtin_amdgcn_readlane(x, l - 1) : 0u);
+      out.S = __builtin_amdgcn_readlane(len[p], l);
+      return true;
+    }
+    before += total;
+  }
+  return false;
+}
+
+// Joins (max, sum of exp(t - max)) of two parts of a row.  A part without
+// rows is (-inf, 0); a NaN sum (an unmapped page, a NaN score) stays NaN.
+__device__ __forceinline__ void join_stats(float& m, float& l, float m2, float l2) {
+  const float mx = fmaxf(m, m2);
+  const float e1 = m == mx ? 1.0f : expf(m - mx);
+  const float e2 = m2 == mx ? 1.0f : expf(m2 - mx);
+  l = l * e1 + l2 * e2;
+  m = mx;
 }
 
 __device__ __forceinline__ u32x4 buffer_load16_nt(__amdgpu_buffer_rsrc_t r, uint32_t voffset) {
@@ -492,9 +609,30 @@ __device__ __forceinline__ uint64_t t_block_base(const SplitArgs& a, uint64_t b,
 // One 16-row block per lane group, all of its K rows requested at once: a
 // wave serves 2^sub_shift consecutive blocks (SubUnits).  The G query heads
 // of a KV head are scored GH at a time against the same K registers (GH = 4
-// bounds the partial sums a lane holds to 64).
+// bounds the partial sums a lane holds to 64).  A workgroup's waves take the
+// next blocks of the same heads and join their statistics through LDS.
+// One wave, but kScoresMaxWaves on rows of more than kScoresLongBlocks
+// blocks: more, held until the slowest is done, measured slower (µs of this
+// launch at 1 / 2 / 4 / 8 waves, 32/8 D=128: B=1 S=131072 47.9 / 50.8 / 50.4
+// / 52.1, S=3001 4.9 / 5.6 / 6.4 / 8.0, B=8 S=32768 92.4 / 97.3), and fewer
+// leave the P.V launch more entries to join than its lanes take at once (S =
+// 131072 53.9 with four waves here, 56.8 with two).  Grid: pieces
+// (batch_piece) of 2^sup_shift rows times units_per_batch head groups.
+constexpr int kScoresMaxWaves = 4;
+constexpr int kScoresLongBlocks = 2048;
+
+// Zeroes the P.V arrival counts of `heads` KV heads from hk0 on of batch b,
+// `tiles` query tiles each (the workgroups of the P.V launch count from it).
+__device__ __forceinline__ void clear_done(const SplitArgs& a, uint32_t b, uint32_t hk0, int heads, int tiles) {
+  if (a.npv == 1) return;
+  const uint32_t per = (uint32_t)(tiles * (1 + (a.npv + kPvFan - 1) / kPvFan));
+  const uint32_t n = min((uint32_t)heads, (uint32_t)a.num_heads_kv - min(hk0, (uint32_t)a.num_heads_kv)) * per;
+  uint32_t* done = a.done + ((uint64_t)b * a.num_heads_kv + hk0) * per;
+  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) done[i] = 0u;
+}
+
 template <int D, int G, int LAYOUT = kLayoutPacked>
-__global__ __launch_bounds__(kBlockThreads) void splitkv_scores_kernel(SplitArgs a) {
+__global__ __launch_bounds__(kBlockThreads * kScoresMaxWaves) void splitkv_scores_kernel(SplitArgs a) {
   constexpr int LPH = D / 8;
   constexpr int HPW = kWaveSize / LPH;
   constexpr int NS = ilog2(LPH);
@@ -505,31 +643,34 @@ __global__ __launch_bounds__(kBlockThreads) void splitkv_scores_kernel(SplitArgs
   constexpr int W = (V >> NS) > 1 ? (V >> NS) : 1;
   constexpr int GS = W < NR ? W : NR;
   constexpr int C = ilog2(NR / GS);
+  __shared__ f32x2_v st_lds[kScoresMaxWaves][HPW][G];
   const int lane = threadIdx.x & (kWaveSize - 1);
-  // Wave order (batch, block group, head group): consecutive waves read
-  // neighbouring heads of the same rows.
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWaveSize));
+  // Workgroup order (piece, head group): consecutive ones read neighbouring
+  // heads of the same rows.
   const SubUnits<HPW> su(a.sub_shift);
-  const uint32_t id = blockIdx.x;
   const uint32_t upb = (uint32_t)a.units_per_batch;
-  const uint32_t nwb = ((uint32_t)a.nblk + (1u << a.sub_shift) - 1) >> a.sub_shift;
-  const uint32_t per_b = nwb * upb;
-  const uint32_t b = id / per_b;
-  if (b >= (uint32_t)a.batch) return;
-  const uint32_t rem = id - b * per_b;
-  const uint32_t wb = rem / upb;
-  const uint32_t hg = rem - wb * upb;
-  const int S = split_len_l<LAYOUT>(a, b);
+  const uint32_t u = blockIdx.x / upb;
+  const uint32_t hg = blockIdx.x - u * upb;
+  RowPiece rp;
+  if (!batch_piece<LAYOUT>(a, u, a.sup_shift, (uint32_t)a.nsup, rp)) return;
+  const uint32_t b = rp.b;
+  const int S = rp.S;
+  if (rp.piece == 0) clear_done(a, b, hg * su.heads(), su.heads(), 1);
+  if (S <= 0 || S > a.max_rows) return;
+  const uint32_t wb = (rp.piece << (a.sup_shift - a.sub_shift - ilog2(NR))) + (uint32_t)wv;
   const int j0 = (int)(wb << a.sub_shift) * NR;  // the wave's first row
-  if (S < 0 || S > a.max_rows || j0 >= S) return;
   const int hkl = lane / LPH;
   const int p = su.unit(hkl);           // this lane group's block of the wave
   const int hk = su.head(hg, hkl);
   const bool head_ok = hk < a.num_heads_kv;
   const int r = lane % LPH;
   const int hq = a.num_heads_q;
-  const int blk = (int)(wb << a.sub_shift) + p;
   const int jb = j0 + p * NR;           // first row of this lane group's block
   const bool block_ok = jb < S;         // else past the row (and maybe past nblk): no writes
+  for (int i = lane; i < HPW * G; i += kWaveSize) st_lds[wv][i / G][i % G] = f32x2_v{-__builtin_inff(), 0.0f};
+  __builtin_amdgcn_wave_barrier();
+  if (j0 < S) {  // wave-uniform
   const __amdgpu_buffer_rsrc_t q_rsrc = make_rsrc(a.q + (uint64_t)b * hq * D, (uint32_t)hq * D * 2);
   // Rows [0, S) of the batch: rows past S read 0 without access.
   SplitRows<D, LAYOUT> kv;
@@ -604,509 +745,29 @@ __global__ __launch_bounds__(kBlockThreads) void splitkv_scores_kernel(SplitArgs
         for (int w = 0; w < GS; ++w) bs += jb + jr0 + w < S ? expf(t[w] - bm) : 0.0f;
         bs = GroupReduce<LPH, L - C, L, false>::run(bs);
         if (writer && (blkl & ((1 << C) - 1)) == 0) {
-          const uint64_t idx = ((uint64_t)b * hq + (uint64_t)hk * G + g) * a.nblk + blk;
-          a.m[idx] = bm;
           // An unmapped page among the block's rows: a NaN sum makes every
           // weight of the batch's heads, hence its outputs, NaN.
-          a.l[idx] = kv_bad ? __builtin_nanf("") : bs;
+          st_lds[wv][hkl][g] = f32x2_v{bm, kv_bad ? __builtin_nanf("") : bs};
         }
       }
     }
   }
-}
-
-// Sum / max over the 64 lanes of a wave (every lane gets the result).
-__device__ __forceinline__ float wave_max(float x) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) x = fmaxf(x, __shfl_xor(x, m, kWaveSize));
-  return x;
-}
-__device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) x += __shfl_xor(x, m, kWaveSize);
-  return x;
-}
-
-// Max or sum over a workgroup of THREADS threads, in a fixed order (wave
-// trees, then waves in index order); every thread gets the result.
-template <int THREADS, bool IS_MAX>
-__device__ __forceinline__ float block_reduce(float x, float* red) {
-  x = IS_MAX ? wave_max(x) : wave_sum(x);
-  if constexpr (THREADS == kWaveSize) {
-    return x;
-  } else {
-    constexpr int NW = THREADS / kWaveSize;
-    if ((threadIdx.x & (kWaveSize - 1)) == 0) red[threadIdx.x / kWaveSize] = x;
-    __syncthreads();
-    float y = red[0];
-#pragma unroll
-    for (int w = 1; w < NW; ++w) y = IS_MAX ? fmaxf(y, red[w]) : y + red[w];
-    __syncthreads();  // red is reused by the next call
-    return y;
   }
-}
-
-// ---------------------------------------------------------------------------
-// 2. stats (rows of more than kPvStatBlocks blocks): per (batch, query
-// head), the global max and sum of exponentials over the row's 16-row
-// blocks.
-// ---------------------------------------------------------------------------
-// Rows of at most 16 blocks: one lane per head, all loads in flight.
-#ifdef FMHA_DECODE_SHARED_KERNELS  // one translation unit emits it (not a template)
-__global__ __launch_bounds__(256) void splitkv_stats_lane_kernel(SplitArgs a) {
-  constexpr int NB = 16;
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;  // b * Hq + h
-  if (i >= (uint64_t)a.batch * a.num_heads_q) return;
-  const uint64_t b = i / (uint64_t)a.num_heads_q;
-  const int S = split_len(a, b);
-  if (S <= 0 || S > a.max_rows) return;
-  const int n = (S + kSplitBlockRows - 1) / kSplitBlockRows;
-  const float* m = a.m + i * a.nblk;
-  const float* l = a.l + i * a.nblk;
-  float xm[NB], xl[NB];
-#pragma unroll
-  for (int c = 0; c < NB; ++c) {
-    xm[c] = c < n ? m[c] : -__builtin_inff();
-    xl[c] = c < n ? l[c] : 0.0f;
-  }
-  float gm = xm[0];
-#pragma unroll
-  for (int c = 1; c < NB; ++c) gm = fmaxf(gm, xm[c]);
-  float gl = 0.0f;
-#pragma unroll
-  for (int c = 0; c < NB; ++c) gl += c < n ? xl[c] * expf(xm[c] - gm) : 0.0f;
-  a.ml[2 * i] = gm;
-  a.ml[2 * i + 1] = gl;
-}
-#endif  // FMHA_DECODE_SHARED_KERNELS
-
-// Longer rows: one THREADS-thread group per head, U loads in flight per
-// thread, reduction order fixed.
-template <int THREADS>
-__global__ __launch_bounds__(THREADS) void splitkv_stats_kernel(SplitArgs a) {
-  constexpr int U = 8;
-  __shared__ float red[THREADS / kWaveSize];
-  const uint64_t i = blockIdx.x;  // b * Hq + h
-  const int t = threadIdx.x;
-  const uint64_t b = i / (uint64_t)a.num_heads_q;
-  const int S = split_len(a, b);
-  if (S <= 0 || S > a.max_rows) return;  // the same for every thread of the group
-  const int n = (S + kSplitBlockRows - 1) / kSplitBlockRows;
-  const float* m = a.m + i * a.nblk;
-  const float* l = a.l + i * a.nblk;
-  float vm = -__builtin_inff();
-  for (int c0 = t; c0 < n; c0 += THREADS * U) {
-    float xm[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int c = c0 + u * THREADS;
-      xm[u] = c < n ? m[c] : -__builtin_inff();
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) vm = fmaxf(vm, xm[u]);
-  }
-  const float gm = block_reduce<THREADS, true>(vm, red);
-  float vs = 0.0f;
-  for (int c0 = t; c0 < n; c0 += THREADS * U) {
-    float xm[U], xl[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int c = c0 + u * THREADS;
-      xm[u] = c < n ? m[c] : 0.0f;
-      xl[u] = c < n ? l[c] : 0.0f;
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) vs += c0 + u * THREADS < n ? xl[u] * expf(xm[u] - gm) : 0.0f;
-  }
-  const float gl = block_reduce<THREADS, false>(vs, red);
-  if (t == 0) {
-    a.ml[2 * i] = gm;
-    a.ml[2 * i + 1] = gl;
-  }
-}
-
-// The global max and sum of exp(t - max) of NS query heads (hqi[i]; ok[i]
-// false: none, 0 and 1 returned) of a row of S rows, for the P.V passes:
-// a.ml when the statistics pass ran, else the scores pass's block
-// statistics reduced here.  The NL lanes whose lane index differs only in the bits of
-// STRIDE * (NL - 1) share each head; lane k of them (k = (lane / STRIDE) %
-// NL) takes blocks k, k + NL, ... (the max, then the sum of l * exp(m -
-// max)), U of them in flight per head, then butterflies over the NL lanes in
-// a fixed order.
-template <int NL, int STRIDE, int NS>
-__device__ __forceinline__ void row_stats(const SplitArgs& a, const uint64_t (&hqi)[NS], const bool (&ok)[NS], int S,
-                                          int lane, float (&gm)[NS], float (&gl)[NS]) {
-  if (a.stat_pass) {
-#pragma unroll
-    for (int i = 0; i < NS; ++i) {
-      gm[i] = ok[i] ? a.ml[2 * hqi[i]] : 0.0f;
-      gl[i] = ok[i] ? a.ml[2 * hqi[i] + 1] : 1.0f;
-    }
-    return;
-  }
-  constexpr int U = 4;
-  const int k = (lane / STRIDE) % NL;
-  const int n = (S + kSplitBlockRows - 1) / kSplitBlockRows;
-  float mx[NS];
-#pragma unroll
-  for (int i = 0; i < NS; ++i) mx[i] = -__builtin_inff();
-  for (int s0 = k; s0 < n; s0 += NL * U) {
-    float x[NS][U];
-#pragma unroll
-    for (int i = 0; i < NS; ++i)
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int s = s0 + u * NL;
-        x[i][u] = ok[i] && s < n ? a.m[hqi[i] * a.nblk + s] : -__builtin_inff();
-      }
-#pragma unroll
-    for (int i = 0; i < NS; ++i)
-#pragma unroll
-      for (int u = 0; u < U; ++u) mx[i] = fmaxf(mx[i], x[i][u]);
-  }
-#pragma unroll
-  for (int i = 0; i < NS; ++i)
-#pragma unroll
-    for (int d = STRIDE; d < STRIDE * NL; d <<= 1) mx[i] = fmaxf(mx[i], __shfl_xor(mx[i], d, kWaveSize));
-  float sm[NS];
-#pragma unroll
-  for (int i = 0; i < NS; ++i) sm[i] = 0.0f;
-  for (int s0 = k; s0 < n; s0 += NL * U) {
-    float x[NS][U], y[NS][U];
-#pragma unroll
-    for (int i = 0; i < NS; ++i)
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int s = s0 + u * NL;
-        const bool in = ok[i] && s < n;
-        x[i][u] = in ? a.m[hqi[i] * a.nblk + s] : 0.0f;
-        y[i][u] = in ? a.l[hqi[i] * a.nblk + s] : 0.0f;
-      }
-#pragma unroll
-    for (int i = 0; i < NS; ++i)
-#pragma unroll
-      for (int u = 0; u < U; ++u) sm[i] += ok[i] && s0 + u * NL < n ? y[i][u] * expf(x[i][u] - mx[i]) : 0.0f;
-  }
-#pragma unroll
-  for (int i = 0; i < NS; ++i) {
-#pragma unroll
-    for (int d = STRIDE; d < STRIDE * NL; d <<= 1) sm[i] += __shfl_xor(sm[i], d, kWaveSize);
-    gm[i] = ok[i] ? mx[i] : 0.0f;
-    gl[i] = ok[i] ? sm[i] : 1.0f;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// 3. P.V per chunk.  DIRECT: every batch fits one chunk, so the wave writes
-// fp16 O itself (and the zero / NaN rows of empty or invalid batches).
-// ---------------------------------------------------------------------------
-template <int D, int G, int NR>
-struct PvSlots {
-  static constexpr int LPH = D / 8;
-  static constexpr int HPW = kWaveSize / LPH;
-  static constexpr int SLOTS = HPW * G * NR;  // weights per sub-block
-  static constexpr int PER_LANE = (SLOTS + kWaveSize - 1) / kWaveSize;
-};
-
-// One sub-block: weights -> LDS -> row pairs -> accumulate.  Slot
-// f = lane + 64*i is (KV head f / (G*NR), query g = (f / NR) % G, row f % NR)
-// of the wave's heads; valid[i] marks slots inside the chunk.
-template <int D, int G, int NR>
-__device__ __forceinline__ void pv_sub_block(const u32x4 (&vr)[NR], const float (&tv)[PvSlots<D, G, NR>::PER_LANE],
-                                             const float (&gm)[PvSlots<D, G, NR>::PER_LANE],
-                                             const float (&gsum)[PvSlots<D, G, NR>::PER_LANE],
-                                             const int (&rows_left)[PvSlots<D, G, NR>::PER_LANE],
-                                             bool (&slot_ok)[PvSlots<D, G, NR>::PER_LANE], uint16_t* lds_p, int hkl,
-                                             int lane, float (&acc)[G][8]) {
-  using P = PvSlots<D, G, NR>;
-  constexpr int VP = G * kMaxSeq;
-#pragma unroll
-  for (int i = 0; i < P::PER_LANE; ++i) {
-    const int f = lane + kWaveSize * i;
-    const int jf = f % NR;
-    const bool valid = slot_ok[i] && jf < rows_left[i];
-    const float p = valid ? expf(tv[i] - gm[i]) / gsum[i] : 0.0f;
-    if (f < P::SLOTS)
-      lds_p[(f / (G * NR)) * VP + ((f / NR) % G) * kMaxSeq + jf] = __builtin_bit_cast(uint16_t, (__bf16)p);
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  const uint32_t* pairs = reinterpret_cast<const uint32_t*>(lds_p + hkl * VP);
-  uint32_t pp[G][(NR + 1) / 2];
-#pragma unroll
-  for (int g = 0; g < G; ++g)
-#pragma unroll
-    for (int jp = 0; jp < NR / 2; ++jp) pp[g][jp] = pairs[g * (kMaxSeq / 2) + jp];
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  accumulate_pv<G, NR>(vr, pp, acc);
-}
-
-template <int D, int G, int NR, bool DIRECT, int LAYOUT = kLayoutPacked>
-__global__ __launch_bounds__(kBlockThreads) void splitkv_pv_kernel(SplitArgs a) {
-  using P = PvSlots<D, G, NR>;
-  constexpr int LPH = P::LPH;
-  constexpr int HPW = P::HPW;
-  constexpr int PL = P::PER_LANE;
-  constexpr int VP = G * kMaxSeq;
-  static_assert(NR % 2 == 0 && NR <= kMaxSeq, "sub-block rows");
-  __shared__ __attribute__((aligned(16))) uint16_t lds_p[HPW * VP];
-  const int lane = threadIdx.x & (kWaveSize - 1);
-  // A wave serves 2^sub_shift consecutive chunks (one per lane group,
-  // SubUnits); DIRECT launches have one chunk per batch and sub_shift = 0.
-  const SubUnits<HPW> su(a.sub_shift);
-  const uint32_t id = blockIdx.x;
-  const uint32_t upb = (uint32_t)a.units_per_batch;
-  const uint32_t nwc = ((uint32_t)a.nchunks + (1u << a.sub_shift) - 1) >> a.sub_shift;
-  const uint32_t per_b = nwc * upb;
-  const uint32_t b = id / per_b;
-  if (b >= (uint32_t)a.batch) return;
-  const uint32_t rem = id - b * per_b;
-  const uint32_t wc = rem / upb;
-  const uint32_t hg = rem - wc * upb;
-  const int S = split_len_l<LAYOUT>(a, b);
-  const bool bad = S < 0 || S > a.max_rows;
-  const int roww = (int)(wc << a.sub_shift) * a.chunk_rows;  // the wave's first row
-  const int hkl = lane / LPH;
-  const int p = su.unit(hkl);
-  const uint32_t c = (wc << a.sub_shift) + (uint32_t)p;     // this lane group's chunk
-  const int row0 = (int)c * a.chunk_rows;
-  const int hk = su.head(hg, hkl);
-  const bool head_ok = hk < a.num_heads_kv;
-  const int r = lane % LPH;
-  const int hq = a.num_heads_q;
-  if (bad || roww >= S) {
-    // Only chunk 0 of a DIRECT launch owns the output of an empty or invalid
-    // batch; the combine kernel covers them otherwise.
-    if constexpr (DIRECT) {
-      if (c != 0) return;
-      const u32x4 fill = bad ? u32x4{0x7e007e00u, 0x7e007e00u, 0x7e007e00u, 0x7e007e00u} : u32x4{0u, 0u, 0u, 0u};
-      const __amdgpu_buffer_rsrc_t o_rsrc = make_rsrc(a.o + (uint64_t)b * hq * D, (uint32_t)hq * D * 2);
-      const uint32_t o_off = head_ok ? (uint32_t)(hk * G * D + r * 8) * 2u : kLaneOutOfRange;
-#pragma unroll
-      for (int g = 0; g < G; ++g) buffer_store16(o_rsrc, o_off + g * D * 2, fill);
-    }
-    return;
-  }
-  // Rows of this lane group's chunk (<= 0: a chunk past the row's end).
-  const int rows = min(S - row0, a.chunk_rows);
-  const int rows_w = min(S - roww, a.chunk_rows);  // the wave's first chunk: the most rows
-  // Each lane group reads its own chunk's rows only: sub-blocks past its
-  // end read 0 without access.
-  SplitRows<D, LAYOUT> vrows;
-  const int rowe = S - roww < (a.chunk_rows << a.sub_shift) ? S : roww + (a.chunk_rows << a.sub_shift);
-  vrows.init(a, a.v, b, split_row_base<LAYOUT>(a, b), roww, rowe, hk, head_ok, r, row0 - roww,
-             row0 - roww + (rows > 0 ? rows : 0));
-  // This batch's scores, [nblk, Hq, 16].
-  const __amdgpu_buffer_rsrc_t t_rsrc =
-      make_rsrc(a.t + t_block_base(a, b, 0), (uint32_t)a.nblk * (uint32_t)hq * kSplitBlockRows * 4u);
-
-  // Weight slot f = lane + 64*i is (wave lane group f / (G*NR), query g =
-  // (f / NR) % G, row f % NR); the lane group gives its head and chunk.
-  float gm[PL], gsum[PL];
-  uint32_t t_off[PL];
-  bool slot_ok[PL];
-  int slot_rows[PL];
-  uint64_t hqi[PL];
-#pragma unroll
-  for (int i = 0; i < PL; ++i) {
-    const int f = lane + kWaveSize * i;
-    const int hklf = f / (G * NR);
-    const int hkf = su.head(hg, hklf);
-    const int gf = (f / NR) % G;
-    const int jf = f % NR;
-    const int row0f = (int)((wc << a.sub_shift) + (uint32_t)su.unit(hklf)) * a.chunk_rows;
-    slot_rows[i] = min(S - row0f, a.chunk_rows);
-    slot_ok[i] = f < P::SLOTS && hkf < a.num_heads_kv && slot_rows[i] > 0;
-    hqi[i] = (uint64_t)b * hq + hkf * G + gf;
-    t_off[i] = slot_ok[i] ? (uint32_t)((row0f / kSplitBlockRows) * hq * kSplitBlockRows +
-                                       (hkf * G + gf) * kSplitBlockRows + jf) * 4u
-                          : kLaneOutOfRange;
-  }
-  // The NR lanes of a slot's (head, query) share its statistics.
-  row_stats<NR, 1, PL>(a, hqi, slot_ok, S, lane, gm, gsum);
-
-  float acc[G][8];
-#pragma unroll
-  for (int g = 0; g < G; ++g)
-#pragma unroll
-    for (int d = 0; d < 8; ++d) acc[g][d] = 0.0f;
-
-  // Two register sets: sub-block s+1 is requested before s is processed.
-  // Requests past a chunk's last row return 0 without memory access (V)
-  // or read scores of other rows (or nothing, past the batch's blocks) that
-  // the row check masks (T).  The wave runs as many sub-blocks as its first
-  // chunk has.
-  const int nsub = (rows_w + NR - 1) / NR;
-  u32x4 va[NR], vb[NR];
-  float ta[PL], tb[PL];
-  // Per-lane page lookups on pages under 16 rows (an entry per row): each
-  // sub-block's block-table entries are requested a step ahead of its rows
-  // (PF).  16-row pages look up one entry per sub-block and keep the
-  // registers (two more would cost the 16-row P.V its second wave per SIMD).
-  constexpr bool PF = LAYOUT == kLayoutPagedLanes;
-  constexpr int NE = PF ? NR : 1;
-  int32_t ea[NE], eb[NE];
-  auto load = [&](u32x4 (&vr)[NR], float (&tv)[PL], int s, const int32_t (&e)[NE]) {
-    if constexpr (PF)
-      vrows.template load_entries<NR>(vr, s * NR, e);
-    else
-      vrows.template load<NR>(vr, s * NR);
-    // Sub-blocks never straddle a 16-row block (chunks start on multiples of 16).
-    const uint32_t sub = (uint32_t)(((s * NR) / kSplitBlockRows) * hq * kSplitBlockRows +
-                                    (s * NR) % kSplitBlockRows) * 4u;
-#pragma unroll
-    for (int i = 0; i < PL; ++i) tv[i] = buffer_load_f32(t_rsrc, t_off[i] + sub);
-  };
-  auto entries = [&](int32_t (&e)[NE], int s) {
-    if constexpr (PF) vrows.template entries<NR>(e, s * NR);
-  };
-  auto left = [&](int (&rl)[PL], int s) {
-#pragma unroll
-    for (int i = 0; i < PL; ++i) rl[i] = slot_rows[i] - s * NR;
-  };
-  entries(ea, 0);
-  load(va, ta, 0, ea);
-  entries(eb, 1);
-  for (int s = 0; s < nsub; s += 2) {
-    int rl[PL];
-    load(vb, tb, s + 1, eb);
-    entries(ea, s + 2);
-    left(rl, s);
-    pv_sub_block<D, G, NR>(va, ta, gm, gsum, rl, slot_ok, lds_p, hkl, lane, acc);
-    load(va, ta, s + 2, ea);
-    entries(eb, s + 3);
-    left(rl, s + 1);
-    if (s + 1 < nsub) pv_sub_block<D, G, NR>(vb, tb, gm, gsum, rl, slot_ok, lds_p, hkl, lane, acc);
-  }
-
-  if constexpr (DIRECT) {
-    const __amdgpu_buffer_rsrc_t o_rsrc = make_rsrc(a.o + (uint64_t)b * hq * D, (uint32_t)hq * D * 2);
-    const uint32_t o_off = head_ok ? (uint32_t)(hk * G * D + r * 8) * 2u : kLaneOutOfRange;
-#pragma unroll
-    for (int g = 0; g < G; ++g) buffer_store16(o_rsrc, o_off + g * D * 2, pack_f16x8(acc[g]));
-  } else {
-    // Partial outputs [Hq][nchunks][D] of this batch, read by the combine
-    // pass right after: default-policy stores keep them in the caches
-    // (non-temporal ones measured 4-9% slower overall).
-    const uint32_t part_bytes = (uint32_t)a.nchunks * D * 4u;
-    const __amdgpu_buffer_rsrc_t p_rsrc =
-        make_rsrc(a.opart + (uint64_t)b * hq * a.nchunks * D, (uint32_t)hq * part_bytes);
-    // A lane group whose chunk starts past the row's end writes nothing.
-    const uint32_t p_off = head_ok && rows > 0 ? (uint32_t)hk * G * part_bytes + (c * D + r * 8) * 4u : kLaneOutOfRange;
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      u32x4 lo, hi;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        lo[i] = __builtin_bit_cast(uint32_t, acc[g][i]);
-        hi[i] = __builtin_bit_cast(uint32_t, acc[g][4 + i]);
-      }
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_gcc, lo), p_rsrc, (int)(p_off + g * part_bytes),
-                                             0, kPolicyDefault);
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_gcc, hi), p_rsrc,
-                                             (int)(p_off + g * part_bytes + 16), 0, kPolicyDefault);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// 4. combine: O = fp16(sum over the batch's chunks of Opart), chunk order.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ void add8(float (&acc)[8], const u32x4& lo, const u32x4& hi) {
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    acc[k] += __builtin_bit_cast(float, (uint32_t)lo[k]);
-    acc[4 + k] += __builtin_bit_cast(float, (uint32_t)hi[k]);
-  }
-}
-
-// Few chunks: one lane per (batch, query head, 8 dims), U chunks in flight.
-template <int D>
-__global__ __launch_bounds__(256) void splitkv_combine_kernel(SplitArgs a) {
-  constexpr int U = 4;
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t per_head = D / 8;
-  if (i >= (uint64_t)a.batch * a.num_heads_q * per_head) return;
-  const uint64_t head = i / per_head;  // b * Hq + h
-  const int d0 = (int)(i - head * per_head) * 8;
-  const uint64_t b = head / (uint64_t)a.num_heads_q;
-  const int S = split_len(a, b);
-  float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  u32x4 out;
-  if (S < 0 || S > a.max_rows) {
-    out = u32x4{0x7e007e00u, 0x7e007e00u, 0x7e007e00u, 0x7e007e00u};
-  } else {
-    const int n = (S + a.chunk_rows - 1) / a.chunk_rows;
-    const float* src = a.opart + head * a.nchunks * D + d0;
-    for (int c0 = 0; c0 < n; c0 += U) {
-      u32x4 lo[U], hi[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int c = c0 + u < n ? c0 + u : c0;
-        lo[u] = *reinterpret_cast<const u32x4*>(src + (uint64_t)c * D);
-        hi[u] = *reinterpret_cast<const u32x4*>(src + (uint64_t)c * D + 4);
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (c0 + u < n) add8(acc, lo[u], hi[u]);
-    }
-    out = pack_f16x8(acc);
-  }
-  *reinterpret_cast<u32x4*>(a.o + head * D + d0) = out;
-}
-
-// Many chunks: one THREADS-thread block per (batch, query head, slice of
-// 32 dims), so that a head's partials are read by D/32 CUs and every chunk's
-// slice is one 128-byte line.  Thread t sums dims [4*(t % 8), +4) of the
-// slice over chunks c = t / 8 + k * CG (U = 8 chunks in flight); then the CG
-// partial sums of each dim are added in order through LDS.
-template <int D, int THREADS>
-__global__ __launch_bounds__(THREADS) void splitkv_combine_block_kernel(SplitArgs a) {
-  constexpr int SLICE = 32;
-  constexpr int NSL = D / SLICE;
-  constexpr int LPS = SLICE / 4;  // lanes per slice
-  constexpr int CG = THREADS / LPS;
-  constexpr int U = 8;
-  __shared__ float part[CG][SLICE];
-  const uint64_t head = blockIdx.x / NSL;  // b * Hq + h
-  const int d0 = (int)(blockIdx.x - head * NSL) * SLICE;
-  const int t = threadIdx.x;
-  const int dl = t % LPS;
-  const int cg = t / LPS;
-  const uint64_t b = head / (uint64_t)a.num_heads_q;
-  const int S = split_len(a, b);
-  const bool bad = S < 0 || S > a.max_rows;
-  const int n = bad ? 0 : (S + a.chunk_rows - 1) / a.chunk_rows;
-  float acc[4] = {0, 0, 0, 0};
-  const float* src = a.opart + head * a.nchunks * D + d0 + dl * 4;
-  for (int c0 = cg; c0 < n; c0 += CG * U) {
-    u32x4 x[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int c = c0 + u * CG < n ? c0 + u * CG : c0;
-      x[u] = *reinterpret_cast<const u32x4*>(src + (uint64_t)c * D);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (c0 + u * CG < n)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) acc[k] += __builtin_bit_cast(float, (uint32_t)x[u][k]);
-  }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) part[cg][dl * 4 + k] = acc[k];
   __syncthreads();
-  if (t >= SLICE / 8) return;
-  // Threads 0..3 each finish 8 dims of the slice: sum over the chunk groups
-  // in order, then one 16-byte fp16 store.
-  float o[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int g = 0; g < CG; ++g)
-#pragma unroll
-    for (int k = 0; k < 8; ++k) o[k] += part[g][t * 8 + k];
-  const u32x4 out = bad ? u32x4{0x7e007e00u, 0x7e007e00u, 0x7e007e00u, 0x7e007e00u} : pack_f16x8(o);
-  *reinterpret_cast<u32x4*>(a.o + head * D + d0 + t * 8) = out;
+  // The workgroup's statistics of each query head, waves and lane groups in
+  // row order.
+  for (int i = (int)threadIdx.x; i < su.heads() * G; i += (int)blockDim.x) {
+    const int h = i / G, g = i % G;
+    const int hko = su.head(hg, h);
+    if (hko >= a.num_heads_kv) continue;
+    float m = -__builtin_inff(), l = 0.0f;
+    for (int w = 0; w < (int)blockDim.x / kWaveSize; ++w)
+      for (int q = 0; q < (1 << a.sub_shift); ++q) {
+        const f32x2_v x = st_lds[w][(q << su.shift) + h][g];
+        join_stats(m, l, x[0], x[1]);
+      }
+    a.st[((uint64_t)b * hq + (uint64_t)hko * G + g) * a.nsup + rp.piece] = f32x2_v{m, l};
+  }
 }
 
 }  // namespace fmha_decode

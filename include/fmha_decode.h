@@ -274,7 +274,8 @@ int fmha_decode_fwd_paged(void* stream,
  * The library picks the kernels: the kernel and numerics of fmha_decode_fwd
  * when max_seqlen_kv <= 16; one single-pass launch when there are at least 512
  * (batch, KV-head group) waves and a row's scores fit the wave's LDS; else
- * four split-KV launches (scores, statistics, P.V per chunk, combine).
+ * two split-KV launches (scores; statistics, P.V and the sum of a row's
+ * partial outputs).
  *
  * The caller provides a device workspace of at least
  * fmha_decode_splitkv_workspace_size(batch, Hq, Hkv, max_seqlen_kv, head_dim)
@@ -390,8 +391,11 @@ const char* fmha_decode_last_error_detail(void);
  * separated by "; " ("" after a rejected or empty call): each a kernel
  * kind with the choices the library made for it, e.g.
  *   "short(numerics=exact D=128 G=1 layout=packed bucket=16 waves_per_cu=4)"
- *   "split(D=128 G=4 layout=packed sub_units=1 blocks=64 chunk_rows=256
- *    chunks=4 passes=4)".
+ *   "split(D=128 G=4 layout=packed sub_units=1 blocks=65 chunk_rows=64
+ *    chunks=17 passes=4 launches=2)",
+ * whose chunks are the rows of one wave of the P.V launch (the whole row with
+ * one workgroup per row) and whose passes count what the launches do: scores,
+ * statistics beyond 64 blocks, P.V, the sum over a row's workgroups.
  * Kinds: short, short_multi (several batches per wave), short_matrix_core,
  * onepass, split, split_matrix_core, pad_query_group.  For tests and
  * diagnostics; no counterpart in the reference. */

@@ -59,11 +59,12 @@ def layout_shapes():
 
 def workspace_traffic(plan, B, hq, hkv, D):
     """Bytes the split-KV passes move through the workspace per call, from the
-    plan the library reports: the scores T (written by the scores pass, read
-    by P.V), the per-block max and sum (written, read by the statistics
-    pass), the per-head max and sum (written, read by P.V) and, with more
-    than one chunk per row, the fp32 partial outputs (written by P.V, read by
-    the combine).  0 for the single pass and the short kernels."""
+    plan the library reports: the scores T (written by the scores launch, read
+    by P.V), the max and sum of every 16 rows or more (written; the P.V
+    workgroups' reads of them hit the caches) and, with more than one P.V
+    workgroup of four chunks per row, the fp32 partial outputs (written, and
+    read by the row's last workgroup).  0 for the single pass and the short
+    kernels."""
     total = 0
     for entry in plan:
         kind, _, rest = entry.partition("(")
@@ -71,10 +72,10 @@ def workspace_traffic(plan, B, hq, hkv, D):
             continue
         f = dict(kv.split("=") for kv in rest.rstrip(")").split())
         heads = B * max(hq, hkv * int(f["G"]))
-        nblk, chunks = int(f["blocks"]), int(f["chunks"])
-        total += 2 * heads * nblk * 16 * 4 + 2 * 2 * heads * nblk * 4 + 2 * heads * 2 * 4
-        if chunks > 1:
-            total += 2 * heads * chunks * D * 4
+        nblk, groups = int(f["blocks"]), (int(f["chunks"]) + 3) // 4
+        total += 2 * heads * nblk * 16 * 4 + heads * nblk * 8
+        if groups > 1:
+            total += 2 * heads * groups * D * 4
     return total
 
 

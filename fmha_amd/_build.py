@@ -4,7 +4,9 @@ Compiles fmha_amd/csrc/fmha_decode_api.hip (the C ABI) and every part of
 fmha_amd/csrc/fmha_decode_inst.hip (the kernel instantiations, one slice per
 -DFMHA_DECODE_PART) with hipcc, in parallel, and links them into
 fmha_amd/libfmha_decode.so, in tree, so the built library travels with the
-source tree.  The objects go to fmha_amd/_build/.
+source tree.  The objects go to fmha_amd/_build/.  build_host() compiles the
+tensor interface's native module (fmha_amd/csrc/fmha_decode_torch.cpp, host
+code only) against the installed torch into fmha_amd/_host.so.
 """
 import concurrent.futures
 import os
@@ -18,6 +20,8 @@ LIB = os.path.join(HERE, "libfmha_decode.so")
 CSRC = os.path.join(HERE, "csrc")
 API_SOURCE = os.path.join(CSRC, "fmha_decode_api.hip")
 INST_SOURCE = os.path.join(CSRC, "fmha_decode_inst.hip")
+HOST_LIB = os.path.join(HERE, "_host.so")
+HOST_SOURCE = os.path.join(CSRC, "fmha_decode_torch.cpp")
 OBJ_DIR = os.path.join(HERE, "_build")
 
 HIPCC_FLAGS = [
@@ -90,5 +94,29 @@ def build(verbose=False, jobs=None):
     return LIB
 
 
+def build_host(verbose=False):
+    """Compile the native module of the tensor interface; raises
+    CalledProcessError on failure."""
+    import sysconfig
+    import torch
+    root = os.path.dirname(torch.__file__)
+    rocm = os.path.dirname(os.path.dirname(hipcc()))
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
+           "-I" + os.path.join(ROOT, "include"), "-isystem", os.path.join(root, "include"),
+           "-isystem", os.path.join(rocm, "include"), "-isystem", sysconfig.get_paths()["include"],
+           HOST_SOURCE, "-o", HOST_LIB + ".tmp", "-L" + os.path.join(root, "lib"),
+           "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    rc, err = _run(cmd)
+    if rc != 0:
+        sys.stderr.write(err + "\n")
+        raise subprocess.CalledProcessError(rc, cmd)
+    os.replace(HOST_LIB + ".tmp", HOST_LIB)
+    return HOST_LIB
+
+
 if __name__ == "__main__":
     print(build(verbose=True))
+    print(build_host(verbose=True))

@@ -12,6 +12,24 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 # library that fmha_amd/_build.py writes.
 LIB_PATH = os.environ.get("FMHA_DECODE_LIB") or os.path.join(_HERE, "libfmha_decode.so")
 
+# The tensor interface's native module (fmha_amd/csrc/fmha_decode_torch.cpp)
+# and the entry points it is bound to, in the order of its Library.
+HOST_PATH = os.path.join(_HERE, "_host.so")
+HOST_ENTRIES = (
+    "fmha_decode_fwd",
+    "fmha_decode_fwd_fast",
+    "fmha_decode_fwd_fp32_weights",
+    "fmha_decode_fwd_exact",
+    "fmha_decode_fwd_uniform",
+    "fmha_decode_fwd_uniform_fast",
+    "fmha_decode_fwd_strided",
+    "fmha_decode_fwd_paged",
+    "fmha_decode_splitkv_workspace_size",
+    "fmha_decode_fwd_splitkv",
+    "fmha_decode_fwd_splitkv_strided",
+    "fmha_decode_fwd_splitkv_paged",
+)
+
 # Every symbol include/fmha_decode.h declares.
 EXPORTED = (
     "fmha_decode_fwd",

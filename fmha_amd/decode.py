@@ -10,9 +10,12 @@ Two levels, both thin wrappers over the C ABI in include/fmha_decode.h:
 * fmha_decode -- tensor level, for torch device tensors: checks shapes,
   dtypes and devices, allocates O if not given, launches on torch's current
   stream.  fmha_decode_strided and fmha_decode_paged do the same for strided
-  (BSHD / BHSD / padded) and paged KV caches.
+  (BSHD / BHSD / padded) and paged KV caches.  Plainly acceptable calls take
+  the native form of these functions (csrc/fmha_decode_torch.cpp), which
+  leaves every other one, with its error message, to the code here.
 """
 import math
+import os
 
 from . import _lib
 
@@ -29,6 +32,24 @@ class FmhaDecodeError(RuntimeError):
         super().__init__(f"fmha_decode error {code} ({message}): {detail}")
         self.code = code
         self.detail = detail
+
+
+_native = None
+
+
+def _load_native():
+    """The native forms of the tensor functions, bound to the loaded library."""
+    global _native
+    import ctypes
+    import torch  # noqa: F401  (its libraries are what the module links to)
+    lib = _lib.load()
+    if not os.path.exists(_lib.HOST_PATH):
+        raise RuntimeError(
+            f"{_lib.HOST_PATH} is not built; run `python -c 'import __graft_entry__ as g; g.build()'`")
+    from . import _host
+    _host.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _lib.HOST_ENTRIES))
+    _native = _host
+    return _host
 
 
 def last_plan():
@@ -181,6 +202,9 @@ def fmha_decode_splitkv(q, k, v, cu_seqlens_kv, max_seqlen_kv, softmax_scale=Non
     k/v packed [rows, Hkv, D] bfloat16, cu_seqlens_kv int32 [B+1], every
     length <= max_seqlen_kv.  workspace: a uint8 device tensor of at least
     splitkv_workspace_size(...) bytes (allocated here when None)."""
+    done = (_native or _load_native()).splitkv(q, k, v, cu_seqlens_kv, max_seqlen_kv, softmax_scale, out, workspace)
+    if done is not None:
+        return done if done.__class__ is not int else _raise_if(done)
     import torch
     B, Hq, D = _q_shape(q)
     out = _check_q_out(q, out)
@@ -265,6 +289,9 @@ def fmha_decode_strided(q, k, v, seqlens_kv=None, softmax_scale=None, out=None, 
     fmha_decode_fwd_splitkv_strided with workspace (a uint8 device tensor of
     splitkv_workspace_size(B, Hq, Hkv, S, D) bytes, allocated here when
     None)."""
+    done = (_native or _load_native()).strided(q, k, v, seqlens_kv, softmax_scale, out, workspace)
+    if done is not None:
+        return done if done.__class__ is not int else _raise_if(done)
     import torch
     B, Hq, D = _q_shape(q)
     out = _check_q_out(q, out)
@@ -304,6 +331,10 @@ def fmha_decode_paged(q, k_cache, v_cache, block_table, seqlens_kv, softmax_scal
     group size above 8 whose rows may reach past a batch's first page).
     Without max_seqlen_kv, a group size above 8 needs pages of at least
     min(16, max_pages * page_size) rows (FmhaDecodeError otherwise)."""
+    done = (_native or _load_native()).paged(q, k_cache, v_cache, block_table, seqlens_kv, softmax_scale, out,
+                                             max_seqlen_kv, workspace)
+    if done is not None:
+        return done if done.__class__ is not int else _raise_if(done)
     import torch
     B, Hq, D = _q_shape(q)
     out = _check_q_out(q, out)
@@ -358,6 +389,10 @@ def fmha_decode(q, k, v, cu_seqlens_kv=None, seqlen_kv=None, softmax_scale=None,
     fp32_weights: keep the softmax weights in fp32 (fmha_vectorized_fma's
       semantics) instead of rounding them to bf16; needs cu_seqlens_kv.
     """
+    done = (_native or _load_native()).decode(q, k, v, cu_seqlens_kv, seqlen_kv, softmax_scale, out, fp32_weights,
+                                              exact, fast)
+    if done is not None:
+        return done if done.__class__ is not int else _raise_if(done)
     import torch
 
     if q.dim() == 4:

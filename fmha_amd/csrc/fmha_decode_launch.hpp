@@ -259,8 +259,8 @@ constexpr int kSplitScoresWavesPerCU = 12;
 // Rows longer than 16 go through one pass (onepass_decode_kernel: one wave
 // per batch and head group, no workspace traffic, one launch) when there are
 // at least 512 such units and the row's scores and weights fit the wave's
-// LDS budget; otherwise through the four split-KV launches.  Measured
-// (µs, split -> one pass, 8 waves per CU): B=2048 Hq=32 Hkv=8 S=128 201 ->
+// LDS budget; otherwise through split-KV.  Measured (against
+// its earlier four launches, µs, split -> one pass, 8 waves per CU): B=2048 Hq=32 Hkv=8 S=128 201 ->
 // 171; B=4096 S=64 206 -> 178; B=16384 S=24 327 -> 296; B=256 S=256 (512
 // units) 69 -> 58; B=128 S=256 (256 units) 43 -> 49 and B=16 S=256 23 -> 49,
 // where a wave's walk over its row outlasts split-KV's shorter waves.
@@ -340,8 +340,35 @@ hipError_t launch_onepass_kernel(const SplitArgs& a, size_t need, int waves, hip
   return hipGetLastError();
 }
 
+// Longest rows first (SplitArgs::order_groups) with more units than start at
+// once and up to kOrderMaxRounds times that: a launch in batch order ends on
+// one wave of a late long row; more rounds hide that.  Not for one query head
+// per KV head on rows of up to four blocks (two on two), where the order
+// leaves the shortest rows, mostly latency, alone at the end (one-row pages
+// gain there too).  µs, in batch order / longest first, lengths log-uniform
+// over max / 32 to max: packed 32/8 D=128 max 100, B=1200 42.8 / 34.0, 3000
+// 82.0 / 69.0, 5000 124.2 / 113.7, 7000 167.8 / 160.7, 12000 (12 rounds)
+// 282.7 / 283.3; 64/8 D=256 max 100 B=2000 127.7 / 101.9; 16-row pages 64/8
+// max 60 B=2000 53.8 / 40.2; 32/32 B=400 max 100 38.1 / 33.4, but max 24 16.0
+// / 17.4, BHSD B=1000 max 64 53.6 / 55.3, D=256 B=700 max 40 52.6 / 59.8;
+// one-row pages B=600 max 40 30.4 / 24.4; all rows equal, B=2000 S=100 32/8
+// 136.0 / 135.4.
+constexpr int kOrderWavesPerCU = 8;
+constexpr int kOrderMaxRounds = 8;
+
+template <int G, int LAYOUT>
+uint32_t onepass_order_groups(const SplitArgs& a) {
+  const int64_t cus = device_cus() > 0 ? device_cus() : 256;
+  const int64_t at_once = kOrderWavesPerCU * cus;
+  const bool order = a.len_mode != fmha_decode::kLenUniform && (G * a.nblk > 4 || LAYOUT == fmha_decode::kLayoutPaged) &&
+                     onepass_waves(a) > at_once && onepass_waves(a) <= kOrderMaxRounds * at_once;
+  return order ? ((uint32_t)a.batch + kWaveSize - 1) / kWaveSize : 0;
+}
+
 template <int D, int G, int LAYOUT, bool MULTI>
-hipError_t launch_onepass_dg(const SplitArgs& a, hipStream_t stream) {
+hipError_t launch_onepass_dg(const SplitArgs& args, hipStream_t stream) {
+  SplitArgs a = args;
+  a.order_groups = MULTI ? 0 : onepass_order_groups<G, LAYOUT>(a);
   const size_t need = fmha_decode::onepass_lds_bytes<D, G>(fmha_decode::onepass_lds_rows(a.nblk));
   int waves = LAYOUT == fmha_decode::kLayoutPaged && G <= 2 ? kOnepassWavesPerCUPagedRows
               : !MULTI && G <= 2 && a.nblk <= 3     ? kOnepassWavesPerCUNarrow
@@ -697,13 +724,16 @@ int onepass_reg_tiles(const SplitArgs& a) {
   }
 }
 
-// Longest rows first (SplitArgs::longest_first) at 16 and 32 tiles per wave
-// with more waves than the CUs hold at once (8 each), where the order decides
-// what the launch ends on; below, every workgroup starts at once, or (8
-// tiles) ends soon, and the lengths' extra round trip costs (µs, all rows
-// equal, without / with: B=128 S=256 32/8 25.9 / 27.3, BHSD B=100 S=512
-// 16/16 69.8 / 72.9; ragged B=256 64/8 over 16-500 rows 46.4 either way).
-constexpr int kOrderWavesPerCU = 8;
+// Longest rows first (SplitArgs::order_groups) at 16 and 32 tiles per wave
+// with more waves than the CUs hold at once (kOrderWavesPerCU each), where
+// the order decides what the launch ends on; below, every workgroup starts
+// at once, or (8 tiles) ends soon, and the lengths' extra round trip costs
+// (µs, all rows equal, without / with: B=128 S=256 32/8 25.9 / 27.3, BHSD
+// B=100 S=512 16/16 69.8 / 72.9; ragged B=256 64/8 over 16-500 rows 46.4
+// either way), and up to kOrderRegMaxRounds times as many (64/8 lengths log-
+// uniform up to 1000: B=300, 9 rounds, 82.1 in batch order / 76.1, B=600
+// 152.8 / 150.1, B=2000 479.0 / 493.7).
+constexpr int kOrderRegMaxRounds = 20;
 
 template <int D, int LAYOUT>
 hipError_t launch_onepass_reg(const SplitArgs& args, int tpw, hipStream_t stream) {
@@ -715,8 +745,9 @@ hipError_t launch_onepass_reg(const SplitArgs& args, int tpw, hipStream_t stream
             layout_name(LAYOUT), nw, tpw, a.nblk);
   const int64_t units = (int64_t)a.batch * a.num_heads_kv;
   const int64_t cus = device_cus() > 0 ? device_cus() : 256;
-  a.longest_first = a.len_mode != fmha_decode::kLenUniform && a.batch > 1 && a.batch <= fmha_decode::kOrderBatches &&
-                    tpw > 8 && units * nw > kOrderWavesPerCU * cus;
+  const bool order = a.len_mode != fmha_decode::kLenUniform && a.batch > 1 && tpw > 8 &&
+                     units * nw > kOrderWavesPerCU * cus && units * nw <= kOrderRegMaxRounds * kOrderWavesPerCU * cus;
+  a.order_groups = order ? ((uint32_t)a.batch + kWaveSize - 1) / kWaveSize : 0;
   const uint32_t round_tiles = (uint32_t)(nw * fmha_decode::onepass_reg_round_tiles(D, tpw, LAYOUT));
   a.round_inv = (65536u + round_tiles - 1) / round_tiles;
   const dim3 grid((uint32_t)units);

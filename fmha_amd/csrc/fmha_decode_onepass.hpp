@@ -83,6 +83,15 @@ constexpr size_t onepass_lds_bytes(int sp, int nw = 1) {
 // would, and forms the weights of its own rows); waves 1..NW-1 hand their
 // P.V sums to wave 0 through LDS, which adds them in wave order.  For rows
 // with too few (batch, KV-head group) units to fill the GPU one wave each.
+// Short rows are bound by latency and by instructions spent past their ends,
+// so the last sub-blocks of a row are peeled off: nothing is scored,
+// multiplied or requested past the last one, and V's first rows are requested
+// right behind the last K rows (µs, every row in pairs of sub-blocks with
+// refills past its end / peeled: packed 32/8 D=128 B=3000 lengths 3-100 75.0
+// / 68.5, S=33 86.0 / 79.5, S=48 106.3 / 102.1, B=1500 S=100 106.1 / 103.9;
+// 32/32 B=600 lengths 2-64 40.7 / 34.8; D=256 B=700 up to 40 75.4 / 59.8).
+// With more units than start at once the longest rows go first
+// (SplitArgs::order_groups; measured at the rule that sets it).
 // ROWS8: 8-row sub-blocks, half the registers of 16-row ones (123 against
 // 208 VGPRs at G = 4 on pages under 16 rows with one batch per wave, 145
 // against 242 at G = 8 packed), for more waves per CU where the LDS leaves
@@ -124,6 +133,7 @@ __global__ __launch_bounds__(kBlockThreads * NW) __attribute__((amdgpu_waves_per
   uint32_t b0, nb, b;
   int sub, hk, S, smax, rel_rows = 0;
   bool head_ok, bad = false;
+  int64_t row_base = 0;  // packed, one batch per wave: its first row
   if constexpr (!MULTI) {
     // One (batch, KV-head group) per wave; the length is the wave's.
     const uint32_t unit = blockIdx.x;
@@ -131,12 +141,17 @@ __global__ __launch_bounds__(kBlockThreads * NW) __attribute__((amdgpu_waves_per
     b = unit / upb;
     if (b >= (uint32_t)a.batch) return;
     const uint32_t hg = unit - b * upb;
+    if (NW == 1 && a.order_groups != 0) {
+      b = longest_of_group<LAYOUT>(a, b, lane, S, row_base);
+    } else {
+      S = split_len_l<LAYOUT>(a, b);
+      row_base = split_row_base<LAYOUT>(a, b);
+    }
     b0 = b;
     nb = 1;
     sub = 0;
     hk = (int)hg * HPW + hkl;
     head_ok = hk < a.num_heads_kv;
-    S = split_len_l<LAYOUT>(a, b);
     smax = S;
     if (S <= 0 || S > a.max_rows) {
       // Empty rows give 0 (the reference loop's result), invalid ones NaN.
@@ -208,7 +223,7 @@ __global__ __launch_bounds__(kBlockThreads * NW) __attribute__((amdgpu_waves_per
   if constexpr (!MULTI || LANES) {
     // One batch per wave, or per-lane pages: each lane group addresses its
     // own batch's rows.
-    const int64_t row_base = split_row_base<LAYOUT>(a, b);
+    if constexpr (MULTI) row_base = split_row_base<LAYOUT>(a, b);
     krows.init(a, a.k, b, row_base, 0, S, hk, head_ok, r);
     vrows.init(a, a.v, b, row_base, 0, S, hk, head_ok, r);
   } else {
@@ -229,7 +244,8 @@ __global__ __launch_bounds__(kBlockThreads * NW) __attribute__((amdgpu_waves_per
   const int lo = wv * wrows;
   const int span = NW == 1 ? smax : (smax - lo < 0 ? 0 : (smax - lo < wrows ? smax - lo : wrows));
   const int sk0 = lo / NR;                              // first sub-block
-  const int nsub = ((span + NR - 1) / NR + 1) / 2 * 2;  // even
+  const int nk = (span + NR - 1) / NR;
+  const int nsub = (nk + 1) / 2 * 2;  // even
   auto load_k = [&](u32x4 (&kr)[NR], int s) { krows.template load<NR>(kr, s * NR); };
   // Per-lane lookups: each sub-block's block-table entries (one per row on
   // pages under 16 rows, else one) are requested two sub-blocks ahead,
@@ -265,6 +281,9 @@ __global__ __launch_bounds__(kBlockThreads * NW) __attribute__((amdgpu_waves_per
   };
   const int sv0 = lo / NRV;    // this wave's first V sub-block
   int32_t eva[NEV], evb[NEV];  // per-lane lookups: the next V entries
+  using VBuf = u32x4[NRV];
+  VBuf va, vb;
+  auto load_v = [&](u32x4 (&vr)[NRV], int s) { vrows.template load<NRV>(vr, s * NRV); };
   {
     // Two sub-blocks in flight: a register set is refilled as soon as it has
     // been scored (past the row's end the refills read 0 without access).
@@ -313,7 +332,8 @@ __global__ __launch_bounds__(kBlockThreads * NW) __attribute__((amdgpu_waves_per
       __builtin_amdgcn_sched_barrier(0);
       load_k(kb, sk0 + 1);
       __builtin_amdgcn_sched_barrier(0);
-      for (int s = sk0; s < sk0 + nsub; s += 2) {
+      int s = sk0;
+      for (; s + 2 < sk0 + nk; s += 2) {
         score(ka, s);
         __builtin_amdgcn_sched_barrier(0);
         load_k(ka, s + 2);
@@ -323,24 +343,24 @@ __global__ __launch_bounds__(kBlockThreads * NW) __attribute__((amdgpu_waves_per
         load_k(kb, s + 3);
         __builtin_amdgcn_sched_barrier(0);
       }
+      // The last one or two refill nothing: the first V sub-blocks follow
+      // them at once and arrive during the softmax.
+      if (NW == 1 || nk > 0) score(ka, s);
+      __builtin_amdgcn_sched_barrier(0);
+      load_v(va, sv0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (s + 1 < sk0 + nk) score(kb, s + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      load_v(vb, sv0 + 1);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
-  // The first two V sub-blocks are requested before the softmax, which they
-  // do not depend on, so they arrive while it runs.
-  using VBuf = u32x4[NRV];
-  VBuf va, vb;
-  auto load_v = [&](u32x4 (&vr)[NRV], int s) { vrows.template load<NRV>(vr, s * NRV); };
   if constexpr (LANES) {
     vrows.template load_entries<NRV>(va, sv0 * NRV, eva);
     __builtin_amdgcn_sched_barrier(0);
     vrows.template entries<NRV>(eva, (sv0 + 2) * NRV);
     __builtin_amdgcn_sched_barrier(0);
     vrows.template load_entries<NRV>(vb, (sv0 + 1) * NRV, evb);
-    __builtin_amdgcn_sched_barrier(0);
-  } else {
-    load_v(va, sv0);
-    __builtin_amdgcn_sched_barrier(0);
-    load_v(vb, sv0 + 1);
     __builtin_amdgcn_sched_barrier(0);
   }
   // An unmapped page among rows [0, S) (seen by the K phase, which reads
@@ -401,7 +421,8 @@ __global__ __launch_bounds__(kBlockThreads * NW) __attribute__((amdgpu_waves_per
   for (int g = 0; g < G; ++g)
 #pragma unroll
     for (int d = 0; d < 8; ++d) acc[g][d] = 0.0f;
-  const int nsv = ((span + NRV - 1) / NRV + 1) / 2 * 2;  // even
+  const int nv = (span + NRV - 1) / NRV;
+  const int nsv = (nv + 1) / 2 * 2;  // even
   auto pv = [&](const u32x4 (&vr)[NRV], int s) {
     uint32_t pp[G][NRV / 2];
 #pragma unroll
@@ -433,7 +454,8 @@ __global__ __launch_bounds__(kBlockThreads * NW) __attribute__((amdgpu_waves_per
     __builtin_amdgcn_sched_barrier(0);
     pv(vb, s + 1);
   } else {
-    for (int s = sv0; s < sv0 + nsv; s += 2) {
+    int s = sv0;
+    for (; s + 2 < sv0 + nv; s += 2) {
       pv(va, s);
       __builtin_amdgcn_sched_barrier(0);
       load_v(va, s + 2);
@@ -443,6 +465,9 @@ __global__ __launch_bounds__(kBlockThreads * NW) __attribute__((amdgpu_waves_per
       load_v(vb, s + 3);
       __builtin_amdgcn_sched_barrier(0);
     }
+    if (NW == 1 || nv > 0) pv(va, s);
+    __builtin_amdgcn_sched_barrier(0);
+    if (s + 1 < sv0 + nv) pv(vb, s + 1);
   }
   if constexpr (NW > 1) {
     // Waves 1..NW-1 hand their sums to wave 0 (LDS after the weights),

@@ -96,13 +96,13 @@ struct SplitArgs {
   // the kernels' G runs as kv_groups groups of G on one launch, launch head
   // hk reading memory head hk / kv_groups of num_heads_kv / kv_groups.
   int32_t kv_groups;
-  // Register single pass: 1: workgroups take the batches longest row first
-  // (longest_first; at most kOrderBatches batches), 0: as they come.
-  int32_t longest_first;
   // Register single pass: ceil(2^16 / n) for the n tiles that the
   // workgroup's waves stage in one round, so that x / n is x * round_inv >>
   // 16 (exact for x * n < 2^16; x is below 512 and n at most 64).
   uint32_t round_inv;
+  // Single passes: ceil(batch / 64) with the batches taken about longest row
+  // first (longest_of_group), 0: as they come.
+  uint32_t order_groups;
 };
 
 // KV heads of the cache in memory, and the one launch head hk reads.
@@ -154,50 +154,40 @@ __device__ __forceinline__ void batch_lengths(const SplitArgs& a, int lane, int 
 }
 
 // The batch that workgroup group i (< batch) of a single-pass launch serves
-// with SplitArgs::longest_first: the one with the i-th longest row, in 16-row
-// blocks, ties in batch order, so that the longest rows start first and the
-// launch does not end on one of them alone.  Every lane of the wave calls it;
-// every wave of every workgroup finds the same order.
+// with SplitArgs::order_groups (n): about the one with the i-th longest row,
+// in 16-row blocks, so that the longest rows start first and the launch does
+// not end on one of them alone.  The batches form n strided groups of up to
+// 64 (group g: g, g + n, g + 2n, ...), one length per lane, each a sample of
+// the whole: every group's longest row goes first, then every group's second
+// longest, and so on (exactly in order up to 64 batches).  Group i of the
+// launch serves the (i / n)-th longest of group i % n, ties in batch order (a
+// group has ceil((batch - g) / n) members, so every batch is served once);
+// equal rows come out as they come.  Every lane of the wave calls it; every
+// wave of every workgroup finds the same order.  Also gives the length and,
+// for packed caches, the batch's first row, which the lanes hold already.
 template <int LAYOUT>
-__device__ __forceinline__ uint32_t longest_first(const SplitArgs& a, uint32_t i, int lane) {
-  if (__builtin_expect(!a.longest_first, 1)) return i;  // the search stays out of the other launches' straight-line code
-  int blocks[kOrderRegs];  // -1: no batch
-  batch_lengths<LAYOUT>(a, lane, blocks);
-#pragma unroll
-  for (int p = 0; p < kOrderRegs; ++p) {
-    const int S = blocks[p];
-    blocks[p] = p * kWaveSize + lane >= a.batch ? -1
-                : S < 0 || S > a.max_rows       ? 0
-                                                : (S + kSplitBlockRows - 1) / kSplitBlockRows;
-  }
-  // Rows of at least v blocks, as a count over the wave.
-  auto at_least = [&](int v) {
-    int n = 0;
-#pragma unroll
-    for (int p = 0; p < kOrderRegs; ++p) n += __popcll(__builtin_amdgcn_ballot_w64(blocks[p] >= v));
-    return n;
-  };
-  // One length for all: as they come.
-  const int first = __builtin_amdgcn_readfirstlane(blocks[0]);
-  if (at_least(first) == a.batch && at_least(first + 1) == 0) return i;
-  // v: the i-th largest block count, bit by bit.
+__device__ __forceinline__ uint32_t longest_of_group(const SplitArgs& a, uint32_t i, int lane, int& S,
+                                                     int64_t& row_base) {
+  const uint32_t n = a.order_groups;
+  const uint32_t rank = i / n;
+  const uint32_t mine = i - rank * n + n * (uint32_t)lane;
+  const uint32_t b = min(mine, (uint32_t)a.batch - 1);
+  const int first = LAYOUT == kLayoutPacked ? a.cu[b] : 0;
+  const int len = LAYOUT == kLayoutPacked ? a.cu[b + 1] - first : split_len_l<LAYOUT>(a, b);
+  const int blocks = mine >= (uint32_t)a.batch       ? -1
+                     : len < 0 || len > a.max_rows ? 0
+                                                   : (len + kSplitBlockRows - 1) / kSplitBlockRows;
+  auto at_least = [&](int v) { return __popcll(__builtin_amdgcn_ballot_w64(blocks >= v)); };
   int v = 0;
   for (int bit = 31 - __clz(a.nblk); bit >= 0; --bit)
-    if (at_least(v | (1 << bit)) > (int)i) v |= 1 << bit;
-  int r = (int)i - at_least(v + 1);  // its place among the rows of v blocks
-  uint32_t found = i;
-#pragma unroll
-  for (int p = 0; p < kOrderRegs; ++p) {
-    const uint64_t m = __builtin_amdgcn_ballot_w64(blocks[p] == v);
-    const int n = __popcll(m);
-    if (r >= 0 && r < n) {
-      const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
-      found = (uint32_t)(p * kWaveSize) +
-              (uint32_t)__builtin_ctzll(__builtin_amdgcn_ballot_w64(blocks[p] == v && before == r));
-    }
-    r -= n;
-  }
-  return found;
+    if (at_least(v | (1 << bit)) > (int)rank) v |= 1 << bit;
+  const int r = (int)rank - at_least(v + 1);  // its place among the rows of v blocks
+  const uint64_t m = __builtin_amdgcn_ballot_w64(blocks == v);
+  const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+  const int found = (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(blocks == v && before == r));
+  S = __builtin_amdgcn_readlane(len, found);
+  row_base = __builtin_amdgcn_readlane(first, found);
+  return (uint32_t)__builtin_amdgcn_readlane((int)mine, found);
 }
 
 // Wave barrier between LDS writes and reads of one wave.

@@ -466,7 +466,7 @@ __global__ __launch_bounds__(kBlockThreads * NW) void onepass_mfma_kernel(SplitA
 //     staging's space), which adds them in wave order and writes fp16 O.
 // Rows past the wave's range are never read (out-of-range offsets read 0).
 // A row's tiles are shared evenly among the waves whatever its length, and
-// with many workgroups the longest rows go first (longest_first): on ragged
+// with many workgroups the longest rows go first (longest_of_group): on ragged
 // batches a launch otherwise ends on one wave of a late long row (µs, 16-row
 // pages, B=64 32/8, lengths log-uniform over 128-4096, 305 MB: 117.6 with
 // shares of the longest row in batch order, 69.7; packed B=256 64/8 32-1024:
@@ -544,10 +544,17 @@ __global__ __launch_bounds__(kBlockThreads * NWMAX) void onepass_mfma_reg_kernel
   const uint32_t bi = blockIdx.x / hkv;
   const uint32_t hk = blockIdx.x - bi * hkv;
   if (bi >= (uint32_t)a.batch) return;
-  const uint32_t b = longest_first<LAYOUT>(a, bi, lane);
+  uint32_t b = bi;
+  int S;
+  int64_t row_base;
+  if (TPW > 8 && __builtin_expect(a.order_groups != 0, 0)) {
+    b = longest_of_group<LAYOUT>(a, bi, lane, S, row_base);
+  } else {
+    S = split_len_l<LAYOUT>(a, b);
+    row_base = split_row_base<LAYOUT>(a, b);
+  }
   const int hq = a.num_heads_q;
   const int G = hq / (int)hkv;  // <= 16
-  const int S = split_len_l<LAYOUT>(a, b);
   const int q = lane >> 4;
   const int n = lane & 15;
   const bool gok = n < G;
@@ -605,7 +612,7 @@ __global__ __launch_bounds__(kBlockThreads * NWMAX) void onepass_mfma_reg_kernel
   const int ph = (s / RT) * KR;  // and its first row in it
   char* stage = onepass_reg_lds + onepass_reg_stage_offset<D>(nw) + (size_t)wv * KSR * NR;
   typename std::conditional<PAGED || PAGED_ROWS, PagedLaneRows<D, PAGED>, LongRows<D, LAYOUT>>::type kr;
-  kr.init(a, a.k, b, split_row_base<LAYOUT>(a, b), lo, lo + span, (int)hk, true, r, ps * NR + ph);
+  kr.init(a, a.k, b, row_base, lo, lo + span, (int)hk, true, r, ps * NR + ph);
   f32x4_v x[TPW];
   float m = -__builtin_inff();
   if (nt > 0) {
@@ -679,7 +686,7 @@ __global__ __launch_bounds__(kBlockThreads * NWMAX) void onepass_mfma_reg_kernel
   // if its K loads have (V reads the same rows through the same table).
   if constexpr (PAGED_ROWS) unmapped = __builtin_amdgcn_ballot_w64(kr.bad != 0) != 0 ? 1 : 0;
   LongRows<D, PAGED || PAGED_ROWS ? kLayoutPacked : LAYOUT> vrw;
-  if constexpr (!PAGED && !PAGED_ROWS) vrw.init(a, a.v, b, split_row_base<LAYOUT>(a, b), 0, S, (int)hk, true, 0);
+  if constexpr (!PAGED && !PAGED_ROWS) vrw.init(a, a.v, b, row_base, 0, S, (int)hk, true, 0);
   const uint32_t v_row_bytes = (uint32_t)kv_heads_mem(a) * D * 2u;       // paged: bytes per slot
   const uint32_t v_head_off = (uint32_t)kv_head_mem(a, (int)hk) * D * 2u;  // paged: this KV head in a slot
   uint32_t vr[PF][4][VW];

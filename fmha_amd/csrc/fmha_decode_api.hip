@@ -547,6 +547,8 @@ struct SplitPlan {
 // B=6 64/8 over 1024-32768 64.9 (430) / 63.3 (215) / 73.4 (107) at 1024 /
 // 2048 / 4096; D=64 B=22 8/8 over 666-21321 65.3 (512) / 71.5 (256) at 2048 /
 // 4096; D=256 B=10 8/8 over 360-11516 65.8 (504) / 69.6 (252) at 512 / 1024).
+// Not a size that leaves the last of two or three pieces of a row mostly
+// empty (D=64 B=57 8/8 S=2233: 72.1 at 2048 rows, 59.9 at 1024). 
 constexpr int64_t kPvMinGroups = 448, kPvFewGroups = 192;
 constexpr int kPvMinShift = 8, kPvMaxShift = 12;
 
@@ -556,9 +558,13 @@ SplitPlan plan_split(int64_t batch, int hq, int hkv, int max_rows, int d) {
   p.units = (hkv + heads_per_wave - 1) / heads_per_wave * batch;
   const auto groups = [&](int shift) { return max_rows <= 0 ? 1 : ((int64_t)max_rows + (1 << shift) - 1) >> shift; };
   p.pv_shift = kPvMaxShift;
-  while (p.pv_shift > kPvMinShift &&
-         (batch * hkv * groups(p.pv_shift) < kPvMinGroups || (max_rows > 1024 && groups(p.pv_shift) < 2)))
-    --p.pv_shift;
+  const auto fits = [&](int shift) {
+    const int64_t n = groups(shift), all = batch * hkv * n;
+    if (max_rows > 1024 && n < 2) return false;
+    if (n > 1 && n < 4 && (int64_t)max_rows * 10 < 7 * (n << shift)) return false;
+    return all >= kPvMinGroups;
+  };
+  while (p.pv_shift > kPvMinShift && !fits(p.pv_shift)) --p.pv_shift;
   // FMHA_DECODE_SPLIT_CHUNK=<128|...|4096>: rows of a P.V workgroup instead
   // (for sweeps; the workspace size follows, and a launch checks its
   // workspace against it).

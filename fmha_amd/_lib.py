@@ -12,9 +12,9 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 # library that fmha_amd/_build.py writes.
 LIB_PATH = os.environ.get("FMHA_DECODE_LIB") or os.path.join(_HERE, "libfmha_decode.so")
 
-# The tensor interface's native module (fmha_amd/csrc/fmha_decode_torch.cpp)
-# and the entry points it is bound to, in the order of its Library.
-HOST_PATH = os.path.join(_HERE, "_host.so")
+# The entry points that the tensor interface's native module
+# (fmha_amd/csrc/fmha_decode_torch.cpp) is bound to, in the order of its
+# Library.
 HOST_ENTRIES = (
     "fmha_decode_fwd",
     "fmha_decode_fwd_fast",

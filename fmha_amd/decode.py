@@ -12,10 +12,12 @@ Two levels, both thin wrappers over the C ABI in include/fmha_decode.h:
   stream.  fmha_decode_strided and fmha_decode_paged do the same for strided
   (BSHD / BHSD / padded) and paged KV caches.  Plainly acceptable calls take
   the native form of these functions (csrc/fmha_decode_torch.cpp), which
-  leaves every other one, with its error message, to the code here.
+  leaves every other one, with its error message, to the code here; where its
+  module does not load, all of them come here.
 """
+import importlib
 import math
-import os
+import warnings
 
 from . import _lib
 
@@ -37,19 +39,36 @@ class FmhaDecodeError(RuntimeError):
 _native = None
 
 
+class _PythonOnly:
+    """The native module's functions where it does not load: every call is
+    left to the Python form."""
+
+    @staticmethod
+    def _leave(*args):
+        return None
+
+    decode = splitkv = strided = paged = _leave
+
+
 def _load_native():
-    """The native forms of the tensor functions, bound to the loaded library."""
+    """The native forms of the tensor functions, bound to the loaded library.
+    The module is compiled against one torch and is a shortcut only: where it
+    is not built, or does not load with the installed torch, the Python forms
+    serve every call (about 8 us more each), and a warning says so once."""
     global _native
     import ctypes
     import torch  # noqa: F401  (its libraries are what the module links to)
     lib = _lib.load()
-    if not os.path.exists(_lib.HOST_PATH):
-        raise RuntimeError(
-            f"{_lib.HOST_PATH} is not built; run `python -c 'import __graft_entry__ as g; g.build()'`")
-    from . import _host
-    _host.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _lib.HOST_ENTRIES))
-    _native = _host
-    return _host
+    try:
+        native = importlib.import_module("._host", __package__)
+    except ImportError as e:
+        warnings.warn(f"fmha_amd: the native call path is not used ({e}); run "
+                      "`python -c 'import __graft_entry__ as g; g.build()'`", RuntimeWarning, stacklevel=3)
+        native = _PythonOnly
+    else:
+        native.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _lib.HOST_ENTRIES))
+    _native = native
+    return native
 
 
 def last_plan():

@@ -2,6 +2,8 @@
 what it takes gives the Python form's results, and what it leaves alone
 raises the Python form's errors."""
 import math
+import sys
+import warnings
 
 import pytest
 import torch
@@ -45,6 +47,32 @@ def test_leaves_what_it_does_not_know():
         n.bind(1)
     with pytest.raises(ValueError):
         n.bind(*([0] * 12))
+
+
+def test_works_without_the_module(monkeypatch):
+    """Where the native module does not load, one warning, and every call is
+    the Python form's, with its errors; the library itself still has to be
+    there."""
+    monkeypatch.setitem(sys.modules, "fmha_amd._host", None)
+    monkeypatch.setattr(decode, "_native", None)
+    q, k, v = _cpu_case()
+    lens = torch.zeros(2, dtype=torch.int32)
+    with pytest.warns(RuntimeWarning, match="native call path"):
+        with pytest.raises(ValueError, match="q must be"):
+            fmha_amd.fmha_decode(q, k, v)
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        with pytest.raises(ValueError):
+            fmha_amd.fmha_decode_splitkv(q, k, v, lens, 3)
+        with pytest.raises(ValueError):
+            fmha_amd.fmha_decode_strided(q, k, v)
+        with pytest.raises(ValueError):
+            fmha_amd.fmha_decode_paged(q, k, v, lens.view(2, 1), lens)
+    monkeypatch.setattr(decode, "_native", None)
+    monkeypatch.setattr(decode._lib, "_lib", None)
+    monkeypatch.setattr(decode._lib, "LIB_PATH", "/nonexistent/libfmha_decode.so")
+    with pytest.raises(RuntimeError, match="not built"):
+        fmha_amd.fmha_decode(q, k, v)
 
 
 def _args(layout):

@@ -127,7 +127,7 @@ constexpr uint32_t kPermHi = 0x07060302u;
 // than every other 16 bytes of 512 (half-written lines doubled the HBM
 // write bytes), and the V^T reads land on distinct banks.
 template <int DPC>
-__device__ __forceinline__ int out_dim(int n, int dt) {
+__host__ __device__ __forceinline__ constexpr int out_dim(int n, int dt) {
   return DPC <= 8 ? n * DPC + dt : (dt / 8) * 128 + n * 8 + dt % 8;
 }
 

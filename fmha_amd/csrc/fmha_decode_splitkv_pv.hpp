@@ -15,8 +15,9 @@
 //     own layout would have every lane form 4 per tile, 16 / G times too
 //     many) and pass through LDS into the A operand of D/16
 //     v_mfma_f32_16x16x16_bf16 per tile; V comes straight from memory in the
-//     B operand's rows (lane (q, n): rows 4q..4q+3 at dims [n D/16, +D/16)),
-//     transposed in registers with v_perm, GT tiles in flight;
+//     B operand's rows (lane (q, n): rows 4q..4q+3 at the D/16 dims of
+//     out_dim(n, ...)), transposed in registers with v_perm, GT tiles in
+//     flight;
 //   * the waves' fp32 sums are added in wave order through LDS and written
 //     as fp16 O by a row's only workgroup, else as fp32 partial outputs, of
 //     which the last workgroup to finish of each kPvFan neighbours adds
@@ -65,8 +66,10 @@ constexpr int pv_lds_bytes() {
 }
 
 // One wave's V tiles (16 rows of one (batch, KV head) each) in the B
-// operand's rows: lane (q, n) gets rows 4q..4q+3 at dims [n DPC, n DPC +
-// DPC).  Tiles are step_tiles apart from row `first` on; rows at or past
+// operand's rows: lane (q, n) gets rows 4q..4q+3 at dims out_dim(n, 0..DPC-1),
+// so that each load instruction reads whole lines of a row (µs of the call
+// at D = 256, 16 neighbouring dims per lane / this: 28/4 B=3 S=66558 on 64-row
+// pages 197 / 179, packed 64/8 B=16 S=4096 106 / 101).  Tiles are step_tiles apart from row `first` on; rows at or past
 // `end` read 0, without memory access (on pages under 16 rows from Q's first
 // row).  Paged: an unmapped page (a negative entry) reads as 0 too; the
 // scores launch has made the batch's statistics NaN then.
@@ -75,7 +78,8 @@ struct VTiles {
   static constexpr bool PAGED = LAYOUT == kLayoutPagedBlock;    // a tile lies in one page
   static constexpr bool PAGED_ROWS = LAYOUT == kLayoutPaged;    // every row through its own entry
   static constexpr int DPC = D / 16;
-  static constexpr int VW = DPC / 2;  // dwords of a lane's run of a row
+  static constexpr int VW = DPC / 2;                 // dwords of a lane's dims of a row
+  static constexpr int RUN = out_dim<DPC>(0, 8);     // dims from a lane's first 16 bytes of a row to its next
   __amdgpu_buffer_rsrc_t rsrc;  // packed, strided: the batch's rows
   const uint16_t* v;
   const uint16_t* safe;
@@ -111,7 +115,7 @@ struct VTiles {
       row_bytes = rows.row_bytes;
       head_off = rows.lane_off;
     }
-    lane_off = head_off + (uint32_t)((lane & 15) * DPC * 2) + (PAGED_ROWS ? 0u : 4u * (uint32_t)q * row_bytes);
+    lane_off = head_off + (uint32_t)out_dim<DPC>(lane & 15, 0) * 2u + (PAGED_ROWS ? 0u : 4u * (uint32_t)q * row_bytes);
   }
 
   // PAGED_ROWS: the block-table entries of this lane's rows of tile k, to be
@@ -144,7 +148,7 @@ struct VTiles {
         } else {
 #pragma unroll
           for (int h = 0; h < VW / 4; ++h) {
-            const u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src) + h);
+            const u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src + h * RUN));
 #pragma unroll
             for (int j = 0; j < 4; ++j) out[i][4 * h + j] = ok ? w[j] : 0u;
           }
@@ -179,7 +183,7 @@ struct VTiles {
 #pragma unroll
           for (int h = 0; h < VW / 4; ++h) {
             const u32x4 w = __builtin_bit_cast(
-                u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off + h * 16, (int)at, kPolicyStream));
+                u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off + h * (RUN * 2), (int)at, kPolicyStream));
 #pragma unroll
             for (int j = 0; j < 4; ++j) out[i][4 * h + j] = w[j];
           }
@@ -434,7 +438,7 @@ __global__ __launch_bounds__(kPvThreads) void splitkv_pv_kernel(SplitArgs a) {
     wave_lds_sync();  // the weights are read
   }
 
-  // Lane (q, n) holds query columns 4q..4q+3, dims [n DPC, n DPC + DPC).
+  // Lane (q, n) holds query columns 4q..4q+3, dims out_dim(n, 0..DPC-1).
   if (nw == 1) {  // the row's only wave
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -442,7 +446,7 @@ __global__ __launch_bounds__(kPvThreads) void splitkv_pv_kernel(SplitArgs a) {
 #pragma unroll
       for (int d = 0; d < DPC; ++d) v[d] = acc[d][e];
       const int g = 4 * q + e;
-      store_f16_run<DPC>(o_rsrc, g < gn ? (uint32_t)(g * D + n * DPC) * 2u : kLaneOutOfRange, v);
+      store_f16_cols<DPC>(o_rsrc, g < gn ? (uint32_t)(g * D) * 2u : kLaneOutOfRange, n, v);
     }
     return;
   }
@@ -456,7 +460,7 @@ __global__ __launch_bounds__(kPvThreads) void splitkv_pv_kernel(SplitArgs a) {
     if (g < GC) {
 #pragma unroll
       for (int d4 = 0; d4 < DPC / 4; ++d4)
-        *reinterpret_cast<f32x4_v*>(red + (wv * GC + g) * D + n * DPC + d4 * 4) =
+        *reinterpret_cast<f32x4_v*>(red + (wv * GC + g) * D + out_dim<DPC>(n, 4 * d4)) =
             f32x4_v{acc[4 * d4][e], acc[4 * d4 + 1][e], acc[4 * d4 + 2][e], acc[4 * d4 + 3][e]};
     }
   }

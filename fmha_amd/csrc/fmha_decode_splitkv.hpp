@@ -358,14 +358,17 @@ struct LongRows {
     if constexpr (LAYOUT == kLayoutPacked) {
       row_bytes = (uint32_t)hkv * D * 2u;
       lane_off = head_ok ? (uint32_t)(hm * D + r * 8) * 2u : kLaneOutOfRange;
-      rsrc = make_rsrc(t + ((uint64_t)row_base + lo) * hkv * D, (uint32_t)n * row_bytes);
+      rsrc = make_rsrc(uniform_ptr(t + ((uint64_t)row_base + lo) * hkv * D),
+                       (uint32_t)__builtin_amdgcn_readfirstlane(n * (int)row_bytes));
     } else if constexpr (LAYOUT == kLayoutStrided) {
       row_bytes = (uint32_t)a.row_stride * 2u;
       lane_off = head_ok ? (uint32_t)(hm * a.head_stride + r * 8) * 2u : kLaneOutOfRange;
       const uint32_t span = n == 0 ? 0u
                                    : ((uint32_t)(n - 1) * (uint32_t)a.row_stride +
                                       (uint32_t)(hkv - 1) * (uint32_t)a.head_stride + D) * 2u;
-      rsrc = make_rsrc(t + (uint64_t)b * (uint64_t)a.batch_stride + (uint64_t)lo * (uint64_t)a.row_stride, span);
+      rsrc = make_rsrc(uniform_ptr(t + (uint64_t)b * (uint64_t)a.batch_stride +
+                                   (uint64_t)lo * (uint64_t)a.row_stride),
+                       (uint32_t)__builtin_amdgcn_readfirstlane((int)span));
     } else {
       row_bytes = (uint32_t)hkv * D * 2u;
       lane_off = head_ok ? (uint32_t)(hm * D + r * 8) * 2u : kLaneOutOfRange;
@@ -646,6 +649,8 @@ __global__ __launch_bounds__(kBlockThreads * kScoresMaxWaves) void splitkv_score
   if (!batch_piece<LAYOUT>(a, u, a.sup_shift, (uint32_t)a.nsup, rp)) return;
   const uint32_t b = rp.b;
   const int S = rp.S;
+  // Ahead of clear_done's stores, behind which it is a vector load.
+  const int64_t row_base = split_row_base<LAYOUT>(a, b);
   if (rp.piece == 0) clear_done(a, b, hg * su.heads(), su.heads(), 1);
   if (S <= 0 || S > a.max_rows) return;
   const uint32_t wb = (rp.piece << (a.sup_shift - a.sub_shift - ilog2(NR))) + (uint32_t)wv;
@@ -664,7 +669,7 @@ __global__ __launch_bounds__(kBlockThreads * kScoresMaxWaves) void splitkv_score
   const __amdgpu_buffer_rsrc_t q_rsrc = make_rsrc(a.q + (uint64_t)b * hq * D, (uint32_t)hq * D * 2);
   // Rows [0, S) of the batch: rows past S read 0 without access.
   SplitRows<D, LAYOUT> kv;
-  kv.init(a, a.k, b, split_row_base<LAYOUT>(a, b), 0, S, hk, head_ok, r, p * NR);
+  kv.init(a, a.k, b, row_base, 0, S, hk, head_ok, r, p * NR);
   const uint32_t q_off = head_ok ? (uint32_t)(hk * G * D + r * 8) * 2u : kLaneOutOfRange;
 
   u32x4 qv[G];

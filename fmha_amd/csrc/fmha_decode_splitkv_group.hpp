@@ -64,6 +64,7 @@ __global__ __launch_bounds__(kBlockThreads) void splitkv_scores_group_kernel(Spl
   const int hq = a.num_heads_q;
   const int G = hq / (int)hkv;
   const int tiles = (G + 15) / 16;
+  const int64_t row_base = split_row_base<LAYOUT>(a, b);  // ahead of clear_done's stores (splitkv_scores_kernel)
   if (rp.piece == 0) clear_done(a, b, hk, 1, tiles);
   if (S <= 0 || S > a.max_rows) return;
   const int j0 = (int)(rp.piece << a.sup_shift);  // the wave's first row
@@ -74,7 +75,7 @@ __global__ __launch_bounds__(kBlockThreads) void splitkv_scores_group_kernel(Spl
 
   // K rows of the wave's blocks (lane group s: rows j0 + 16 s + j).
   GroupRows<D, LAYOUT> kv;
-  kv.init(a, a.k, b, split_row_base<LAYOUT>(a, b), 0, S, (int)hk, true, r, s * NR);
+  kv.init(a, a.k, b, row_base, 0, S, (int)hk, true, r, s * NR);
   u32x4 kr[NR];
   kv.template load<NR>(kr, j0);
   const bool kv_bad = kv.any_bad();

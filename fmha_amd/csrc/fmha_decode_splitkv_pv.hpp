@@ -165,7 +165,7 @@ struct VTiles {
         const int left = end - row0;
         const int rows = pr.unmapped || left < 0 ? 0 : (left < kSplitBlockRows ? left : kSplitBlockRows);
         r = make_rsrc(uniform_ptr(v + (uint64_t)pr.page * page_stride + (uint64_t)pr.slot * (row_bytes >> 1)),
-                      (uint32_t)rows * row_bytes);
+                      (uint32_t)__builtin_amdgcn_readfirstlane(rows * (int)row_bytes));
       } else {
         r = rsrc;
         at = (uint32_t)row0 * row_bytes;

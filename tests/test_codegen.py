@@ -30,12 +30,14 @@ def listings(tmp_path_factory):
     out = tmp / "kernels.s"
     subprocess.run([_build.hipcc(), *_build.HIPCC_FLAGS, "-I" + _build.CSRC, "-I" + os.path.join(_build.ROOT, "include"),
                     "-S", "--cuda-device-only", "-o", str(out), str(src)], check=True, capture_output=True)
-    found = {}
+    found, lines = {}, None
     for line in out.read_text().split("\n"):
         m = re.match(r"_ZN11fmha_decode\d+(\w+?)ILi(\w+?)EEEv", line)
         if m and line.split(";")[0].rstrip().endswith(":"):
             lines = found.setdefault((m.group(1), m.group(2).replace("ELi", ", ")), [])
-        elif found:
+        elif line.startswith(".Lfunc_end"):
+            lines = None
+        elif lines is not None:
             lines.append(line.strip())
     layouts = {"kLayoutPacked": "0", "kLayoutStrided": "1", "kLayoutPaged": "2", "kLayoutPagedBlock": "3"}
     by_name = {}
@@ -59,3 +61,20 @@ def test_wide_rows_are_read_in_whole_lines(listings):
         assert wide
         assert sum(re.search(r"offset:256\b", l) is not None for l in wide) == len(wide) // 2, k
         assert not any(re.search(r"offset:16\b", l) for l in wide), k
+
+
+@pytest.mark.parametrize("kernel", KERNELS)
+def test_descriptors_are_scalar(listings, kernel):
+    """No load goes through a loop over the lanes, which the compiler makes
+    of a buffer descriptor that it holds in vector registers."""
+    label, start, loops = None, 0, []
+    lines = listings[kernel]
+    for i, line in enumerate(lines):
+        m = re.match(r"(\.LBB\w+):", line)
+        if m:
+            label, start = m.group(1), i
+        elif label and line.startswith("s_cbranch_execnz") and label in line:
+            body = lines[start:i]
+            if any(l.startswith("v_readfirstlane") for l in body) and any(l.startswith("buffer_") for l in body):
+                loops.append(body)
+    assert not loops, "%d loops, the first:\n%s" % (len(loops), "\n".join(loops[0]))

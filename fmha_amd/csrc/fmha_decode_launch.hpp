@@ -474,24 +474,12 @@ hipError_t launch_onepass_group(const SplitArgs& a, hipStream_t stream) {
 
 // Launchers of the kernels every long-row path shares, defined once in the
 // part that owns them (fmha_decode_inst.hip, FMHA_DECODE_PART 0).
-// Rows of more than this many 16-row blocks count their statistics as a pass
-// of the plan text: joining them takes a P.V workgroup more than one load.
-constexpr int kPvStatBlocks = 64;
-
-// P.V workgroups of the longest row as the plan has it.
-inline int split_groups(const SplitArgs& a) { return (a.max_rows + (1 << a.pv_shift) - 1) >> a.pv_shift; }
-// Phases of a split-KV plan, for its text: scores, the statistics of rows of
-// more than kPvStatBlocks blocks, P.V, and the sum over the workgroups of a
-// row with more than one.
-inline int split_passes(const SplitArgs& a) { return 2 + (a.nblk > kPvStatBlocks) + (split_groups(a) > 1); }
-// The rows of one P.V wave's share (chunk) of the longest row, for its text:
-// the row itself, rounded up to blocks, with one workgroup per row.
-inline int split_chunk_rows(const SplitArgs& a) {
-  return split_groups(a) > 1 ? (1 << a.pv_shift) / fmha_decode::kPvWaves : a.nblk * fmha_decode::kSplitBlockRows;
-}
-inline int split_chunks(const SplitArgs& a) {
-  return split_groups(a) > 1 ? (a.max_rows + split_chunk_rows(a) - 1) / split_chunk_rows(a) : 1;
-}
+// The two launches of split-KV for the plan text: the rows of a scores
+// workgroup (each leaves one entry of the row's statistics), the rows of a P.V
+// workgroup (a piece) as planned and at least (the device may take shorter
+// ones), and the pieces of the longest row as planned.
+#define FMHA_DECODE_SPLIT_PLAN "scores_rows=%d pv_rows=%d pv_rows_least=%d pieces=%d launches=2"
+inline int split_pieces(const SplitArgs& a) { return (a.max_rows + (1 << a.pv_shift) - 1) >> a.pv_shift; }
 
 // The P.V launch of split-KV (splitkv_pv_kernel) after the scores launch of
 // either kind; instantiated in its own parts, which the others link to.
@@ -946,8 +934,8 @@ hipError_t launch_split_dg(const SplitArgs& a, hipStream_t stream, bool onepass_
   as.nsup = (a.max_rows + (1 << as.sup_shift) - 1) >> as.sup_shift;
   const int64_t groups = (int64_t)a.batch * as.nsup * as.units_per_batch;
   if (groups > INT32_MAX) return hipErrorInvalidValue;
-  plan_note("split(D=%d G=%d layout=%s sub_units=%d blocks=%d chunk_rows=%d chunks=%d passes=%d launches=2)", D, G,
-            layout_name(LAYOUT), 1 << shift, a.nblk, split_chunk_rows(a), split_chunks(a), split_passes(a));
+  plan_note("split(D=%d G=%d layout=%s sub_units=%d blocks=%d " FMHA_DECODE_SPLIT_PLAN ")", D, G, layout_name(LAYOUT),
+            1 << shift, a.nblk, 1 << as.sup_shift, 1 << a.pv_shift, 1 << a.pv_fine, split_pieces(a));
   constexpr auto kernel = fmha_decode::splitkv_scores_kernel<D, G, LAYOUT>;
   hipLaunchKernelGGL(kernel, dim3((uint32_t)groups), dim3(kBlockThreads * wpg),
                      lds_reserve_kernel<kernel>(kSplitScoresWavesPerCU / wpg), stream, as);
@@ -991,9 +979,9 @@ hipError_t launch_split_group_d(const SplitArgs& a, hipStream_t stream) {
   am.nsup = (a.max_rows + (1 << am.sup_shift) - 1) >> am.sup_shift;
   const int64_t groups = (int64_t)a.batch * am.nsup * a.num_heads_kv;
   if (groups > INT32_MAX) return hipErrorInvalidValue;
-  plan_note("split_matrix_core(D=%d G=%d layout=%s blocks=%d chunk_rows=%d chunks=%d passes=%d launches=2)", D,
-            a.num_heads_q / a.num_heads_kv, layout_name(LAYOUT), a.nblk, split_chunk_rows(a), split_chunks(a),
-            split_passes(a));
+  plan_note("split_matrix_core(D=%d G=%d layout=%s blocks=%d " FMHA_DECODE_SPLIT_PLAN ")", D,
+            a.num_heads_q / a.num_heads_kv, layout_name(LAYOUT), a.nblk, 1 << am.sup_shift, 1 << a.pv_shift,
+            1 << a.pv_fine, split_pieces(a));
   constexpr auto kernel = fmha_decode::splitkv_scores_group_kernel<D, LAYOUT>;
   hipLaunchKernelGGL(kernel, dim3((uint32_t)groups), dim3(kBlockThreads),
                      lds_reserve_kernel<kernel>(kSplitScoresWavesPerCU), stream, am);

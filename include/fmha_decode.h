@@ -391,11 +391,12 @@ const char* fmha_decode_last_error_detail(void);
  * separated by "; " ("" after a rejected or empty call): each a kernel
  * kind with the choices the library made for it, e.g.
  *   "short(numerics=exact D=128 G=1 layout=packed bucket=16 waves_per_cu=4)"
- *   "split(D=128 G=4 layout=packed sub_units=1 blocks=65 chunk_rows=64
- *    chunks=17 passes=4 launches=2)",
- * whose chunks are the rows of one wave of the P.V launch (the whole row with
- * one workgroup per row) and whose passes count what the launches do: scores,
- * statistics beyond 64 blocks, P.V, the sum over a row's workgroups.
+ *   "split(D=128 G=4 layout=packed sub_units=1 blocks=65 scores_rows=16
+ *    pv_rows=256 pv_rows_least=256 pieces=5 launches=2)",
+ * with the 16-row blocks of the longest row, the rows of a workgroup of the
+ * scores launch and of the P.V launch (and the least that the device may make
+ * of the latter where the lengths are short), and the pieces of that many rows
+ * which the longest row has.
  * Kinds: short, short_multi (several batches per wave), short_matrix_core,
  * onepass, split, split_matrix_core, pad_query_group.  For tests and
  * diagnostics; no counterpart in the reference. */

@@ -60,10 +60,10 @@ def layout_shapes():
 def workspace_traffic(plan, B, hq, hkv, D):
     """Bytes the split-KV passes move through the workspace per call, from the
     plan the library reports: the scores T (written by the scores launch, read
-    by P.V), the max and sum of every 16 rows or more (written; the P.V
-    workgroups' reads of them hit the caches) and, with more than one P.V
-    workgroup of four chunks per row, the fp32 partial outputs (written, and
-    read by the row's last workgroup).  0 for the single pass and the short
+    by P.V), the max and sum of every scores workgroup's rows (written; the
+    P.V workgroups' reads of them hit the caches) and, with more than one P.V
+    workgroup per row, the fp32 partial outputs of each (written, and read by
+    the row's last).  0 for the single pass and the short
     kernels."""
     total = 0
     for entry in plan:
@@ -72,10 +72,10 @@ def workspace_traffic(plan, B, hq, hkv, D):
             continue
         f = dict(kv.split("=") for kv in rest.rstrip(")").split())
         heads = B * max(hq, hkv * int(f["G"]))
-        nblk, groups = int(f["blocks"]), (int(f["chunks"]) + 3) // 4
-        total += 2 * heads * nblk * 16 * 4 + heads * nblk * 8
-        if groups > 1:
-            total += 2 * heads * groups * D * 4
+        rows, pieces = int(f["blocks"]) * 16, int(f["pieces"])
+        total += 2 * heads * rows * 4 + heads * rows // int(f["scores_rows"]) * 8
+        if pieces > 1:
+            total += 2 * heads * pieces * D * 4
     return total
 
 

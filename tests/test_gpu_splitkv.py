@@ -51,51 +51,52 @@ def test_block_boundaries(D, Hq, Hkv):
     _case(len(seqlens), Hq, Hkv, D, seqlens, 64, seed=11 + D)
 
 
-def test_mid_chunk_count():
-    """16 < chunks <= 256 with four query heads per KV head: rows of more
-    P.V waves than one combine group (16), summed in two levels."""
-    rng = np.random.default_rng(12)
-    seqlens = rng.integers(6000, 8193, size=4).astype(np.int32)
-    seqlens[0] = 8192
-    _case(4, 32, 8, 128, seqlens, 8192, seed=12, std=0.5)
-    assert 16 < _launch("split")["chunks"] <= 256
+def test_sums_in_two_levels():
+    """Rows of more than 16 P.V workgroups, whose partial outputs are summed
+    16 at a time and then once more, and of at most 16 in the same call."""
+    seqlens = np.array([8192, 6001, 700], np.int32)
+    _case(3, 8, 8, 128, seqlens, 8192, seed=12, std=0.5)
+    assert _launch("split")["pieces"] > 16
 
 
-def test_mid_block_count():
-    """512 < blocks <= 2048 on one long row: the 256-thread statistics pass."""
-    _case(1, 32, 8, 128, np.array([20000], np.int32), 20000, seed=13, std=0.5)
-    split = _launch("split")
-    assert 512 < split["blocks"] <= 2048 and split["passes"] == 4
+def _entries(launch, max_len):
+    """Entries of a row's statistics, one per scores workgroup."""
+    return (max_len + launch["scores_rows"] - 1) // launch["scores_rows"]
 
 
-# (B, Hq, Hkv, D, max_len, kind, passes): rows of up to 64 blocks, whose P.V
-# waves reduce the block statistics themselves (no statistics pass), and one
-# block more; one chunk per row (O from the P.V pass) or several (combine).
+# (B, Hq, Hkv, D, max_len, kind, statistics entries): the entries that a P.V
+# wave joins for a query head, at and past one load per lane (64), the four
+# that it takes at once on short rows (256), and, with four query heads a wave
+# (groups above 8), the eight of its first round (512); scores workgroups of
+# one wave with one or four blocks for a head, and of the matrix cores.
 STAT_CASES = [
-    (6, 32, 8, 128, 1024, "split", 3),
-    (6, 32, 8, 128, 1040, "split", 4),
-    (256, 32, 8, 128, 1024, "split", 2),
-    (256, 32, 8, 128, 1040, "split", 4),
-    (8, 8, 2, 64, 1000, "split", 3),               # lane groups on several chunks
-    (8, 64, 4, 128, 1024, "split_matrix_core", 3),
-    (8, 64, 4, 128, 1040, "split_matrix_core", 4),
-    (512, 64, 4, 256, 700, "split_matrix_core", 2),
+    (6, 32, 8, 128, 1024, "split", 64),
+    (6, 32, 8, 128, 1040, "split", 65),
+    (256, 32, 8, 128, 1024, "split", 64),
+    (256, 32, 8, 128, 1040, "split", 65),
+    (2, 8, 8, 128, 4096, "split", 256),
+    (2, 8, 8, 128, 4097, "split", 257),
+    (8, 8, 2, 64, 1000, "split", 16),               # lane groups on several blocks
+    (8, 64, 4, 128, 1024, "split_matrix_core", 16),
+    (8, 64, 4, 128, 1040, "split_matrix_core", 17),
+    (512, 64, 4, 256, 700, "split_matrix_core", 22),
+    (1, 32, 1, 128, 32768, "split_matrix_core", 512),
+    (1, 32, 1, 128, 33000, "split_matrix_core", 516),
 ]
 
 
-@pytest.mark.parametrize("B,Hq,Hkv,D,max_len,kind,passes", STAT_CASES)
-def test_block_statistics_in_pv(monkeypatch, B, Hq, Hkv, D, max_len, kind, passes):
-    """The P.V waves' own reduction of the block statistics, at and past its
-    64-block limit, with ragged lengths (0, 1, one block, the maximum); the
-    matrix-core single passes off (FMHA_DECODE_ONEPASS_MFMA=0,
-    FMHA_DECODE_ONEPASS_REG=0)."""
+@pytest.mark.parametrize("B,Hq,Hkv,D,max_len,kind,entries", STAT_CASES)
+def test_block_statistics_in_pv(monkeypatch, B, Hq, Hkv, D, max_len, kind, entries):
+    """The P.V workgroups' joining of a row's statistics, with ragged lengths
+    (0, 1, one block, the maximum); the matrix-core single passes off
+    (FMHA_DECODE_ONEPASS_MFMA=0, FMHA_DECODE_ONEPASS_REG=0)."""
     monkeypatch.setenv("FMHA_DECODE_ONEPASS_MFMA", "0")
     monkeypatch.setenv("FMHA_DECODE_ONEPASS_REG", "0")
     rng = np.random.default_rng(B + max_len + Hq)
     seqlens = rng.integers(0, max_len + 1, size=B).astype(np.int32)
-    seqlens[:4] = [max_len, 0, 1, 16]
+    seqlens[:4] = [max_len, 0, 1, 16][:B]
     _case(B, Hq, Hkv, D, seqlens, max_len, seed=B * 7 + D + Hq, std=0.5)
-    assert _launch(kind)["passes"] == passes
+    assert _entries(_launch(kind), max_len) == entries
 
 
 @pytest.mark.parametrize("max_len", [16, 5])
@@ -114,19 +115,18 @@ def test_short_lengths_match_short_path(max_len):
 
 
 def test_many_batches_direct_path():
-    """max length fits one chunk: the PV kernel writes O directly."""
+    """One P.V workgroup of one wave per row, which writes O itself."""
     seqlens = np.random.default_rng(3).integers(0, 41, size=200).astype(np.int32)
     _case(200, 8, 8, 128, seqlens, 40, seed=6)
-    split = _launch("split")
-    assert split["chunks"] == 1 and split["passes"] == 2
+    assert _launch("split")["pieces"] == 1
 
 
 def test_one_long_sequence():
-    """More than 256 chunks (the 1024-thread combine), more than 2048 blocks
-    (the 1024-thread statistics)."""
+    """More than 2048 blocks: scores workgroups of four waves, and sums of
+    partial outputs in two levels."""
     _case(1, 32, 8, 128, np.array([40000], np.int32), 40000, seed=7, std=0.5)
     split = _launch("split")
-    assert split["chunks"] > 256 and split["blocks"] > 2048 and split["passes"] == 4
+    assert split["scores_rows"] == 64 and split["pieces"] > 16
 
 
 # (B, Hq, Hkv, D, max_len): fewer (batch, KV-head group) units than the

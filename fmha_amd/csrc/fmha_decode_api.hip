@@ -525,81 +525,39 @@ constexpr size_t kWorkspaceAlign = 256;
 size_t align_up(size_t x) { return (x + kWorkspaceAlign - 1) / kWorkspaceAlign * kWorkspaceAlign; }
 
 struct SplitPlan {
-  int nblk = 1;      // 16-row blocks of a row
-  int pv_shift = 8;  // log2 of the rows of a P.V workgroup
-  int pv_fine = 8;   // the least the device may make it
-  int pv_few = 1, pv_many = 1, pv_big = 12;  // SplitArgs
-  int npv = 1;       // P.V workgroups of a row, at most
+  int nblk = 1;  // 16-row blocks of a row
+  fmha_decode::PvPieces pv{};
   int64_t units = 0;
   size_t off_t = 0, off_st = 0, off_done = 0, off_opart = 0, total = 0;
 };
 
-// The split passes' workspace and the rows of a P.V workgroup: the largest
-// of 256 to 4096 that leaves kPvMinGroups workgroups, about two for each CU
-// (all of them at once: µs of the call at 2048 / 4096 rows, 32/8 B=8 S=32768
-// 194.4 / 192.3, 64/8 218.6 / 207.0; more, shorter ones pay a workgroup's 8
-// us of start and end again: B=1 S=131072, P.V alone, 71 / 59 / 54 at 512 /
-// 1024 / 2048), and divides rows of more than 1024.  Where the lengths turn
-// out to leave fewer than kPvFewGroups (from 4096 rows, 1024 at D = 256, on
-// kPvMinGroups) the device makes it up to four times smaller (row_piece; µs
-// of ragged calls by rows, their workgroups in brackets: B=48 8/1 over
-// 250-8000 rows 26.9 (420) / 25.1 (210) / 26.6 (105) at 256 / 512 / 1024;
-// B=6 64/8 over 1024-32768 64.9 (430) / 63.3 (215) / 73.4 (107) at 1024 /
-// 2048 / 4096; D=64 B=22 8/8 over 666-21321 65.3 (512) / 71.5 (256) at 2048 /
-// 4096; D=256 B=10 8/8 over 360-11516 65.8 (504) / 69.6 (252) at 512 / 1024).
-// Not a size that leaves the last of two or three pieces of a row mostly
-// empty (D=64 B=57 8/8 S=2233: 72.1 at 2048 rows, 59.9 at 1024). 
-constexpr int64_t kPvMinGroups = 448, kPvFewGroups = 192;
-constexpr int kPvMinShift = 8, kPvMaxShift = 12;
-
+// The split passes' workspace and the pieces of the P.V launch.
 SplitPlan plan_split(int64_t batch, int hq, int hkv, int max_rows, int d) {
   SplitPlan p;
   const int heads_per_wave = kWaveSize / (d / 8);
   p.units = (hkv + heads_per_wave - 1) / heads_per_wave * batch;
-  const auto groups = [&](int shift) { return max_rows <= 0 ? 1 : ((int64_t)max_rows + (1 << shift) - 1) >> shift; };
-  p.pv_shift = kPvMaxShift;
-  const auto fits = [&](int shift) {
-    const int64_t n = groups(shift), all = batch * hkv * n;
-    if (max_rows > 1024 && n < 2) return false;
-    if (n > 1 && n < 4 && (int64_t)max_rows * 10 < 7 * (n << shift)) return false;
-    return all >= kPvMinGroups;
-  };
-  while (p.pv_shift > kPvMinShift && !fits(p.pv_shift)) --p.pv_shift;
   // FMHA_DECODE_SPLIT_CHUNK=<128|...|4096>: rows of a P.V workgroup instead
   // (for sweeps; the workspace size follows, and a launch checks its
   // workspace against it).
-  bool forced = false;
+  int forced = 0;
   if (const char* e = std::getenv("FMHA_DECODE_SPLIT_CHUNK")) {
     const int v = std::atoi(e);
-    forced = v >= 128 && v <= 4096 && (v & (v - 1)) == 0;
-    if (forced) p.pv_shift = fmha_decode::ilog2(v);
+    if (v >= 128 && v <= 4096 && (v & (v - 1)) == 0) forced = v;
   }
-  const bool adapts = !forced && batch <= fmha_decode::kOrderBatches;
-  p.pv_fine = !adapts || p.pv_shift <= kPvMinShift ? p.pv_shift
-              : p.pv_shift - 2 > kPvMinShift       ? p.pv_shift - 2
-                                                   : kPvMinShift;
-  p.pv_few = (int)((kPvFewGroups + hkv - 1) / hkv);
-  p.pv_many = (int)((kPvMinGroups + hkv - 1) / hkv);
-  p.pv_big = d == 256 ? 10 : 12;
-  p.npv = (int)groups(p.pv_fine);
+  p.pv = fmha_decode::plan_pv_pieces(batch, hkv, max_rows, d, forced);
   p.nblk = max_rows <= 0 ? 1 : (max_rows + fmha_decode::kSplitBlockRows - 1) / fmha_decode::kSplitBlockRows;
   const size_t heads = (size_t)batch * hq;
-  const size_t fans = (size_t)(p.npv + fmha_decode::kPvFan - 1) / fmha_decode::kPvFan;
+  const size_t fans = (size_t)(p.pv.npv + fmha_decode::kPvFan - 1) / fmha_decode::kPvFan;
   size_t off = 0;
   p.off_t = off;
   off += align_up(heads * (size_t)p.nblk * fmha_decode::kSplitBlockRows * 4);
   p.off_st = off;
   off += align_up(heads * (size_t)p.nblk * 8);
-  if (p.npv > 1) {
+  if (p.pv.npv > 1) {
     p.off_done = off;
-    off += align_up((size_t)batch * hkv * (1 + fans) * 4);
-    // Partial outputs of every piece: those of pv_shift rows, or the shorter
-    // ones the device takes, less than twice pv_many and one per batch.
-    const int64_t coarse = batch * groups(p.pv_shift), fine = batch * groups(p.pv_fine);
-    const int64_t few = 2 * (int64_t)p.pv_many + batch;
-    const int64_t pieces = coarse > few ? coarse : (fine < few ? fine : few);
+    off += align_up((size_t)batch * hkv * p.pv.parts * (1 + fans) * 4);
     p.off_opart = off;
-    off += align_up((size_t)pieces * hq * d * 4);
+    off += align_up((size_t)p.pv.total * hq * d * 4);
   }
   p.total = off;
   return p;
@@ -905,7 +863,7 @@ int split_prepare(const void* Q, const void* K, const void* V, void* O, int32_t 
                   float softmax_scale, void* workspace, size_t workspace_bytes, int64_t kv_span_bytes, SplitArgs& a) {
   const SplitPlan plan = plan_split(batch, num_heads_q, num_heads_kv, max_seqlen_kv, head_dim);
   const int64_t padded_rows = (int64_t)plan.nblk * fmha_decode::kSplitBlockRows;
-  const int64_t part_bytes = (int64_t)num_heads_q * plan.npv * head_dim * 4;  // one batch's partials
+  const int64_t part_bytes = (int64_t)num_heads_q * plan.pv.npv * head_dim * 4;  // one batch's partials
   if (kv_span_bytes >= (int64_t(1) << 30) || padded_rows * num_heads_q * 4 >= (int64_t(1) << 30) ||
       part_bytes >= (int64_t(1) << 30))
     return reject(FMHA_DECODE_ERROR_INVALID_VALUE, "max_seqlen_kv too large for this head count (%d)", max_seqlen_kv);
@@ -932,12 +890,7 @@ int split_prepare(const void* Q, const void* K, const void* V, void* O, int32_t 
   a.kv_groups = kv_groups;
   a.units_per_batch = (int32_t)(plan.units / batch);
   a.nblk = plan.nblk;
-  a.npv = plan.npv;
-  a.pv_shift = plan.pv_shift;
-  a.pv_fine = plan.pv_fine;
-  a.pv_few = plan.pv_few;
-  a.pv_many = plan.pv_many;
-  a.pv_big = plan.pv_big;
+  a.pv = plan.pv;
   a.max_rows = max_seqlen_kv;
   a.batch = batch;
   a.scale = softmax_scale;

@@ -477,32 +477,40 @@ hipError_t launch_onepass_group(const SplitArgs& a, hipStream_t stream) {
 // The two launches of split-KV for the plan text: the rows of a scores
 // workgroup (each leaves one entry of the row's statistics), the rows of a P.V
 // workgroup (a piece) as planned and at least (the device may take shorter
-// ones), and the pieces of the longest row as planned.
-#define FMHA_DECODE_SPLIT_PLAN "scores_rows=%d pv_rows=%d pv_rows_least=%d pieces=%d launches=2"
-inline int split_pieces(const SplitArgs& a) { return (a.max_rows + (1 << a.pv_shift) - 1) >> a.pv_shift; }
+// ones), the pieces of the longest row as planned, and the workgroups that
+// share a piece's dims.
+#define FMHA_DECODE_SPLIT_PLAN "scores_rows=%d pv_rows=%d pv_rows_least=%d pieces=%d pv_parts=%d launches=2"
+inline int split_pieces(const SplitArgs& a) { return (a.max_rows + (1 << a.pv.shift) - 1) >> a.pv.shift; }
 
 // The P.V launch of split-KV (splitkv_pv_kernel) after the scores launch of
 // either kind; instantiated in its own parts, which the others link to.
-template <int D, int LAYOUT>
-hipError_t launch_split_pv(const SplitArgs& a, hipStream_t stream) {
+template <int D, int LAYOUT, int PARTS>
+hipError_t launch_split_pv_parts(const SplitArgs& a, hipStream_t stream) {
   const int g = a.num_heads_q / a.num_heads_kv;
-  const int64_t tiles = (g + 15) / 16;
-  const int64_t units = (int64_t)a.batch * a.npv * a.num_heads_kv;
-  const int64_t groups = (units + 7) / 8 * 8 * tiles;
+  const int64_t subs = (int64_t)(g + 15) / 16 * PARTS;
+  const int64_t units = a.pv.total * a.num_heads_kv;
+  const int64_t groups = (units + 7) / 8 * 8 * subs;
   if (groups > INT32_MAX) return hipErrorInvalidValue;
   const dim3 grid((uint32_t)groups);
   const dim3 block(a.max_rows <= fmha_decode::kPvOneWaveRows ? kBlockThreads : fmha_decode::kPvThreads);
   if (g <= 1)
-    hipLaunchKernelGGL((fmha_decode::splitkv_pv_kernel<D, 1, LAYOUT>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((fmha_decode::splitkv_pv_kernel<D, 1, LAYOUT, PARTS>), grid, block, 0, stream, a);
   else if (g <= 2)
-    hipLaunchKernelGGL((fmha_decode::splitkv_pv_kernel<D, 2, LAYOUT>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((fmha_decode::splitkv_pv_kernel<D, 2, LAYOUT, PARTS>), grid, block, 0, stream, a);
   else if (g <= 4)
-    hipLaunchKernelGGL((fmha_decode::splitkv_pv_kernel<D, 4, LAYOUT>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((fmha_decode::splitkv_pv_kernel<D, 4, LAYOUT, PARTS>), grid, block, 0, stream, a);
   else if (g <= 8)
-    hipLaunchKernelGGL((fmha_decode::splitkv_pv_kernel<D, 8, LAYOUT>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((fmha_decode::splitkv_pv_kernel<D, 8, LAYOUT, PARTS>), grid, block, 0, stream, a);
   else
-    hipLaunchKernelGGL((fmha_decode::splitkv_pv_kernel<D, 16, LAYOUT>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((fmha_decode::splitkv_pv_kernel<D, 16, LAYOUT, PARTS>), grid, block, 0, stream, a);
   return hipGetLastError();
+}
+
+template <int D, int LAYOUT>
+hipError_t launch_split_pv(const SplitArgs& a, hipStream_t stream) {
+  if constexpr (D == 256)
+    if (a.pv.parts == 2) return launch_split_pv_parts<D, LAYOUT, 2>(a, stream);
+  return launch_split_pv_parts<D, LAYOUT, 1>(a, stream);
 }
 
 #ifndef FMHA_DECODE_INSTANTIATING_PV
@@ -935,7 +943,7 @@ hipError_t launch_split_dg(const SplitArgs& a, hipStream_t stream, bool onepass_
   const int64_t groups = (int64_t)a.batch * as.nsup * as.units_per_batch;
   if (groups > INT32_MAX) return hipErrorInvalidValue;
   plan_note("split(D=%d G=%d layout=%s sub_units=%d blocks=%d " FMHA_DECODE_SPLIT_PLAN ")", D, G, layout_name(LAYOUT),
-            1 << shift, a.nblk, 1 << as.sup_shift, 1 << a.pv_shift, 1 << a.pv_fine, split_pieces(a));
+            1 << shift, a.nblk, 1 << as.sup_shift, 1 << a.pv.shift, 1 << a.pv.fine, split_pieces(a), a.pv.parts);
   constexpr auto kernel = fmha_decode::splitkv_scores_kernel<D, G, LAYOUT>;
   hipLaunchKernelGGL(kernel, dim3((uint32_t)groups), dim3(kBlockThreads * wpg),
                      lds_reserve_kernel<kernel>(kSplitScoresWavesPerCU / wpg), stream, as);
@@ -980,8 +988,8 @@ hipError_t launch_split_group_d(const SplitArgs& a, hipStream_t stream) {
   const int64_t groups = (int64_t)a.batch * am.nsup * a.num_heads_kv;
   if (groups > INT32_MAX) return hipErrorInvalidValue;
   plan_note("split_matrix_core(D=%d G=%d layout=%s blocks=%d " FMHA_DECODE_SPLIT_PLAN ")", D,
-            a.num_heads_q / a.num_heads_kv, layout_name(LAYOUT), a.nblk, 1 << am.sup_shift, 1 << a.pv_shift,
-            1 << a.pv_fine, split_pieces(a));
+            a.num_heads_q / a.num_heads_kv, layout_name(LAYOUT), a.nblk, 1 << am.sup_shift, 1 << a.pv.shift,
+            1 << a.pv.fine, split_pieces(a), a.pv.parts);
   constexpr auto kernel = fmha_decode::splitkv_scores_group_kernel<D, LAYOUT>;
   hipLaunchKernelGGL(kernel, dim3((uint32_t)groups), dim3(kBlockThreads),
                      lds_reserve_kernel<kernel>(kSplitScoresWavesPerCU), stream, am);

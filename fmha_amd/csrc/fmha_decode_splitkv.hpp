@@ -40,6 +40,7 @@
 #include <type_traits>
 
 #include "fmha_decode_kernel.hpp"
+#include "fmha_decode_pieces.hpp"
 
 namespace fmha_decode {
 
@@ -62,17 +63,12 @@ struct SplitArgs {
   float* t;               // [batch, nblk, Hq, 16] scaled scores
   f32x2_v* st;            // [batch, Hq, nsup] max and sum of exp(t - max) of nsup-th parts of a row
   float* opart;           // [P.V pieces, Hkv, G, D] partial outputs
-  uint32_t* done;         // [batch, Hkv, tiles, 1 + ceil(npv / kPvFan)] finished P.V workgroups
+  uint32_t* done;         // [batch, Hkv, tiles, pv.parts, 1 + ceil(pv.npv / kPvFan)] finished P.V workgroups
   int32_t num_heads_q;
   int32_t num_heads_kv;
   int32_t units_per_batch;  // KV-head groups per batch: ceil(Hkv / HPW)
   int32_t nblk;           // 16-row blocks per batch row: ceil(max_rows / 16)
-  int32_t npv;            // P.V workgroups of the longest row, at most: ceil(max_rows / 2^pv_fine)
-  int32_t pv_shift;       // log2 of the rows of a P.V workgroup
-  int32_t pv_fine;        // the least it may be made on the device (row_piece)
-  int32_t pv_few;         // per KV head, the workgroups below which it is,
-  int32_t pv_many;        // and those below which it is from pv_big on
-  int32_t pv_big;
+  PvPieces pv;            // pieces of the P.V launch
   int32_t sup_shift;      // log2 of the rows of a scores workgroup
   int32_t nsup;           // scores workgroups per batch row: ceil(max_rows / 2^sup_shift)
   int32_t max_rows;       // lengths above this are invalid (NaN output)
@@ -140,7 +136,6 @@ constexpr int kSplitBlockRows = kMaxSeq;  // rows per scores wave
 // The lengths of all of a call's batches (at most kOrderBatches), batch p *
 // kWaveSize + lane in len[p]; 0 past the last.  Every load is requested at
 // once, with no branch between them.
-constexpr int kOrderBatches = 256;
 constexpr int kOrderRegs = kOrderBatches / kWaveSize;
 
 template <int LAYOUT>
@@ -228,47 +223,38 @@ __device__ __forceinline__ int wave_scan(int x) {
   return x;
 }
 
-// The P.V workgroups' pieces: piece u of a call whose batches have max(1,
-// ceil(S / 2^shift)) each (one for an empty or invalid batch), in batch order;
-// false past the last.  Up to kOrderBatches batches the wave adds up the
-// pieces of the lengths, so that the workgroups past the rows that exist are
-// the last of the grid, and takes shorter pieces than the host, which saw
-// only the longest row allowed, where they would leave CUs without one (µs,
-// B=30 8/8 over 140-4500 rows 45.3 with the host's 2048 rows, 37.1 with the
-// 1024 taken; plan_split has the limits); above, and with one length for all, as batch_piece.
-// Every lane of every wave of a workgroup calls it.
+// The P.V workgroups' pieces: piece u of a call whose batches have
+// pv_row_pieces each, in batch order; false past the last.  Up to
+// kOrderBatches batches the wave adds up the lengths, so that the workgroups
+// past the rows that exist are the last of the grid, and takes shorter pieces
+// than the host, which saw only the longest row allowed, where they would
+// leave CUs without one (pv_device_shift; µs, B=30 8/8 over 140-4500 rows 45.3
+// with the host's 2048 rows, 37.1 with the 1024 taken); above, and with one
+// length for all, as batch_piece.  Every lane of every wave of a workgroup
+// calls it.
 template <int LAYOUT>
 __device__ __forceinline__ bool row_piece(const SplitArgs& a, uint32_t u, int lane, RowPiece& out) {
-  const auto finer = [&](int rows) {
-    int s = a.pv_shift;
-    while (s > a.pv_fine && (rows >> s) < (s >= a.pv_big ? a.pv_many : a.pv_few)) --s;
-    return s;
-  };
   if (a.len_mode == kLenUniform || a.batch > kOrderBatches)
-    return batch_piece<LAYOUT>(a, u, a.pv_shift, ((uint32_t)a.max_rows + (1u << a.pv_shift) - 1) >> a.pv_shift, out);
+    return batch_piece<LAYOUT>(a, u, a.pv.shift, (uint32_t)pv_row_pieces(a.max_rows, a.max_rows, a.pv.shift), out);
   if (a.batch == 1) {
     out.b = 0;
     out.piece = u;
     out.S = split_len_l<LAYOUT>(a, 0);
-    const bool valid = out.S > 0 && out.S <= a.max_rows;
-    out.shift = finer(valid ? out.S : 0);
-    return u == 0 || (valid && (int)(u << out.shift) < out.S);
+    out.shift = pv_device_shift(a.pv, pv_counted_rows(out.S, a.max_rows));
+    return u < (uint32_t)pv_row_pieces(out.S, a.max_rows, out.shift);
   }
   int len[kOrderRegs];
   batch_lengths<LAYOUT>(a, lane, len);
-  // All valid rows (a row's part capped: the sum stays below 2^31).
   int rows = 0;
 #pragma unroll
-  for (int p = 0; p < kOrderRegs; ++p) rows += len[p] <= 0 || len[p] > a.max_rows ? 0 : min(len[p], 1 << 22);
-  out.shift = finer(__builtin_amdgcn_readlane(wave_scan(rows), kWaveSize - 1));
-  const int round = (1 << out.shift) - 1;
+  for (int p = 0; p < kOrderRegs; ++p) rows += pv_counted_rows(len[p], a.max_rows);
+  out.shift = pv_device_shift(a.pv, __builtin_amdgcn_readlane(wave_scan(rows), kWaveSize - 1));
   uint32_t before = 0;  // pieces of the batches of earlier p
 #pragma unroll
   for (int p = 0; p < kOrderRegs; ++p) {
     if (p * kWaveSize >= a.batch) break;
-    const int x = wave_scan(p * kWaveSize + lane >= a.batch      ? 0
-                            : len[p] <= 0 || len[p] > a.max_rows ? 1
-                                                                 : (len[p] + round) >> out.shift);
+    const int x =
+        wave_scan(p * kWaveSize + lane >= a.batch ? 0 : pv_row_pieces(len[p], a.max_rows, out.shift));
     const uint32_t total = (uint32_t)__builtin_amdgcn_readlane(x, kWaveSize - 1);
     if (u < before + total) {
       const int l = __popcll(__builtin_amdgcn_ballot_w64(before + (uint32_t)x <= u));
@@ -615,10 +601,11 @@ constexpr int kScoresMaxWaves = 4;
 constexpr int kScoresLongBlocks = 2048;
 
 // Zeroes the P.V arrival counts of `heads` KV heads from hk0 on of batch b,
-// `tiles` query tiles each (the workgroups of the P.V launch count from it).
-__device__ __forceinline__ void clear_done(const SplitArgs& a, uint32_t b, uint32_t hk0, int heads, int tiles) {
-  if (a.npv == 1) return;
-  const uint32_t per = (uint32_t)(tiles * (1 + (a.npv + kPvFan - 1) / kPvFan));
+// `subs` (query tiles times parts of the dims) each; the workgroups of the P.V
+// launch count from it.
+__device__ __forceinline__ void clear_done(const SplitArgs& a, uint32_t b, uint32_t hk0, int heads, int subs) {
+  if (a.pv.npv == 1) return;
+  const uint32_t per = (uint32_t)(subs * (1 + (a.pv.npv + kPvFan - 1) / kPvFan));
   const uint32_t n = min((uint32_t)heads, (uint32_t)a.num_heads_kv - min(hk0, (uint32_t)a.num_heads_kv)) * per;
   uint32_t* done = a.done + ((uint64_t)b * a.num_heads_kv + hk0) * per;
   for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) done[i] = 0u;
@@ -651,7 +638,7 @@ __global__ __launch_bounds__(kBlockThreads * kScoresMaxWaves) void splitkv_score
   const int S = rp.S;
   // Ahead of clear_done's stores, behind which it is a vector load.
   const int64_t row_base = split_row_base<LAYOUT>(a, b);
-  if (rp.piece == 0) clear_done(a, b, hg * su.heads(), su.heads(), 1);
+  if (rp.piece == 0) clear_done(a, b, hg * su.heads(), su.heads(), a.pv.parts);
   if (S <= 0 || S > a.max_rows) return;
   const uint32_t wb = (rp.piece << (a.sup_shift - a.sub_shift - ilog2(NR))) + (uint32_t)wv;
   const int j0 = (int)(wb << a.sub_shift) * NR;  // the wave's first row

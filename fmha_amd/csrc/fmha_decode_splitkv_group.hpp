@@ -65,7 +65,7 @@ __global__ __launch_bounds__(kBlockThreads) void splitkv_scores_group_kernel(Spl
   const int G = hq / (int)hkv;
   const int tiles = (G + 15) / 16;
   const int64_t row_base = split_row_base<LAYOUT>(a, b);  // ahead of clear_done's stores (splitkv_scores_kernel)
-  if (rp.piece == 0) clear_done(a, b, hk, 1, tiles);
+  if (rp.piece == 0) clear_done(a, b, hk, 1, tiles * a.pv.parts);
   if (S <= 0 || S > a.max_rows) return;
   const int j0 = (int)(rp.piece << a.sup_shift);  // the wave's first row
   const int s = lane / LPH;  // this lane group's block of the wave

@@ -3,9 +3,9 @@
 // row's workgroups, gfx950.
 //
 // A workgroup of kPvWaves waves takes 2^shift V rows (row_piece) of one (batch, KV
-// head) for up to 16 of its query heads (a tile; larger groups take several
-// workgroups, placed on one XCD so that V comes from its L2 after the
-// first):
+// head) for up to 16 of its query heads (a tile), all of its dims or half of
+// them (PARTS = 2); larger groups and halves take several workgroups, placed
+// on one XCD so that V or the scores come from its L2 after the first:
 //   * its waves request their first scores T and V tiles, then join the
 //     statistics that the scores launch left per part of the row into each
 //     query head's max and sum;
@@ -13,11 +13,11 @@
 //     the group's 16 * GT * GC weights bf16(exp(t - max) / sum), GC >= G
 //     query columns, are formed one per lane and step (the matrix cores'
 //     own layout would have every lane form 4 per tile, 16 / G times too
-//     many) and pass through LDS into the A operand of D/16
+//     many) and pass through LDS into the A operand of DV/16 (DV: the
+//     workgroup's dims)
 //     v_mfma_f32_16x16x16_bf16 per tile; V comes straight from memory in the
-//     B operand's rows (lane (q, n): rows 4q..4q+3 at the D/16 dims of
-//     out_dim(n, ...)), transposed in registers with v_perm, GT tiles in
-//     flight;
+//     B operand's rows (lane (q, n): rows 4q..4q+3 at dims [n DV/16,
+//     +DV/16)), transposed in registers with v_perm, GT tiles in flight;
 //   * the waves' fp32 sums are added in wave order through LDS and written
 //     as fp16 O by a row's only workgroup, else as fp32 partial outputs, of
 //     which the last workgroup to finish of each kPvFan neighbours adds
@@ -58,28 +58,29 @@ constexpr int kPvGroupTiles = 2;
 
 // LDS bytes: the waves' weights of a tile group, then (reusing them) their
 // sums.
-template <int D, int GC>
+template <int DV, int GC>
 constexpr int pv_lds_bytes() {
   constexpr int weights = kPvWaves * kPvGroupTiles * GC * kSplitBlockRows * 2;
-  constexpr int sums = kPvWaves * GC * D * 4;
+  constexpr int sums = kPvWaves * GC * DV * 4;
   return weights > sums ? weights : sums;
 }
 
-// One wave's V tiles (16 rows of one (batch, KV head) each) in the B
-// operand's rows: lane (q, n) gets rows 4q..4q+3 at dims out_dim(n, 0..DPC-1),
-// so that each load instruction reads whole lines of a row (µs of the call
-// at D = 256, 16 neighbouring dims per lane / this: 28/4 B=3 S=66558 on 64-row
-// pages 197 / 179, packed 64/8 B=16 S=4096 106 / 101).  Tiles are step_tiles apart from row `first` on; rows at or past
+// One wave's V tiles (16 rows of one (batch, KV head) each, the workgroup's
+// dims) in the B operand's rows: lane (q, n) gets rows 4q..4q+3 at dims
+// out_dim(n, 0..DPC-1), so that each load instruction reads whole lines of a
+// row (µs of the call at D = 256, 16 neighbouring dims per lane / this: 28/4
+// B=3 S=66558 on 64-row pages 197 / 179, packed 64/8 B=16 S=4096 106 / 101).
+// Tiles are step_tiles apart from row `first` on; rows at or past
 // `end` read 0, without memory access (on pages under 16 rows from Q's first
 // row).  Paged: an unmapped page (a negative entry) reads as 0 too; the
 // scores launch has made the batch's statistics NaN then.
-template <int D, int LAYOUT>
+template <int D, int LAYOUT, int PARTS>
 struct VTiles {
   static constexpr bool PAGED = LAYOUT == kLayoutPagedBlock;    // a tile lies in one page
   static constexpr bool PAGED_ROWS = LAYOUT == kLayoutPaged;    // every row through its own entry
-  static constexpr int DPC = D / 16;
-  static constexpr int VW = DPC / 2;                 // dwords of a lane's dims of a row
-  static constexpr int RUN = out_dim<DPC>(0, 8);     // dims from a lane's first 16 bytes of a row to its next
+  static constexpr int DPC = D / PARTS / 16;
+  static constexpr int VW = DPC / 2;              // dwords of a lane's dims of a row
+  static constexpr int RUN = out_dim<DPC>(0, 8);  // dims from a lane's first 16 bytes of a row to its next
   __amdgpu_buffer_rsrc_t rsrc;  // packed, strided: the batch's rows
   const uint16_t* v;
   const uint16_t* safe;
@@ -89,7 +90,7 @@ struct VTiles {
   int first, end, step, q;
   int32_t tile_entry;  // PAGED: lane k holds the entry of the wave's tile k (64 at most)
 
-  __device__ __forceinline__ void init(const SplitArgs& a, uint32_t b, int hk, int S, int first_, int end_,
+  __device__ __forceinline__ void init(const SplitArgs& a, uint32_t b, int hk, int part, int S, int first_, int end_,
                                        int step_tiles, int lane) {
     uint32_t head_off;
     first = first_;
@@ -115,7 +116,7 @@ struct VTiles {
       row_bytes = rows.row_bytes;
       head_off = rows.lane_off;
     }
-    lane_off = head_off + (uint32_t)out_dim<DPC>(lane & 15, 0) * 2u + (PAGED_ROWS ? 0u : 4u * (uint32_t)q * row_bytes);
+    lane_off = head_off + (uint32_t)(part * (D / PARTS) + out_dim<DPC>(lane & 15, 0)) * 2u + (PAGED_ROWS ? 0u : 4u * (uint32_t)q * row_bytes);
   }
 
   // PAGED_ROWS: the block-table entries of this lane's rows of tile k, to be
@@ -245,23 +246,23 @@ __device__ __forceinline__ f32x2_v sum_partials(const float* p, int n, size_t st
   return s;
 }
 
-// Grid: units = pieces (row_piece) * Hkv, unit u * Hkv +
-// hk, each with `tiles` = ceil(G / 16) query tiles; ceil(units / 8) * 8 *
-// tiles workgroups, workgroup w serving unit ((w / 8) / tiles) * 8 + w % 8
-// and tile (w / 8) % tiles, so that the tiles of one unit run on one XCD
-// (dispatch is round-robin over the 8 XCDs).  GC: query columns formed, at
-// least min(G, 16).
-template <int D, int GC, int LAYOUT>
+// Grid: units = pieces (row_piece) * Hkv, unit u * Hkv + hk, each with `subs`
+// workgroups: ceil(G / 16) query tiles times PARTS parts of the dims; ceil(units / 8) * 8 * subs workgroups, workgroup w serving
+// unit ((w / 8) / subs) * 8 + w % 8 and tile and part (w / 8) % subs, so that
+// one unit's run on one XCD (dispatch is round-robin over the 8 XCDs).  GC:
+// query columns formed, at least min(G, 16).
+template <int D, int GC, int LAYOUT, int PARTS>
 __global__ __launch_bounds__(kPvThreads) void splitkv_pv_kernel(SplitArgs a) {
-  using VT = VTiles<D, LAYOUT>;
+  using VT = VTiles<D, LAYOUT, PARTS>;
   constexpr int NR = kSplitBlockRows;
   constexpr int DPC = VT::DPC;
+  constexpr int DV = D / PARTS;  // the workgroup's dims
   constexpr int GT = kPvGroupTiles;
   constexpr int SLOTS = GT * NR * GC;                                 // weights of a tile group
   constexpr int PL = (SLOTS + kWaveSize - 1) / kWaveSize;             // per lane
   constexpr int ND = GC >= 4 ? GC / 4 : 1;                            // query columns a lane's slots cover
   static_assert(GC == 1 || GC == 2 || GC == 4 || GC == 8 || GC == 16, "query columns");
-  __shared__ __attribute__((aligned(16))) char lds[pv_lds_bytes<D, GC>()];
+  __shared__ __attribute__((aligned(16))) char lds[pv_lds_bytes<DV, GC>()];
   __shared__ f32x2_v heads[GC];  // (max, sum) per query column
   __shared__ uint32_t flag;
   const int lane = threadIdx.x & (kWaveSize - 1);
@@ -271,7 +272,8 @@ __global__ __launch_bounds__(kPvThreads) void splitkv_pv_kernel(SplitArgs a) {
   const int hq = a.num_heads_q;
   const int G = hq / (int)hkv;
   const uint32_t tiles = (uint32_t)(G + 15) / 16;
-  const uint32_t rest = blockIdx.x >> 3;
+  const uint32_t part = (blockIdx.x >> 3) % (uint32_t)PARTS;
+  const uint32_t rest = (blockIdx.x >> 3) / (uint32_t)PARTS;
   const uint32_t qt = tiles == 1 ? 0 : rest % tiles;
   const uint32_t unit = (tiles == 1 ? rest : rest / tiles) * 8u + (blockIdx.x & 7u);
   const uint32_t u = unit / hkv;
@@ -282,11 +284,13 @@ __global__ __launch_bounds__(kPvThreads) void splitkv_pv_kernel(SplitArgs a) {
   const int S = rp.S;
   const int gn = G - (int)qt * 16 < GC ? G - (int)qt * 16 : GC;  // query heads of this tile
   const uint64_t head0 = (uint64_t)b * hq + (uint64_t)hk * G + qt * 16;
-  const __amdgpu_buffer_rsrc_t o_rsrc = make_rsrc(a.o + head0 * D, (uint32_t)gn * D * 2u);
+  // The workgroup's dims of its query heads' outputs, D apart.
+  const __amdgpu_buffer_rsrc_t o_rsrc = make_rsrc(a.o + head0 * D + part * DV, (uint32_t)((gn - 1) * D + DV) * 2u);
   if (S <= 0 || S > a.max_rows) {
     // Empty rows give 0 (the reference loop's result), invalid ones NaN.
     const u32x4 fill = S == 0 ? u32x4{0u, 0u, 0u, 0u} : u32x4{0x7e007e00u, 0x7e007e00u, 0x7e007e00u, 0x7e007e00u};
-    for (int i = (int)threadIdx.x; i < gn * (D / 8); i += (int)blockDim.x) buffer_store16(o_rsrc, (uint32_t)i * 16u, fill);
+    for (int i = (int)threadIdx.x; i < gn * (DV / 8); i += (int)blockDim.x)
+      buffer_store16(o_rsrc, (uint32_t)(i / (DV / 8) * D + i % (DV / 8) * 8) * 2u, fill);
     return;
   }
   const int row0 = (int)rp.piece << rp.shift;
@@ -319,7 +323,7 @@ __global__ __launch_bounds__(kPvThreads) void splitkv_pv_kernel(SplitArgs a) {
                              t_off + (uint32_t)(i % ND) * (4 * NR * 4) + (uint32_t)(k * GT + slot_tile(i)) * t_tile);
   };
   VT vt;
-  vt.init(a, b, (int)hk, S, first, end, nw, lane);
+  vt.init(a, b, (int)hk, (int)part, S, first, end, nw, lane);
   uint32_t vr[GT][4][VT::VW];
   int32_t ev[GT][4];
   // The row's statistics: wave w joins those of query columns w, w + kPvWaves,
@@ -453,20 +457,20 @@ __global__ __launch_bounds__(kPvThreads) void splitkv_pv_kernel(SplitArgs a) {
 
   // ---- the waves' sums, in wave order ----
   __syncthreads();  // the weights are read
-  float* red = reinterpret_cast<float*>(lds);  // [wave][GC][D]
+  float* red = reinterpret_cast<float*>(lds);  // [wave][GC][DV]
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int g = 4 * q + e;
     if (g < GC) {
 #pragma unroll
       for (int d4 = 0; d4 < DPC / 4; ++d4)
-        *reinterpret_cast<f32x4_v*>(red + (wv * GC + g) * D + out_dim<DPC>(n, 4 * d4)) =
+        *reinterpret_cast<f32x4_v*>(red + (wv * GC + g) * DV + out_dim<DPC>(n, 4 * d4)) =
             f32x4_v{acc[4 * d4][e], acc[4 * d4 + 1][e], acc[4 * d4 + 2][e], acc[4 * d4 + 3][e]};
     }
   }
   __syncthreads();
-  constexpr int PT = (GC * D / 2 + kPvThreads - 1) / kPvThreads;  // pairs of dims per thread
-  const int pairs = gn * (D / 2);
+  constexpr int PT = (GC * DV / 2 + kPvThreads - 1) / kPvThreads;  // pairs of dims per thread
+  const int pairs = gn * (DV / 2);
   f32x2_v sum[PT];
   // Thread t's i-th pair, 2 * (t + i * kPvThreads) floats on.
   auto each = [&](auto body) {
@@ -480,34 +484,34 @@ __global__ __launch_bounds__(kPvThreads) void splitkv_pv_kernel(SplitArgs a) {
     sum[i] = f32x2_v{0.0f, 0.0f};
 #pragma unroll
     for (int w = 0; w < kPvWaves; ++w)
-      sum[i] += *reinterpret_cast<const f32x2_v*>(red + w * (GC * D) + e);
+      sum[i] += *reinterpret_cast<const f32x2_v*>(red + w * (GC * DV) + e);
   });
 
   // ---- a row's workgroups, kPvFan at a time, in row order ----
   const int np = (S + (1 << rp.shift) - 1) >> rp.shift;  // of this row
   if (np > 1) {
-    const int nfan = (a.npv + kPvFan - 1) / kPvFan;  // of the longest row
-    // Piece c of the row leaves its heads' sums at part + c * stride.
+    const int nfan = (a.pv.npv + kPvFan - 1) / kPvFan;  // of the longest row
+    // Piece c of the row leaves its heads' sums at out + c * stride.
     const size_t stride = (size_t)hq * D;
-    float* part = a.opart + (uint64_t)(u - rp.piece) * stride + ((uint64_t)hk * G + qt * 16) * D;
-    uint32_t* done = a.done + (((uint64_t)b * hkv + hk) * tiles + qt) * (1 + nfan);
+    float* out = a.opart + (uint64_t)(u - rp.piece) * stride + ((uint64_t)hk * G + qt * 16) * D + part * (gn * DV);
+    uint32_t* done = a.done + ((((uint64_t)b * hkv + hk) * tiles + qt) * PARTS + part) * (1 + nfan);
     const int fan = (int)rp.piece / kPvFan;
     const int fan_n = np - fan * kPvFan < kPvFan ? np - fan * kPvFan : kPvFan;
-    each([&](int i, int e) { store_partial(part + rp.piece * stride + e, sum[i]); });
+    each([&](int i, int e) { store_partial(out + rp.piece * stride + e, sum[i]); });
     if (!last_to_finish(done + 1 + fan, (uint32_t)fan_n, &flag)) return;
-    each([&](int i, int e) { sum[i] = sum_partials(part + (size_t)fan * kPvFan * stride + e, fan_n, stride); });
+    each([&](int i, int e) { sum[i] = sum_partials(out + (size_t)fan * kPvFan * stride + e, fan_n, stride); });
     if (np > kPvFan) {
       // In the place of the first of them, which this thread has read.
-      each([&](int i, int e) { store_partial(part + (size_t)fan * kPvFan * stride + e, sum[i]); });
+      each([&](int i, int e) { store_partial(out + (size_t)fan * kPvFan * stride + e, sum[i]); });
       const int fans = (np + kPvFan - 1) / kPvFan;
       if (!last_to_finish(done, (uint32_t)fans, &flag)) return;
-      each([&](int i, int e) { sum[i] = sum_partials(part + e, fans, kPvFan * stride); });
+      each([&](int i, int e) { sum[i] = sum_partials(out + e, fans, kPvFan * stride); });
     }
   }
   each([&](int i, int e) {
     const uint32_t h0 = __builtin_bit_cast(uint16_t, (_Float16)sum[i][0]);
     const uint32_t h1 = __builtin_bit_cast(uint16_t, (_Float16)sum[i][1]);
-    __builtin_amdgcn_raw_buffer_store_b32(h0 | (h1 << 16), o_rsrc, e * 2, 0, kPolicyStreamStore);
+    __builtin_amdgcn_raw_buffer_store_b32(h0 | (h1 << 16), o_rsrc, (e / DV * D + e % DV) * 2, 0, kPolicyStreamStore);
   });
 }
 

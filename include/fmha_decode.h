@@ -392,11 +392,11 @@ const char* fmha_decode_last_error_detail(void);
  * kind with the choices the library made for it, e.g.
  *   "short(numerics=exact D=128 G=1 layout=packed bucket=16 waves_per_cu=4)"
  *   "split(D=128 G=4 layout=packed sub_units=1 blocks=65 scores_rows=16
- *    pv_rows=256 pv_rows_least=256 pieces=5 launches=2)",
+ *    pv_rows=256 pv_rows_least=256 pieces=5 pv_parts=1 launches=2)",
  * with the 16-row blocks of the longest row, the rows of a workgroup of the
  * scores launch and of the P.V launch (and the least that the device may make
- * of the latter where the lengths are short), and the pieces of that many rows
- * which the longest row has.
+ * of the latter where the lengths are short), the pieces of that many rows
+ * which the longest row has, and the P.V workgroups that share a piece's dims.
  * Kinds: short, short_multi (several batches per wave), short_matrix_core,
  * onepass, split, split_matrix_core, pad_query_group.  For tests and
  * diagnostics; no counterpart in the reference. */

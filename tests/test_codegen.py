@@ -11,9 +11,10 @@ import pytest
 from fmha_amd import _build
 
 KERNELS = (
-    "splitkv_pv_kernel<256, 8, kLayoutPagedBlock>",
-    "splitkv_pv_kernel<128, 4, kLayoutPagedBlock>",
-    "splitkv_pv_kernel<256, 4, kLayoutPacked>",
+    "splitkv_pv_kernel<256, 8, kLayoutPagedBlock, 1>",
+    "splitkv_pv_kernel<256, 8, kLayoutPagedBlock, 2>",
+    "splitkv_pv_kernel<128, 4, kLayoutPagedBlock, 1>",
+    "splitkv_pv_kernel<256, 4, kLayoutPacked, 1>",
     "splitkv_scores_kernel<128, 4, kLayoutPacked>",
     "splitkv_scores_kernel<64, 1, kLayoutStrided>",
     "splitkv_scores_group_kernel<256, kLayoutPacked>",
@@ -50,12 +51,12 @@ def listings(tmp_path_factory):
 
 
 def test_wide_rows_are_read_in_whole_lines(listings):
-    """P.V at 256 dims: a lane's second 16 bytes of a V row lie 256 bytes
+    """P.V at 256 dims of one workgroup: a lane's second 16 bytes of a V row lie 256 bytes
     after its first, so that each load instruction reads 256 neighbouring
     bytes of a row (16 bytes after them, every instruction took every other
     16 bytes of 512, and every line twice)."""
     for k in KERNELS:
-        if not k.startswith("splitkv_pv_kernel<256"):
+        if not re.match(r"splitkv_pv_kernel<256.* 1>", k):
             continue
         wide = [l for l in listings[k] if l.startswith("buffer_load_dwordx4")]
         assert wide

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import oracle
-from tests.common import assert_pass, default_scale, make_inputs, plan_kinds, plan_launch, to_dev
+from tests.common import assert_pass, default_scale, last_plan, make_inputs, plan_kinds, plan_launch, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -110,6 +110,89 @@ def test_many_calls_same_bits():
         torch.cuda.synchronize()
         for o in got:
             assert torch.equal(o.view(torch.int16), first.view(torch.int16)), i
+
+
+# (layout, Hq, Hkv, D, max_len, lengths, P.V rows planned, parts): lengths far
+# below the longest row allowed, for which the device takes shorter pieces than
+# planned (one batch, a few, one register of lengths and more), and as long,
+# for which it keeps them; head dims whole and by halves; empty and invalid
+# batches.  -1 stands for max_len + 1.
+CHOSEN = [
+    ("packed", 32, 8, 128, 131072, [5000], 2048, 1),
+    ("packed", 8, 8, 256, 60000, [3000], 4096, 2),
+    ("paged16", 64, 8, 128, 32768, [9000, 0, 2049, -1, 700, 1], 2048, 1),
+    ("strided", 8, 8, 64, 9000, [9000] + [400] * 11, 2048, 1),
+    ("packed", 16, 2, 256, 16384, [6000, 0, 300, 16], 1024, 2),
+    ("paged16", 8, 8, 256, 11516, [4000, -1, 0, 900, 257] + [100] * 5, 4096, 1),
+    ("strided", 2, 2, 256, 4096, [3000] + [150] * 43, 4096, 2),
+    ("paged1", 8, 1, 256, 8192, [5000, 600] + [250] * 18, 1024, 2),
+    ("packed", 1, 1, 64, 8000, [8000] + [300] * 69, 1024, 1),
+    ("packed", 8, 8, 64, 2233, [2233] * 57, 4096, 1),
+    ("paged16", 8, 8, 256, 4000, [4000] * 10 + [3500] * 12, 4096, 1),
+]
+
+
+@pytest.mark.parametrize("layout,Hq,Hkv,D,max_len,lens,rows,parts", CHOSEN)
+def test_device_chosen_pieces(monkeypatch, layout, Hq, Hkv, D, max_len, lens, rows, parts):
+    """What the device makes of the lengths, with a workspace of exactly the
+    size asked for between guard bytes, which stay."""
+    import torch
+    import fmha_amd
+    monkeypatch.setenv("FMHA_DECODE_ONEPASS_REG", "0")
+    monkeypatch.setenv("FMHA_DECODE_ONEPASS_MFMA", "0")
+    B = len(lens)
+    invalid = [b for b, n in enumerate(lens) if n < 0]
+    said = np.array([max_len + 1 if n < 0 else n for n in lens], np.int32)
+    # An invalid batch's rows are not read: packed caches have none of it here.
+    held = np.array([0 if n < 0 else n for n in lens], np.int32)
+    assert layout != "packed" or not invalid
+    q, k, v, cu = make_inputs(B, Hq, Hkv, D, held, seed=B + D + Hq + max_len, std=0.5)
+    need, guard = fmha_amd.splitkv_workspace_size(B, Hq, Hkv, max_len, D), 4096
+    room = torch.full((guard + need + guard,), 0xA5, dtype=torch.uint8, device="cuda")
+    ws = room[guard:guard + need]
+    ws.fill_(0xFF)
+    scale = default_scale(D)
+    ln = torch.from_numpy(said).cuda()
+    if layout == "packed":
+        call = lambda: _call(to_dev(q), to_dev(k), to_dev(v), torch.from_numpy(cu).cuda(), max_len, D, ws)  # noqa: E731
+    elif layout == "strided":
+        kc, vc = (torch.zeros(B, max_len, Hkv, D, dtype=torch.int16) for _ in range(2))
+        for b in range(B):
+            kc[b, :held[b]] = torch.from_numpy(k[cu[b]:cu[b + 1]].view(np.int16))
+            vc[b, :held[b]] = torch.from_numpy(v[cu[b]:cu[b + 1]].view(np.int16))
+        kc, vc = (x.cuda().view(torch.bfloat16) for x in (kc, vc))
+        call = lambda: fmha_amd.fmha_decode_strided(to_dev(q), kc, vc, ln, softmax_scale=scale, workspace=ws)  # noqa: E731
+    else:
+        page = int(layout[5:])
+        used = [(int(n) + page - 1) // page for n in held]
+        perm = np.random.default_rng(3).permutation(sum(used)).astype(np.int32)
+        table = np.full((B, (max_len + page - 1) // page), -1, np.int32)
+        slots = np.zeros(len(k), np.int64)
+        at = 0
+        for b in range(B):
+            table[b, :used[b]] = perm[at:at + used[b]]
+            at += used[b]
+            j = np.arange(held[b])
+            slots[cu[b]:cu[b + 1]] = table[b, j // page].astype(np.int64) * page + j % page
+        kc, vc = (np.zeros((sum(used) * page, Hkv, D), np.uint16) for _ in range(2))
+        kc[slots], vc[slots] = k, v
+        kc, vc = (to_dev(x.reshape(-1, page, Hkv, D)) for x in (kc, vc))
+        bt = torch.from_numpy(table).cuda()
+        call = lambda: fmha_amd.fmha_decode_paged(to_dev(q), kc, vc, bt, ln, softmax_scale=scale,  # noqa: E731
+                                                  max_seqlen_kv=max_len, workspace=ws)
+    first = call()
+    split = [f for kind, f in last_plan() if kind.startswith("split")]
+    assert len(split) == 1 and split[0]["pv_rows"] == rows and split[0]["pv_parts"] == parts, split
+    second = call()
+    torch.cuda.synchronize()
+    assert bool((room[:guard] == 0xA5).all()) and bool((room[guard + need:] == 0xA5).all())
+    bits = first.view(torch.int16).cpu().numpy().view(np.uint16)
+    assert np.array_equal(bits, second.view(torch.int16).cpu().numpy().view(np.uint16))
+    r, slack = oracle.decode(q, k, v, cu, Hq, Hkv, D, scale, with_slack=True, max_seqlen=max_len)
+    bits = bits.reshape(r.shape)
+    assert np.all(np.isnan(oracle.f16_to_f32(bits[invalid])))
+    ok = [b for b in range(B) if b not in invalid]
+    assert_pass(oracle.compare(bits[ok], r[ok], slack[ok]), f"{layout} B={B} G={Hq // Hkv} D={D} max={max_len}")
 
 
 @pytest.mark.parametrize("page_size", [1, 16, 64])

@@ -532,7 +532,9 @@ struct SplitPlan {
 };
 
 // The split passes' workspace and the pieces of the P.V launch.
-SplitPlan plan_split(int64_t batch, int hq, int hkv, int max_rows, int d) {
+// pv_units: the (KV head, query tile) pairs that the P.V launch serves for
+// each piece of a row, as far as the group size tells.
+SplitPlan plan_split(int64_t batch, int hq, int hkv, int pv_units, int max_rows, int d) {
   SplitPlan p;
   const int heads_per_wave = kWaveSize / (d / 8);
   p.units = (hkv + heads_per_wave - 1) / heads_per_wave * batch;
@@ -544,7 +546,7 @@ SplitPlan plan_split(int64_t batch, int hq, int hkv, int max_rows, int d) {
     const int v = std::atoi(e);
     if (v >= 128 && v <= 4096 && (v & (v - 1)) == 0) forced = v;
   }
-  p.pv = fmha_decode::plan_pv_pieces(batch, hkv, max_rows, d, forced);
+  p.pv = fmha_decode::plan_pv_pieces(batch, pv_units, max_rows, d, forced);
   p.nblk = max_rows <= 0 ? 1 : (max_rows + fmha_decode::kSplitBlockRows - 1) / fmha_decode::kSplitBlockRows;
   const size_t heads = (size_t)batch * hq;
   const size_t fans = (size_t)(p.pv.npv + fmha_decode::kPvFan - 1) / fmha_decode::kPvFan;
@@ -842,14 +844,16 @@ extern "C" size_t fmha_decode_splitkv_workspace_size(int32_t batch, int32_t num_
       (head_dim != 64 && head_dim != 128 && head_dim != 256))
     return 0;
   const int g = num_heads_q % num_heads_kv == 0 ? num_heads_q / num_heads_kv : 0;
-  if (g == 0 || valu_group(g)) return plan_split(batch, num_heads_q, num_heads_kv, max_seqlen_kv, head_dim).total;
+  if (g == 0 || valu_group(g))
+    return plan_split(batch, num_heads_q, num_heads_kv, num_heads_kv, max_seqlen_kv, head_dim).total;
   // G > 8: ns groups of 8 per KV head on Hkv * ns launch KV heads; Q and O
   // copies unless G is a multiple of 8.  G = 3, 5-7: the copies padded to
   // 4 or 8, and the plan for Hkv * GP heads.
   const int gp = long_row_group(g);
   const int ns = g > 8 ? gp / 8 : 1;
   const size_t pad = gp == g ? 0 : 2 * group_pad_bytes(batch, num_heads_kv, gp, head_dim);
-  return pad + plan_split(batch, num_heads_kv * gp, num_heads_kv * ns, max_seqlen_kv, head_dim).total;
+  return pad + plan_split(batch, num_heads_kv * gp, num_heads_kv * ns, num_heads_kv * ((gp + 15) / 16), max_seqlen_kv,
+                          head_dim).total;
 }
 
 namespace {
@@ -861,7 +865,9 @@ namespace {
 int split_prepare(const void* Q, const void* K, const void* V, void* O, int32_t max_seqlen_kv,
                   int32_t batch, int32_t num_heads_q, int32_t num_heads_kv, int32_t kv_groups, int32_t head_dim,
                   float softmax_scale, void* workspace, size_t workspace_bytes, int64_t kv_span_bytes, SplitArgs& a) {
-  const SplitPlan plan = plan_split(batch, num_heads_q, num_heads_kv, max_seqlen_kv, head_dim);
+  const int g_mem = num_heads_q / num_heads_kv * kv_groups;
+  const SplitPlan plan = plan_split(batch, num_heads_q, num_heads_kv, num_heads_kv / kv_groups * ((g_mem + 15) / 16),
+                                    max_seqlen_kv, head_dim);
   const int64_t padded_rows = (int64_t)plan.nblk * fmha_decode::kSplitBlockRows;
   const int64_t part_bytes = (int64_t)num_heads_q * plan.pv.npv * head_dim * 4;  // one batch's partials
   if (kv_span_bytes >= (int64_t(1) << 30) || padded_rows * num_heads_q * 4 >= (int64_t(1) << 30) ||

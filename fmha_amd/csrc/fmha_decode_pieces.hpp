@@ -22,22 +22,20 @@ constexpr int kPvMinShift = 8, kPvMaxShift = 12;  // planned pieces: 256 to 4096
 // Batches up to which the device adds up the lengths.
 constexpr int kOrderBatches = 256;
 
-// Workgroups a plan for full rows asks for, about two for each CU, all of them
-// at once (µs of the call at 2048 / 4096 rows, 32/8 B=8 S=32768 194.4 / 192.3,
-// 64/8 218.6 / 207.0; P.V alone, B=1 S=131072 71 / 59 / 54 at 512 / 1024 /
-// 2048).  At 256 dims, with twice the bytes in flight for each wave or head,
-// fewer do (8/1 B=9 S=40879 on 64-row pages, by halves, 180 workgroups 82.1,
-// 720 85.9; 64/8 B=16 S=4096 256 95.4, 512 100.0; 16/2 B=4 S=16384 on 16-row
-// pages 256 37.7, 512 40.1, 128 41.0).
-constexpr int64_t kPvMinGroups = 448, kPvMinGroupsWide = 176;
-// Ragged batches: the workgroups below which the device takes shorter pieces
-// (from pv.big on kPvMinGroups; µs by rows, their workgroups in brackets: B=48
+// A piece's start and end in rows of it, and the CUs: a CU streams for about
+// one workgroup at a time (for two at 64 dims), whatever it holds.
+constexpr int64_t kPvPieceRows = 600, kPvCus = 256;
+// Pieces of kPvMaxShift from which on a workgroup takes all of 256 dims.
+constexpr int64_t kPvWholeGroups = 176;
+// Ragged batches: the workgroups below which the device takes shorter pieces,
+// and those below which it does from pv.big on (µs by rows, their workgroups in
+// brackets: B=48
 // 8/1 over 250-8000 rows 26.9 (420) / 25.1 (210) / 26.6 (105) at 256 / 512 /
 // 1024; B=6 64/8 over 1024-32768 64.9 (430) / 63.3 (215) / 73.4 (107) at 1024
 // / 2048 / 4096; D=64 B=22 8/8 over 666-21321 65.3 (512) / 71.5 (256) at 2048
 // / 4096; D=256 B=8 40/8 over 188-6000 on 64-row pages 39.7 (425) / 41.3
 // (212) at 512 / 1024).
-constexpr int64_t kPvFewGroups = 192;
+constexpr int64_t kPvFewGroups = 192, kPvManyGroups = 448;
 
 struct PvPieces {
   int32_t shift;  // log2 of a piece's rows where the batches are full,
@@ -73,39 +71,52 @@ FMHA_DECODE_HD int pv_device_shift(const PvPieces& pv, int rows) {
   return s;
 }
 
-// The plan for batch rows of up to max_rows on hkv KV heads: the longest
-// pieces that leave enough workgroups, but not a size that leaves the last of
-// two or three pieces of a row mostly empty (64-row pages D=64 B=57 8/8 S=2233:
-// 67.6 at 2048 rows, 58.1 at 1024, 52.8 in one), and, where the device adds up
-// the lengths, no row of more than 1024 in one piece in a ragged batch (packed
-// D=64 8/8 over 62-2000 rows: B=120 40.1 in one, 37.9 at 1024, but B=300 75.5
-// and 88.5, where the pieces that short rows don't have are launched too).  At 256 dims with fewer than
-// kPvMinGroupsWide pieces of kPvMaxShift, two workgroups share a head's dims:
-// half the sums for each (µs, one / two: B=1 32/4 S=5000 24.8 / 18.8, 32/1
-// S=4000 28.5 / 20.5, 64/8 B=16 S=4096 99.1 / 95.4; above, each reads half of
-// every 512 bytes: 28/4 B=3 S=66558 162 / 170, BHSD 32/16 B=1 S=61035 160 /
-// 165).  forced_rows > 0: pieces of so many rows, everywhere.
-inline PvPieces plan_pv_pieces(int64_t batch, int hkv, int max_rows, int d, int forced_rows) {
+// The plan for `batch` rows of up to max_rows and `units` (KV head, query tile)
+// pairs: the size whose busiest CU is done first.  While all workgroups start
+// at once (four to a CU, three of 256 dims) that CU has one more of them than
+// others may, each as long as a full piece; more of them fill up the CUs as
+// they free up.  µs of the call by rows, with the workgroups in brackets: 32/32
+// D=128 B=9 S=6663 on 16-row pages 186.4 (576) / 168.5 (1152) / 170.3 (2016) at
+// 4096 / 2048 / 1024; 32/8 B=1 S=131072 102.2 (256) / 103.4 (512) / 106.9
+// (1024); 16/2 D=256 B=4 S=16384 41.1 (128) / 37.9 (256) / 40.5 (512) at 2048 /
+// 1024 / 512; 8/8 D=64 B=57 S=2233 on 64-row pages 53.1 (456) / 68.3 (912) / 58.5
+// (1368) at 4096 / 2048 / 1024; 4/1 D=64 B=12 S=30000 44.4 (96) / 35.2 (180) /
+// 33.1 (360) / 33.4 (708) at 4096 / 2048 / 1024 / 512.
+//
+// Where the device adds up the lengths, no row of more than 1024 is one piece
+// in a ragged batch (packed D=64 8/8 over 62-2000 rows: B=120 40.1 in one, 37.9
+// at 1024, but B=300 75.5 and 88.5, where the pieces that short rows don't have
+// are launched too).
+//
+// At 256 dims with fewer than kPvWholeGroups pieces of kPvMaxShift, two
+// workgroups share a head's dims: half the sums for each (µs, one / two: B=1
+// 32/4 S=5000 24.8 / 18.8, 32/1 S=4000 28.5 / 20.4, 64/8 B=16 S=4096 99.1 /
+// 95.4; above, each reads half of every 512 bytes: 28/4 B=3 S=66558 162 / 170,
+// BHSD 32/16 B=1 S=61035 160 / 165).  forced_rows > 0: pieces of so many rows,
+// everywhere.
+inline PvPieces plan_pv_pieces(int64_t batch, int units, int max_rows, int d, int forced_rows) {
   const auto groups = [&](int s) { return max_rows <= 0 ? 1 : ((int64_t)max_rows + (1 << s) - 1) >> s; };
   PvPieces pv{};
   const bool wide = d == 256;
-  const int64_t enough = wide ? kPvMinGroupsWide : kPvMinGroups;
-  pv.parts = wide && batch * hkv * groups(kPvMaxShift) < enough ? 2 : 1;
-  const int64_t heads = (int64_t)hkv * pv.parts;
-  const auto fits = [&](int s) {
-    const int64_t n = groups(s);
-    if (n > 1 && n < 4 && (int64_t)max_rows * 10 < 7 * (n << s)) return false;
-    return batch * heads * n >= enough;
+  pv.parts = wide && batch * units * groups(kPvMaxShift) < kPvWholeGroups ? 2 : 1;
+  const int64_t heads = (int64_t)units * pv.parts;
+  const int64_t places = d == 64 ? 2 * kPvCus : kPvCus;
+  const int64_t at_once = kPvCus * (wide && pv.parts == 1 ? 3 : 4);
+  const auto cost = [&](int s) {  // in half rows
+    const int64_t n = groups(s), w = batch * heads * n;
+    if (w <= at_once) return 2 * ((w + places - 1) / places) * ((n == 1 ? max_rows : 1 << s) + kPvPieceRows);
+    return (2 * w + places) * ((max_rows + n - 1) / n + kPvPieceRows) / places;
   };
   pv.shift = kPvMaxShift;
-  while (pv.shift > kPvMinShift && !fits(pv.shift)) --pv.shift;
+  for (int s = kPvMaxShift - 1; s >= kPvMinShift; --s)
+    if (cost(s) < cost(pv.shift)) pv.shift = s;
   if (forced_rows > 0)
     for (pv.shift = 0; 1 << pv.shift < forced_rows;) ++pv.shift;
   pv.fine = forced_rows > 0 || batch > kOrderBatches || pv.shift < kPvMinShift ? pv.shift : kPvMinShift;
   pv.most = pv.shift;
   while (pv.most > pv.fine && max_rows > 1024 && groups(pv.most) == 1) --pv.most;
   pv.few = (int32_t)((kPvFewGroups + heads - 1) / heads);
-  pv.many = (int32_t)((kPvMinGroups + heads - 1) / heads);
+  pv.many = (int32_t)((kPvManyGroups + heads - 1) / heads);
   pv.big = wide ? 10 : kPvMaxShift;
   const int64_t allowed = batch * pv_counted_rows(max_rows, max_rows);  // below 2^31 where the device adds up
   pv.full = allowed / 4 * 3 < INT32_MAX ? (int32_t)(allowed / 4 * 3) : INT32_MAX;

@@ -118,15 +118,15 @@ def test_many_calls_same_bits():
 # for which it keeps them; head dims whole and by halves; empty and invalid
 # batches.  -1 stands for max_len + 1.
 CHOSEN = [
-    ("packed", 32, 8, 128, 131072, [5000], 2048, 1),
+    ("packed", 32, 8, 128, 131072, [5000], 4096, 1),
     ("packed", 8, 8, 256, 60000, [3000], 4096, 2),
     ("paged16", 64, 8, 128, 32768, [9000, 0, 2049, -1, 700, 1], 2048, 1),
     ("strided", 8, 8, 64, 9000, [9000] + [400] * 11, 2048, 1),
     ("packed", 16, 2, 256, 16384, [6000, 0, 300, 16], 1024, 2),
     ("paged16", 8, 8, 256, 11516, [4000, -1, 0, 900, 257] + [100] * 5, 4096, 1),
     ("strided", 2, 2, 256, 4096, [3000] + [150] * 43, 4096, 2),
-    ("paged1", 8, 1, 256, 8192, [5000, 600] + [250] * 18, 1024, 2),
-    ("packed", 1, 1, 64, 8000, [8000] + [300] * 69, 1024, 1),
+    ("paged1", 8, 1, 256, 8192, [5000, 600] + [250] * 18, 2048, 2),
+    ("packed", 1, 1, 64, 8000, [8000] + [300] * 69, 2048, 1),
     ("packed", 8, 8, 64, 2233, [2233] * 57, 4096, 1),
     ("paged16", 8, 8, 256, 4000, [4000] * 10 + [3500] * 12, 4096, 1),
 ]

@@ -51,9 +51,10 @@ def test_block_boundaries(D, Hq, Hkv):
     _case(len(seqlens), Hq, Hkv, D, seqlens, 64, seed=11 + D)
 
 
-def test_sums_in_two_levels():
+def test_sums_in_two_levels(monkeypatch):
     """Rows of more than 16 P.V workgroups, whose partial outputs are summed
     16 at a time and then once more, and of at most 16 in the same call."""
+    monkeypatch.setenv("FMHA_DECODE_SPLIT_CHUNK", "256")
     seqlens = np.array([8192, 6001, 700], np.int32)
     _case(3, 8, 8, 128, seqlens, 8192, seed=12, std=0.5)
     assert _launch("split")["pieces"] > 16

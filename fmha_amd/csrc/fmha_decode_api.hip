@@ -532,9 +532,9 @@ struct SplitPlan {
 };
 
 // The split passes' workspace and the pieces of the P.V launch.
-// pv_units: the (KV head, query tile) pairs that the P.V launch serves for
-// each piece of a row, as far as the group size tells.
-SplitPlan plan_split(int64_t batch, int hq, int hkv, int pv_units, int max_rows, int d) {
+// kv_groups: launch KV heads per KV head of the cache (SplitArgs); scattered:
+// pages under 16 rows.
+SplitPlan plan_split(int64_t batch, int hq, int hkv, int kv_groups, int max_rows, int d, bool scattered) {
   SplitPlan p;
   const int heads_per_wave = kWaveSize / (d / 8);
   p.units = (hkv + heads_per_wave - 1) / heads_per_wave * batch;
@@ -546,7 +546,9 @@ SplitPlan plan_split(int64_t batch, int hq, int hkv, int pv_units, int max_rows,
     const int v = std::atoi(e);
     if (v >= 128 && v <= 4096 && (v & (v - 1)) == 0) forced = v;
   }
-  p.pv = fmha_decode::plan_pv_pieces(batch, pv_units, max_rows, d, forced);
+  // Groups above 8 mostly take the matrix cores, 16 query heads a workgroup.
+  const int hkv_mem = hkv / kv_groups, g = hq < hkv_mem ? 1 : hq / hkv_mem;
+  p.pv = fmha_decode::plan_pv_pieces(batch, hkv_mem * ((g + 15) / 16), g, max_rows, d, scattered, forced);
   p.nblk = max_rows <= 0 ? 1 : (max_rows + fmha_decode::kSplitBlockRows - 1) / fmha_decode::kSplitBlockRows;
   const size_t heads = (size_t)batch * hq;
   const size_t fans = (size_t)(p.pv.npv + fmha_decode::kPvFan - 1) / fmha_decode::kPvFan;
@@ -844,16 +846,20 @@ extern "C" size_t fmha_decode_splitkv_workspace_size(int32_t batch, int32_t num_
       (head_dim != 64 && head_dim != 128 && head_dim != 256))
     return 0;
   const int g = num_heads_q % num_heads_kv == 0 ? num_heads_q / num_heads_kv : 0;
-  if (g == 0 || valu_group(g))
-    return plan_split(batch, num_heads_q, num_heads_kv, num_heads_kv, max_seqlen_kv, head_dim).total;
+  // The larger of the plans that the layouts take.
+  const auto plan_total = [&](int hq, int hkv, int kvg) {
+    const size_t a = plan_split(batch, hq, hkv, kvg, max_seqlen_kv, head_dim, false).total;
+    const size_t b = plan_split(batch, hq, hkv, kvg, max_seqlen_kv, head_dim, true).total;
+    return a > b ? a : b;
+  };
+  if (g == 0 || valu_group(g)) return plan_total(num_heads_q, num_heads_kv, 1);
   // G > 8: ns groups of 8 per KV head on Hkv * ns launch KV heads; Q and O
   // copies unless G is a multiple of 8.  G = 3, 5-7: the copies padded to
   // 4 or 8, and the plan for Hkv * GP heads.
   const int gp = long_row_group(g);
   const int ns = g > 8 ? gp / 8 : 1;
   const size_t pad = gp == g ? 0 : 2 * group_pad_bytes(batch, num_heads_kv, gp, head_dim);
-  return pad + plan_split(batch, num_heads_kv * gp, num_heads_kv * ns, num_heads_kv * ((gp + 15) / 16), max_seqlen_kv,
-                          head_dim).total;
+  return pad + plan_total(num_heads_kv * gp, num_heads_kv * ns, ns);
 }
 
 namespace {
@@ -862,12 +868,10 @@ namespace {
 // layout-independent fields of the launch.  kv_span_bytes: the largest byte
 // range one wave's K/V descriptor covers in the caller's layout (must stay
 // below 2^30, as must one batch's scores and partial outputs).
-int split_prepare(const void* Q, const void* K, const void* V, void* O, int32_t max_seqlen_kv,
+int split_prepare(bool scattered, const void* Q, const void* K, const void* V, void* O, int32_t max_seqlen_kv,
                   int32_t batch, int32_t num_heads_q, int32_t num_heads_kv, int32_t kv_groups, int32_t head_dim,
                   float softmax_scale, void* workspace, size_t workspace_bytes, int64_t kv_span_bytes, SplitArgs& a) {
-  const int g_mem = num_heads_q / num_heads_kv * kv_groups;
-  const SplitPlan plan = plan_split(batch, num_heads_q, num_heads_kv, num_heads_kv / kv_groups * ((g_mem + 15) / 16),
-                                    max_seqlen_kv, head_dim);
+  const SplitPlan plan = plan_split(batch, num_heads_q, num_heads_kv, kv_groups, max_seqlen_kv, head_dim, scattered);
   const int64_t padded_rows = (int64_t)plan.nblk * fmha_decode::kSplitBlockRows;
   const int64_t part_bytes = (int64_t)num_heads_q * plan.pv.npv * head_dim * 4;  // one batch's partials
   if (kv_span_bytes >= (int64_t(1) << 30) || padded_rows * num_heads_q * 4 >= (int64_t(1) << 30) ||
@@ -1056,7 +1060,7 @@ int splitkv_packed(void* stream, const void* Q, const void* K, const void* V, vo
     if (numerics != Numerics::kExact && use_mfma_kernel(num_heads_q / num_heads_kv))
       return launch_mfma(stream, fmha_decode::kLayoutPacked, d, batch, head_dim_q, rows_hint);
     SplitArgs unused;
-    rc = split_prepare(Q, K, V, O, max_seqlen_kv, batch, num_heads_q, num_heads_kv, 1,
+    rc = split_prepare(false, Q, K, V, O, max_seqlen_kv, batch, num_heads_q, num_heads_kv, 1,
                        head_dim_q, softmax_scale, workspace, workspace_bytes, span, unused);
     if (rc != FMHA_DECODE_SUCCESS) return rc;
     d.rows_feedback = feedback_word(stream, may_allocate);
@@ -1067,7 +1071,7 @@ int splitkv_packed(void* stream, const void* Q, const void* K, const void* V, vo
       stream, Q, O, batch, num_heads_q, num_heads_kv, head_dim_q, workspace, workspace_bytes,
       [&](const void* q, void* o, int32_t hq, int32_t hkv, int32_t kvg, void* ws, size_t ws_bytes) {
         SplitArgs a;
-        int rc2 = split_prepare(q, K, V, o, max_seqlen_kv, batch, hq, hkv, kvg,
+        int rc2 = split_prepare(false, q, K, V, o, max_seqlen_kv, batch, hq, hkv, kvg,
                                 head_dim_q, softmax_scale, ws, ws_bytes, span, a);
         if (rc2 != FMHA_DECODE_SUCCESS) return rc2;
         a.cu = cu_seqlens_kv;
@@ -1182,7 +1186,7 @@ extern "C" int fmha_decode_fwd_splitkv_strided(void* stream, const void* Q, cons
       stream, Q, O, batch, num_heads_q, num_heads_kv, head_dim_q, workspace, workspace_bytes,
       [&](const void* q, void* o, int32_t hq, int32_t hkv, int32_t kvg, void* ws, size_t ws_bytes) {
         SplitArgs a;
-        int rc2 = split_prepare(q, K, V, o, max_seqlen_kv, batch, hq, hkv, kvg,
+        int rc2 = split_prepare(false, q, K, V, o, max_seqlen_kv, batch, hq, hkv, kvg,
                                 head_dim_q, softmax_scale, ws, ws_bytes, extent, a);
         if (rc2 != FMHA_DECODE_SUCCESS) return rc2;
         a.cu = seqlens_kv;
@@ -1225,8 +1229,8 @@ extern "C" int fmha_decode_fwd_splitkv_paged(void* stream, const void* Q, const 
       stream, Q, O, batch, num_heads_q, num_heads_kv, head_dim_q, workspace, workspace_bytes,
       [&](const void* q, void* o, int32_t hq, int32_t hkv, int32_t kvg, void* ws, size_t ws_bytes) {
         SplitArgs a;
-        int rc2 = split_prepare(q, K_cache, V_cache, o, max_seqlen_kv, batch, hq, hkv, kvg, head_dim_q,
-                                softmax_scale, ws, ws_bytes, 16 * row_bytes, a);
+        int rc2 = split_prepare(page_layout == fmha_decode::kLayoutPaged, q, K_cache, V_cache, o, max_seqlen_kv, batch,
+                                hq, hkv, kvg, head_dim_q, softmax_scale, ws, ws_bytes, 16 * row_bytes, a);
         if (rc2 != FMHA_DECODE_SUCCESS) return rc2;
         a.cu = seqlens_kv;
         a.len_mode = fmha_decode::kLenArray;

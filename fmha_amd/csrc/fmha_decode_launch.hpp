@@ -937,7 +937,9 @@ hipError_t launch_split_dg(const SplitArgs& a, hipStream_t stream, bool onepass_
   SplitArgs as = a;
   as.sub_shift = shift;
   as.units_per_batch = (a.num_heads_kv + (HPW >> shift) - 1) / (HPW >> shift);
-  const int wpg = (a.nblk >> shift) > fmha_decode::kScoresLongBlocks ? fmha_decode::kScoresMaxWaves : 1;
+  const int wpg = (a.nblk >> shift) <= fmha_decode::kScoresLongBlocks ? 1
+                  : G <= 2                                            ? fmha_decode::kScoresMaxWaves / 2
+                                                                      : fmha_decode::kScoresMaxWaves;
   as.sup_shift = 4 + shift + fmha_decode::ilog2(wpg);
   as.nsup = (a.max_rows + (1 << as.sup_shift) - 1) >> as.sup_shift;
   const int64_t groups = (int64_t)a.batch * as.nsup * as.units_per_batch;

@@ -22,19 +22,20 @@ constexpr int kPvMinShift = 8, kPvMaxShift = 12;  // planned pieces: 256 to 4096
 // Batches up to which the device adds up the lengths.
 constexpr int kOrderBatches = 256;
 
-// A piece's start and end in rows of it, and the CUs: a CU streams for about
-// one workgroup at a time (for two at 64 dims), whatever it holds.
-constexpr int64_t kPvPieceRows = 600, kPvCus = 256;
+// What of a piece's start and end its CU's other workgroups don't hide, in rows
+// of it, and the CUs.
+constexpr int64_t kPvPieceRows = 400, kPvSlowPieceRows = 600, kPvCus = 256;
 // Pieces of kPvMaxShift from which on a workgroup takes all of 256 dims.
 constexpr int64_t kPvWholeGroups = 176;
 // Ragged batches: the workgroups below which the device takes shorter pieces,
-// and those below which it does from pv.big on (µs by rows, their workgroups in
-// brackets: B=48
+// and those below which it does from pv.big on; one with a group above 8 counts
+// twice (µs by rows, their workgroups in brackets: B=48
 // 8/1 over 250-8000 rows 26.9 (420) / 25.1 (210) / 26.6 (105) at 256 / 512 /
 // 1024; B=6 64/8 over 1024-32768 64.9 (430) / 63.3 (215) / 73.4 (107) at 1024
 // / 2048 / 4096; D=64 B=22 8/8 over 666-21321 65.3 (512) / 71.5 (256) at 2048
 // / 4096; D=256 B=8 40/8 over 188-6000 on 64-row pages 39.7 (425) / 41.3
-// (212) at 512 / 1024).
+// (212) at 512 / 1024; 32/1 B=48 over 97-3119 28.0 (330) / 25.0 (170) at 256 /
+// 512).
 constexpr int64_t kPvFewGroups = 192, kPvManyGroups = 448;
 
 struct PvPieces {
@@ -72,21 +73,36 @@ FMHA_DECODE_HD int pv_device_shift(const PvPieces& pv, int rows) {
 }
 
 // The plan for `batch` rows of up to max_rows and `units` (KV head, query tile)
-// pairs: the size whose busiest CU is done first.  While all workgroups start
+// pairs of groups of g: the size whose busiest CU is done first.  While all workgroups start
 // at once (four to a CU, three of 256 dims) that CU has one more of them than
 // others may, each as long as a full piece; more of them fill up the CUs as
-// they free up.  µs of the call by rows, with the workgroups in brackets: 32/32
+// they free up.  A CU streams for about one workgroup at a time, whatever it
+// holds, but for two where they are slow: at 64 dims, with groups above 8
+// (weights of 16 query columns) and on scattered rows (pages under 16 rows, an
+// entry for each), and then with no fewer than kPvManyGroups, but for groups
+// above 8.  µs of the call by rows, with the workgroups in brackets: 32/32
 // D=128 B=9 S=6663 on 16-row pages 186.4 (576) / 168.5 (1152) / 170.3 (2016) at
 // 4096 / 2048 / 1024; 32/8 B=1 S=131072 102.2 (256) / 103.4 (512) / 106.9
 // (1024); 16/2 D=256 B=4 S=16384 41.1 (128) / 37.9 (256) / 40.5 (512) at 2048 /
 // 1024 / 512; 8/8 D=64 B=57 S=2233 on 64-row pages 53.1 (456) / 68.3 (912) / 58.5
 // (1368) at 4096 / 2048 / 1024; 4/1 D=64 B=12 S=30000 44.4 (96) / 35.2 (180) /
-// 33.1 (360) / 33.4 (708) at 4096 / 2048 / 1024 / 512.
+// 33.1 (360) / 33.4 (708) at 4096 / 2048 / 1024 / 512; 32/1 B=60 S=4777 on 16-row
+// pages 74.0 (240) / 68.9 (360) / 64.7 (600) at 4096 / 2048 / 1024; BHSD 28/4 B=23
+// S=1208 29.1 (184) / 25.3 (460) at 1024 / 256; one-row pages D=128 32/8 B=1
+// S=100000 102.9 (200) / 92.8 (392) / 98.5 (784) at 4096 / 2048 / 1024, 16/16 B=2
+// S=9000 47.9 (160) / 42.7 (288) / 40.4 (576) at 2048 / 1024 / 512.
 //
-// Where the device adds up the lengths, no row of more than 1024 is one piece
-// in a ragged batch (packed D=64 8/8 over 62-2000 rows: B=120 40.1 in one, 37.9
-// at 1024, but B=300 75.5 and 88.5, where the pieces that short rows don't have
-// are launched too).
+// Rows of up to 512 are one piece (µs at 256 / 512 rows, S=300 8/8 D=128 B=4 11.3
+// / 10.7, 32/8 B=8 on 16-row pages 13.8 / 12.8; S=512 11.6 / 11.4, 14.1 / 14.1).
+// With more batches than the device adds up, the longest of at most 2048 rows
+// that leave kPvManyGroups: the pieces that short rows don't have are launched
+// too (packed D=64 8/8 B=300 over 62-2000 rows 75.5 in one piece each, 88.5 at
+// 1024; 32/1 B=291 over 22-713 29.7 in one, 37.7 at 512; BHSD D=64 4/1 B=764
+// over 160-5107 88 at 2048, 107 at 4096).
+//
+// A ragged batch takes no more than a third of its longest row at once, from
+// 1024 rows on (packed D=64 8/8 B=120 over 62-2000 rows 40.1 in one, 37.9 at
+// 1024; 16-row pages B=100 over 94-3000 48.1 at 2048, 44.2 at 1024).
 //
 // At 256 dims with fewer than kPvWholeGroups pieces of kPvMaxShift, two
 // workgroups share a head's dims: half the sums for each (µs, one / two: B=1
@@ -94,29 +110,36 @@ FMHA_DECODE_HD int pv_device_shift(const PvPieces& pv, int rows) {
 // 95.4; above, each reads half of every 512 bytes: 28/4 B=3 S=66558 162 / 170,
 // BHSD 32/16 B=1 S=61035 160 / 165).  forced_rows > 0: pieces of so many rows,
 // everywhere.
-inline PvPieces plan_pv_pieces(int64_t batch, int units, int max_rows, int d, int forced_rows) {
+inline PvPieces plan_pv_pieces(int64_t batch, int units, int g, int max_rows, int d, bool scattered,
+                               int forced_rows) {
   const auto groups = [&](int s) { return max_rows <= 0 ? 1 : ((int64_t)max_rows + (1 << s) - 1) >> s; };
   PvPieces pv{};
   const bool wide = d == 256;
   pv.parts = wide && batch * units * groups(kPvMaxShift) < kPvWholeGroups ? 2 : 1;
   const int64_t heads = (int64_t)units * pv.parts;
-  const int64_t places = d == 64 ? 2 * kPvCus : kPvCus;
+  const bool slow = d == 64 || scattered;
+  const int64_t places = slow || g > 8 ? 2 * kPvCus : kPvCus;
+  const int64_t ends = slow ? kPvSlowPieceRows : kPvPieceRows;
   const int64_t at_once = kPvCus * (wide && pv.parts == 1 ? 3 : 4);
   const auto cost = [&](int s) {  // in half rows
     const int64_t n = groups(s), w = batch * heads * n;
-    if (w <= at_once) return 2 * ((w + places - 1) / places) * ((n == 1 ? max_rows : 1 << s) + kPvPieceRows);
-    return (2 * w + places) * ((max_rows + n - 1) / n + kPvPieceRows) / places;
+    if (w <= at_once) return 2 * ((w + places - 1) / places) * ((n == 1 ? max_rows : 1 << s) + ends);
+    return (2 * w + (slow ? 2 : 1) * places) * ((max_rows + n - 1) / n + ends) / places;
   };
-  pv.shift = kPvMaxShift;
-  for (int s = kPvMaxShift - 1; s >= kPvMinShift; --s)
-    if (cost(s) < cost(pv.shift)) pv.shift = s;
+  const int least = max_rows <= 1 << (kPvMinShift + 1) ? kPvMinShift + 1 : kPvMinShift;
+  pv.shift = batch > kOrderBatches ? kPvMaxShift - 1 : kPvMaxShift;
+  for (int s = pv.shift - 1; s >= least; --s) {
+    const bool few = batch * heads * groups(pv.shift) < kPvManyGroups;
+    if (batch > kOrderBatches ? few : cost(s) < cost(pv.shift) || (slow && few)) pv.shift = s;
+  }
   if (forced_rows > 0)
     for (pv.shift = 0; 1 << pv.shift < forced_rows;) ++pv.shift;
-  pv.fine = forced_rows > 0 || batch > kOrderBatches || pv.shift < kPvMinShift ? pv.shift : kPvMinShift;
+  pv.fine = forced_rows > 0 || batch > kOrderBatches || pv.shift < least ? pv.shift : least;
   pv.most = pv.shift;
-  while (pv.most > pv.fine && max_rows > 1024 && groups(pv.most) == 1) --pv.most;
-  pv.few = (int32_t)((kPvFewGroups + heads - 1) / heads);
-  pv.many = (int32_t)((kPvManyGroups + heads - 1) / heads);
+  while (pv.most > pv.fine && pv.most > 10 && groups(pv.most) < 3) --pv.most;
+  const int64_t counted = heads * (g > 8 ? 2 : 1);
+  pv.few = (int32_t)((kPvFewGroups + counted - 1) / counted);
+  pv.many = (int32_t)((kPvManyGroups + counted - 1) / counted);
   pv.big = wide ? 10 : kPvMaxShift;
   const int64_t allowed = batch * pv_counted_rows(max_rows, max_rows);  // below 2^31 where the device adds up
   pv.full = allowed / 4 * 3 < INT32_MAX ? (int32_t)(allowed / 4 * 3) : INT32_MAX;

@@ -590,12 +590,15 @@ __device__ __forceinline__ uint64_t t_block_base(const SplitArgs& a, uint64_t b,
 // of a KV head are scored GH at a time against the same K registers (GH = 4
 // bounds the partial sums a lane holds to 64).  A workgroup's waves take the
 // next blocks of the same heads and join their statistics through LDS.
-// One wave, but kScoresMaxWaves on rows of more than kScoresLongBlocks
-// blocks: more, held until the slowest is done, measured slower (µs of this
+// One wave, but on rows of more than kScoresLongBlocks blocks kScoresMaxWaves
+// (half of them with one or two query heads per KV head): more, held until the slowest is done, measured slower (µs of this
 // launch at 1 / 2 / 4 / 8 waves, 32/8 D=128: B=1 S=131072 47.9 / 50.8 / 50.4
 // / 52.1, S=3001 4.9 / 5.6 / 6.4 / 8.0, B=8 S=32768 92.4 / 97.3), and fewer
 // leave the P.V launch more entries to join than its lanes take at once (S =
-// 131072 53.9 with four waves here, 56.8 with two).  Grid: pieces
+// 131072 53.9 with four waves here, 56.8 with two; µs of the call at 1 / 2 / 4
+// waves, 16/16 B=1 S=60000 87.0 / 84.7 / 89.5, 32/16 88.2 / 86.0 / 91.4, 8/8 D=256
+// S=70000 110.9 / 106.2 / 109.1, 32/32 D=64 S=71980 121.4 / 117.0 / 118.8, 32/8 D=64
+// S=131072 80.0 / 73.1 / 69.2).  Grid: pieces
 // (batch_piece) of 2^sup_shift rows times units_per_batch head groups.
 constexpr int kScoresMaxWaves = 4;
 constexpr int kScoresLongBlocks = 2048;

@@ -10,8 +10,8 @@
 extern "C" {
 
 // out: shift, fine, parts, npv, total, full.
-void pv_plan(int64_t batch, int hkv, int max_rows, int d, int forced_rows, int64_t* out) {
-  const fmha_decode::PvPieces pv = fmha_decode::plan_pv_pieces(batch, hkv, max_rows, d, forced_rows);
+void pv_plan(int64_t batch, int units, int g, int max_rows, int d, int scattered, int forced_rows, int64_t* out) {
+  const fmha_decode::PvPieces pv = fmha_decode::plan_pv_pieces(batch, units, g, max_rows, d, scattered != 0, forced_rows);
   const int64_t v[6] = {pv.shift, pv.fine, pv.parts, pv.npv, pv.total, pv.full};
   for (int i = 0; i < 6; ++i) out[i] = v[i];
 }
@@ -19,9 +19,9 @@ void pv_plan(int64_t batch, int hkv, int max_rows, int d, int forced_rows, int64
 // What the kernels make of the lengths: the size taken (as they add the rows
 // up: in 32 bits, up to kOrderBatches batches), and the pieces of all batches
 // and of the batch that has the most.
-void pv_take(int64_t batch, int hkv, int max_rows, int d, int forced_rows, int uniform, const int32_t* lens,
-             int64_t* shift, int64_t* all, int64_t* most) {
-  const fmha_decode::PvPieces pv = fmha_decode::plan_pv_pieces(batch, hkv, max_rows, d, forced_rows);
+void pv_take(int64_t batch, int units, int g, int max_rows, int d, int scattered, int forced_rows, int uniform,
+             const int32_t* lens, int64_t* shift, int64_t* all, int64_t* most) {
+  const fmha_decode::PvPieces pv = fmha_decode::plan_pv_pieces(batch, units, g, max_rows, d, scattered != 0, forced_rows);
   int s = pv.shift;
   if (!uniform && batch <= fmha_decode::kOrderBatches) {
     int rows = 0;

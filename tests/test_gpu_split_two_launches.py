@@ -112,28 +112,28 @@ def test_many_calls_same_bits():
             assert torch.equal(o.view(torch.int16), first.view(torch.int16)), i
 
 
-# (layout, Hq, Hkv, D, max_len, lengths, P.V rows planned, parts): lengths far
+# (layout, Hq, Hkv, D, max_len, lengths, parts): lengths far
 # below the longest row allowed, for which the device takes shorter pieces than
 # planned (one batch, a few, one register of lengths and more), and as long,
 # for which it keeps them; head dims whole and by halves; empty and invalid
 # batches.  -1 stands for max_len + 1.
 CHOSEN = [
-    ("packed", 32, 8, 128, 131072, [5000], 4096, 1),
-    ("packed", 8, 8, 256, 60000, [3000], 4096, 2),
-    ("paged16", 64, 8, 128, 32768, [9000, 0, 2049, -1, 700, 1], 2048, 1),
-    ("strided", 8, 8, 64, 9000, [9000] + [400] * 11, 2048, 1),
-    ("packed", 16, 2, 256, 16384, [6000, 0, 300, 16], 1024, 2),
-    ("paged16", 8, 8, 256, 11516, [4000, -1, 0, 900, 257] + [100] * 5, 4096, 1),
-    ("strided", 2, 2, 256, 4096, [3000] + [150] * 43, 4096, 2),
-    ("paged1", 8, 1, 256, 8192, [5000, 600] + [250] * 18, 2048, 2),
-    ("packed", 1, 1, 64, 8000, [8000] + [300] * 69, 2048, 1),
-    ("packed", 8, 8, 64, 2233, [2233] * 57, 4096, 1),
-    ("paged16", 8, 8, 256, 4000, [4000] * 10 + [3500] * 12, 4096, 1),
+    ("packed", 32, 8, 128, 131072, [5000], 1),
+    ("packed", 8, 8, 256, 60000, [3000], 2),
+    ("paged16", 64, 8, 128, 32768, [9000, 0, 2049, -1, 700, 1], 1),
+    ("strided", 8, 8, 64, 9000, [9000] + [400] * 11, 1),
+    ("packed", 16, 2, 256, 16384, [6000, 0, 300, 16], 2),
+    ("paged16", 8, 8, 256, 11516, [4000, -1, 0, 900, 257] + [100] * 5, 1),
+    ("strided", 2, 2, 256, 4096, [3000] + [150] * 43, 2),
+    ("paged1", 8, 1, 256, 8192, [5000, 600] + [250] * 18, 2),
+    ("packed", 1, 1, 64, 8000, [8000] + [300] * 69, 1),
+    ("packed", 8, 8, 64, 2233, [2233] * 57, 1),
+    ("paged16", 8, 8, 256, 4000, [4000] * 10 + [3500] * 12, 1),
 ]
 
 
-@pytest.mark.parametrize("layout,Hq,Hkv,D,max_len,lens,rows,parts", CHOSEN)
-def test_device_chosen_pieces(monkeypatch, layout, Hq, Hkv, D, max_len, lens, rows, parts):
+@pytest.mark.parametrize("layout,Hq,Hkv,D,max_len,lens,parts", CHOSEN)
+def test_device_chosen_pieces(monkeypatch, layout, Hq, Hkv, D, max_len, lens, parts):
     """What the device makes of the lengths, with a workspace of exactly the
     size asked for between guard bytes, which stay."""
     import torch
@@ -182,7 +182,8 @@ def test_device_chosen_pieces(monkeypatch, layout, Hq, Hkv, D, max_len, lens, ro
                                                   max_seqlen_kv=max_len, workspace=ws)
     first = call()
     split = [f for kind, f in last_plan() if kind.startswith("split")]
-    assert len(split) == 1 and split[0]["pv_rows"] == rows and split[0]["pv_parts"] == parts, split
+    assert len(split) == 1 and split[0]["pv_parts"] == parts, split
+    assert split[0]["pv_rows"] > split[0]["pv_rows_least"] == 256, split  # the device has a choice
     second = call()
     torch.cuda.synchronize()
     assert bool((room[:guard] == 0xA5).all()) and bool((room[guard + need:] == 0xA5).all())

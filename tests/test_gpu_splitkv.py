@@ -122,12 +122,14 @@ def test_many_batches_direct_path():
     assert _launch("split")["pieces"] == 1
 
 
-def test_one_long_sequence():
-    """More than 2048 blocks: scores workgroups of four waves, and sums of
-    partial outputs in two levels."""
-    _case(1, 32, 8, 128, np.array([40000], np.int32), 40000, seed=7, std=0.5)
+@pytest.mark.parametrize("Hq,Hkv,rows", [(32, 8, 64), (8, 8, 32), (16, 8, 32)])
+def test_one_long_sequence(monkeypatch, Hq, Hkv, rows):
+    """More than 2048 blocks: scores workgroups of four waves (two with one or
+    two query heads per KV head), and sums of partial outputs in two levels."""
+    monkeypatch.setenv("FMHA_DECODE_SPLIT_CHUNK", "2048")
+    _case(1, Hq, Hkv, 128, np.array([40000], np.int32), 40000, seed=7, std=0.5)
     split = _launch("split")
-    assert split["scores_rows"] == 64 and split["pieces"] > 16
+    assert split["scores_rows"] == rows and split["pieces"] > 16
 
 
 # (B, Hq, Hkv, D, max_len): fewer (batch, KV-head group) units than the

@@ -24,15 +24,15 @@ def lib(tmp_path_factory):
     return ctypes.CDLL(out)
 
 
-def _plan(lib, batch, hkv, max_rows, d, forced=0):
+def _plan(lib, batch, units, g, max_rows, d, forced=0, scattered=0):
     out = (ctypes.c_int64 * 6)()
-    lib.pv_plan(ctypes.c_int64(batch), hkv, max_rows, d, forced, out)
+    lib.pv_plan(ctypes.c_int64(batch), units, g, max_rows, d, scattered, forced, out)
     return dict(zip(("shift", "fine", "parts", "npv", "total", "full"), out))
 
 
-def _take(lib, batch, hkv, max_rows, d, lens, forced=0, uniform=0):
+def _take(lib, batch, units, g, max_rows, d, lens, forced=0, uniform=0, scattered=0):
     got = [ctypes.c_int64() for _ in range(3)]
-    lib.pv_take(ctypes.c_int64(batch), hkv, max_rows, d, forced, uniform, (ctypes.c_int32 * len(lens))(*lens),
+    lib.pv_take(ctypes.c_int64(batch), units, g, max_rows, d, scattered, forced, uniform, (ctypes.c_int32 * len(lens))(*lens),
                 *(ctypes.byref(x) for x in got))
     return [x.value for x in got]
 
@@ -58,15 +58,17 @@ def test_pieces_fit_what_the_host_set_aside(lib):
     finer = 0
     for i in range(20000):
         batch = rng.choice((1, 1, 2, 3, rng.randint(1, 64), rng.randint(65, 300)))
-        hkv = rng.choice((1, 2, 3, 4, 8, 16, 32, 64))
+        units = rng.choice((1, 2, 3, 4, 8, 16, 32, 64))
+        g = rng.choice((1, 4, 8, 16, 32))
         d = rng.choice((64, 128, 256))
         max_rows = rng.choice((rng.randint(17, 300), rng.randint(17, 9000), int(2 ** rng.uniform(5, 28))))
         forced = rng.choice((0, 0, 0, 128, 512, 4096))
         uniform = int(rng.random() < 0.1)
+        scattered = rng.randrange(2)
         lens = _lengths(rng, batch, max_rows)
-        p = _plan(lib, batch, hkv, max_rows, d, forced)
-        shift, pieces, most = _take(lib, batch, hkv, max_rows, d, lens, forced, uniform)
-        case = (batch, hkv, max_rows, d, forced, uniform, lens[:8], p, shift, pieces, most)
+        p = _plan(lib, batch, units, g, max_rows, d, forced, scattered)
+        shift, pieces, most = _take(lib, batch, units, g, max_rows, d, lens, forced, uniform, scattered)
+        case = (batch, units, g, max_rows, d, scattered, forced, uniform, lens[:8], p, shift, pieces, most)
         assert p["fine"] <= shift <= p["shift"], case
         assert pieces <= p["total"] and most <= p["npv"], case
         assert shift == p["shift"] or not (forced or uniform or batch > 256), case
@@ -76,9 +78,9 @@ def test_pieces_fit_what_the_host_set_aside(lib):
 
 
 def test_full_batches_keep_the_planned_size(lib):
-    for batch, hkv, max_rows, d in ((3, 4, 66558, 256), (1, 8, 108751, 256), (8, 8, 32768, 128), (57, 8, 2233, 64)):
-        p = _plan(lib, batch, hkv, max_rows, d)
+    for batch, units, max_rows, d in ((3, 4, 66558, 256), (1, 8, 108751, 256), (8, 8, 32768, 128), (57, 8, 2233, 64)):
+        p = _plan(lib, batch, units, 4, max_rows, d)
         assert p["shift"] == 12  # few, long pieces
-        assert _take(lib, batch, hkv, max_rows, d, [max_rows] * batch)[0] == 12
+        assert _take(lib, batch, units, 4, max_rows, d, [max_rows] * batch)[0] == 12
         short = [max_rows // 20] * batch
-        assert _take(lib, batch, hkv, max_rows, d, short)[0] < 12
+        assert _take(lib, batch, units, 4, max_rows, d, short)[0] < 12

@@ -15,8 +15,8 @@
 //      butterfly (shared with the short kernel); scaled scores t_j -> T, and
 //      per query head the max m and the sum of exp(t_j - m) of the
 //      workgroup's rows, joined through LDS.
-//   2. P.V (fmha_decode_splitkv_pv.hpp): workgroups of eight waves, each
-//      joining its row's statistics, weighting a chunk of V rows and, with
+//   2. P.V (fmha_decode_splitkv_pv.hpp): workgroups of four waves, each
+//      joining its row's statistics, weighting a piece of the V rows and, with
 //      more than one workgroup per row, leaving a partial output; the last
 //      one of a row to finish adds them.
 //
@@ -24,7 +24,7 @@
 // four launches cost a short row more than its bytes (µs of kernels, B=1
 // S=3001 32/8 on 16-row pages 20.9 -> 14.1, B=8 of 47-1500 rows 16/16 D=64
 // BHSD 17.0 -> 11.8, ragged B=48 8/1 over 250-8000 rows 34.6 -> 24; long rows
-// keep their time, B=1 S=131072 104.6 -> 104.3, or gain with groups of 8,
+// keep their time, B=1 S=131072 104.6 -> 102.0, or gain with groups of 8,
 // B=8 S=32768 64/8 221 -> 207).  P.V workgroups find their batch in the
 // lengths (row_piece), so that those past the rows of a ragged batch come
 // last and end at once, where a grid over the longest row interleaves them
@@ -329,16 +329,14 @@ struct LongRows {
   int bad = 0;
   __device__ __forceinline__ bool any_bad() const { return bad != 0; }
 
-  // lane_rows_: this lane's rows start that many rows after lo, and end at
-  // lane_end (relative to lo, at most hi - lo): lane groups serving
-  // different blocks or chunks.  Both 0 / hi - lo for the paged layouts.
+  // lane_rows_: this lane's rows start that many rows after lo (lane groups
+  // serving different blocks; 0 for the paged layouts).
   __device__ __forceinline__ void init(const SplitArgs& a, const uint16_t* t, uint32_t b, int64_t row_base, int lo_,
-                                       int hi, int hk, bool head_ok, int r, int lane_rows_ = 0,
-                                       int lane_end = 1 << 30) {
+                                       int hi, int hk, bool head_ok, int r, int lane_rows_ = 0) {
     lo = lo_;
     n = hi > lo_ ? hi - lo_ : 0;
     lane_rows = lane_rows_;
-    lane_n = lane_end < n ? lane_end : n;
+    lane_n = n;
     const int hkv = kv_heads_mem(a);
     const int hm = kv_head_mem(a, hk);
     if constexpr (LAYOUT == kLayoutPacked) {
@@ -477,11 +475,11 @@ struct PagedLaneRows {
   __device__ __forceinline__ bool any_bad() const { return __builtin_amdgcn_ballot_w64(bad != 0) != 0; }
 
   __device__ __forceinline__ void init(const SplitArgs& a, const uint16_t* t, uint32_t b, int64_t, int lo_, int hi,
-                                       int hk, bool head_ok, int r, int lane_rows_ = 0, int lane_end = 1 << 30) {
+                                       int hk, bool head_ok, int r, int lane_rows_ = 0) {
     const int n = hi > lo_ ? hi - lo_ : 0;
     lo = lo_;
     lane_rows = lane_rows_;
-    lane_n = head_ok ? (lane_end < n ? lane_end : n) : 0;
+    lane_n = head_ok ? n : 0;
     base = t + (uint64_t)kv_head_mem(a, hk) * D + r * 8;
     safe = a.q + r * 8;
     pages = a.block_table + (uint64_t)b * (uint64_t)a.bt_stride;

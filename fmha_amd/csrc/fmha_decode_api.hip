@@ -303,10 +303,11 @@ int launch(void* stream, int layout, DecodeArgs a, int32_t batch, int32_t dq, in
 // keeps the VALU kernel wherever it exists (for comparisons).
 // Long rows, by the launch's group (g_launch = launch query heads per launch
 // KV head: 8 for G = 5-8 and, as kv_groups groups of 8, for every G > 8):
-// the matrix-core split passes for G > 8 and for G = 5-8 on the packed,
+// the matrix-core scores pass for G > 8 and for G = 5-8 on the packed,
 // strided and 16-row-page layouts, and on pages under 16 rows when the
 // batch has fewer KV heads than half a wave (hkv launch KV heads, head dim
-// d); the VALU passes otherwise.  Against the VALU passes at G = 8 and 5-7
+// d); the VALU one otherwise.  Against the VALU passes at G = 8 and 5-7, when
+// each kind had a P.V pass of its own
 // (µs, each at its best chunk size; D = 128 unless given): B=8 S=32768
 // Hq/Hkv 64/8 232 vs 223, B=256 S=1024 64/8 233 vs 221, B=64 S=4096 64/8
 // 219 vs 218, 32/4 125 vs 123, 8/1 52 vs 46, D=64 B=32 64/8 99 vs 87,
@@ -867,15 +868,14 @@ namespace {
 // Checks shared by the split-KV entry points, then the plan and the
 // layout-independent fields of the launch.  kv_span_bytes: the largest byte
 // range one wave's K/V descriptor covers in the caller's layout (must stay
-// below 2^30, as must one batch's scores and partial outputs).
+// below 2^30, as must one batch's scores; partial outputs are addressed in 64
+// bits).
 int split_prepare(bool scattered, const void* Q, const void* K, const void* V, void* O, int32_t max_seqlen_kv,
                   int32_t batch, int32_t num_heads_q, int32_t num_heads_kv, int32_t kv_groups, int32_t head_dim,
                   float softmax_scale, void* workspace, size_t workspace_bytes, int64_t kv_span_bytes, SplitArgs& a) {
   const SplitPlan plan = plan_split(batch, num_heads_q, num_heads_kv, kv_groups, max_seqlen_kv, head_dim, scattered);
   const int64_t padded_rows = (int64_t)plan.nblk * fmha_decode::kSplitBlockRows;
-  const int64_t part_bytes = (int64_t)num_heads_q * plan.pv.npv * head_dim * 4;  // one batch's partials
-  if (kv_span_bytes >= (int64_t(1) << 30) || padded_rows * num_heads_q * 4 >= (int64_t(1) << 30) ||
-      part_bytes >= (int64_t(1) << 30))
+  if (kv_span_bytes >= (int64_t(1) << 30) || padded_rows * num_heads_q * 4 >= (int64_t(1) << 30))
     return reject(FMHA_DECODE_ERROR_INVALID_VALUE, "max_seqlen_kv too large for this head count (%d)", max_seqlen_kv);
   if (!workspace) return reject(FMHA_DECODE_ERROR_INVALID_VALUE, "workspace must be non-null");
   if ((reinterpret_cast<uintptr_t>(workspace) & (kWorkspaceAlign - 1)) != 0)
@@ -912,8 +912,8 @@ int split_launch(void* stream, int layout, const SplitArgs& a, int32_t head_dim)
   const int g = a.num_heads_q / a.num_heads_kv;
   hipError_t err;
   // Paged caches with fewer KV heads than a wave holds read through
-  // per-lane addresses, so that the idle lane groups take other blocks or
-  // chunks of the same heads (sub-units, as on packed caches).
+  // per-lane addresses, so that the idle lane groups take other blocks of the
+  // same heads (sub-units, as on packed caches).
   const int hpw = kWaveSize / (head_dim / 8);
   const bool lanes = 2 * a.num_heads_kv <= hpw && hpw % (2 * a.num_heads_kv) == 0;
   // The VALU long-row kernels; onepass_only: their single pass or nothing.
@@ -1214,7 +1214,7 @@ extern "C" int fmha_decode_fwd_splitkv_paged(void* stream, const void* Q, const 
   // Short rows take the short kernels directly: the VALU paged kernel for G
   // <= 8, the matrix-core one above where rows lie within a batch's first
   // page (paged_mfma_layout); otherwise they go through the split kernels
-  // below like longer rows (one 16-row block, one chunk).  µs, B=7812 Hq/Hkv
+  // below like longer rows (one 16-row block, one piece).  µs, B=7812 Hq/Hkv
   // 128/8 S=16 D=128 on 16-row pages: split 331.0, matrix-core short kernel
   // 147.4 (packed 149.5).
   if (max_seqlen_kv <= FMHA_DECODE_MAX_SEQLEN_KV &&

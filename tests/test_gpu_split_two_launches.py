@@ -196,6 +196,31 @@ def test_device_chosen_pieces(monkeypatch, layout, Hq, Hkv, D, max_len, lens, pa
     assert_pass(oracle.compare(bits[ok], r[ok], slack[ok]), f"{layout} B={B} G={Hq // Hkv} D={D} max={max_len}")
 
 
+def test_longest_rows_allowed():
+    """The longest rows that a batch's scores allow (below 2^30 bytes), of
+    which few are there: accepted, the row's pieces counted in 131072 places;
+    16 rows more are refused."""
+    import torch
+    import fmha_amd
+    Hq, D, n, page = 8, 256, 700, 64
+    max_len = 2 ** 25 - 16
+    lens = np.array([n], np.int32)
+    q, k, v, cu = make_inputs(1, Hq, Hq, D, lens, seed=9, std=0.5)
+    used = (n + page - 1) // page
+    kc, vc = (np.zeros((used * page, Hq, D), np.uint16) for _ in range(2))
+    kc[:n], vc[:n] = k, v
+    table = torch.full((1, (max_len + 16 + page - 1) // page), -1, dtype=torch.int32, device="cuda")
+    table[0, :used] = torch.arange(used, dtype=torch.int32)
+    args = (to_dev(q), *(to_dev(x.reshape(-1, page, Hq, D)) for x in (kc, vc)), table, torch.from_numpy(lens).cuda())
+    o = fmha_amd.fmha_decode_paged(*args, softmax_scale=default_scale(D), max_seqlen_kv=max_len)
+    torch.cuda.synchronize()
+    r, slack = oracle.decode(q, k, v, cu, Hq, Hq, D, default_scale(D), with_slack=True, max_seqlen=n)
+    bits = o.view(torch.int16).cpu().numpy().view(np.uint16)
+    assert_pass(oracle.compare(bits.reshape(r.shape), r, slack), "longest rows")
+    with pytest.raises(fmha_amd.FmhaDecodeError, match="too large"):
+        fmha_amd.fmha_decode_paged(*args, softmax_scale=default_scale(D), max_seqlen_kv=max_len + 16)
+
+
 @pytest.mark.parametrize("page_size", [1, 16, 64])
 @pytest.mark.parametrize("Hq,Hkv,D", [(8, 8, 128), (16, 2, 64), (32, 1, 128), (4, 2, 256)])
 def test_paged_ragged_rows(monkeypatch, page_size, Hq, Hkv, D):

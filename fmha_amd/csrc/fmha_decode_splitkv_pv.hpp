@@ -35,9 +35,13 @@
 // Four waves per workgroup: with eight, two workgroups per CU start and end
 // together, nothing streaming meanwhile (µs of this launch, 32/8 B=1
 // S=131072 80 / 65, B=48 8/1 over 250-8000 rows 28 / 16).  What bounds it: V's
-// bytes for long rows (4.9 TB/s at B=1 S=131072, 53.9 us); for short ones the
-// chain lengths -> scores and V -> weights -> sums -> count, about 8 us.  The
-// order of every sum is fixed, whichever workgroup is last.
+// bytes for long rows (5.6 TB/s at B=1 S=131072, 51.5 us; D = 256 28/4 B=3
+// S=66558 on 64-row pages 5.0 TB/s, 87.9 us), behind each workgroup's joining of
+// the whole row's statistics; for short ones the chain lengths -> scores and V
+// -> weights -> sums -> count, about 8 us.  Every descriptor comes from scalar
+// registers: from vector ones each load was a loop over the lanes (µs of the
+// call, packed MQA 32/1 B=16 S=32768 93.8 / 91.4, 8/8 D = 256 B=10 up to 11516
+// rows on 16-row pages 58.5 / 55.9).  The order of every sum is fixed, whichever workgroup is last.
 #pragma once
 
 #include "fmha_decode_group.hpp"

@@ -24,7 +24,8 @@ constexpr int kOrderBatches = 256;
 
 // What of a piece's start and end its CU's other workgroups don't hide, in rows
 // of it, and the CUs.
-constexpr int64_t kPvPieceRows = 400, kPvSlowPieceRows = 600, kPvCus = 256;
+constexpr int64_t kPvPieceRows = 400, kPvSlowPieceRows = 600;
+constexpr int kPvCusShift = 8;  // log2
 // Pieces of kPvMaxShift from which on a workgroup takes all of 256 dims.
 constexpr int64_t kPvWholeGroups = 176;
 // Ragged batches: the workgroups below which the device takes shorter pieces,
@@ -118,19 +119,24 @@ inline PvPieces plan_pv_pieces(int64_t batch, int units, int g, int max_rows, in
   pv.parts = wide && batch * units * groups(kPvMaxShift) < kPvWholeGroups ? 2 : 1;
   const int64_t heads = (int64_t)units * pv.parts;
   const bool slow = d == 64 || scattered;
-  const int64_t places = slow || g > 8 ? 2 * kPvCus : kPvCus;
+  const int places = kPvCusShift + (slow || g > 8 ? 1 : 0);  // log2
   const int64_t ends = slow ? kPvSlowPieceRows : kPvPieceRows;
-  const int64_t at_once = kPvCus * (wide && pv.parts == 1 ? 3 : 4);
+  const int64_t at_once = (int64_t)(wide && pv.parts == 1 ? 3 : 4) << kPvCusShift;
   const auto cost = [&](int s) {  // in half rows
     const int64_t n = groups(s), w = batch * heads * n;
-    if (w <= at_once) return 2 * ((w + places - 1) / places) * ((n == 1 ? max_rows : 1 << s) + ends);
-    return (2 * w + (slow ? 2 : 1) * places) * ((max_rows + n - 1) / n + ends) / places;
+    if (w <= at_once) return 2 * ((w + (1 << places) - 1) >> places) * ((n == 1 ? max_rows : 1 << s) + ends);
+    return ((2 * w + ((slow ? 2 : 1) << places)) * ((max_rows + n - 1) / n + ends)) >> places;
   };
   const int least = max_rows <= 1 << (kPvMinShift + 1) ? kPvMinShift + 1 : kPvMinShift;
   pv.shift = batch > kOrderBatches ? kPvMaxShift - 1 : kPvMaxShift;
+  int64_t best = cost(pv.shift);
   for (int s = pv.shift - 1; s >= least; --s) {
     const bool few = batch * heads * groups(pv.shift) < kPvManyGroups;
-    if (batch > kOrderBatches ? few : cost(s) < cost(pv.shift) || (slow && few)) pv.shift = s;
+    const int64_t c = cost(s);
+    if (batch > kOrderBatches ? few : c < best || (slow && few)) {
+      pv.shift = s;
+      best = c;
+    }
   }
   if (forced_rows > 0)
     for (pv.shift = 0; 1 << pv.shift < forced_rows;) ++pv.shift;
